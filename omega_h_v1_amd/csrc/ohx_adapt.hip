@@ -132,18 +132,23 @@ __global__ __launch_bounds__(BLOCK) void indset_round(u32 n, u32 const* __restri
   wave_flag(flag, undecided);
 }
 
-// The same round over the edges of a 3D mesh with the neighbours taken
-// from the tets around each edge (up(1,3), down(3,1)): an edge's
-// neighbours are the other edges of its tets, which as a set is the edge
-// star star(1,3) (the two other edges of every triangle through the edge
-// and the opposite edge of every tet through it); the rule depends only on
-// that set, so the star itself, which would need up(1,2), is not built.
-__global__ __launch_bounds__(BLOCK) void indset_round_tets(u32 n, u32 const* __restrict__ uo,
-                                                           u32 const* __restrict__ ua, u32 const* __restrict__ ud,
-                                                           u32 const* __restrict__ er,
-                                                           double const* __restrict__ good,
-                                                           u32 const* __restrict__ old, u32* __restrict__ state,
-                                                           u32* __restrict__ flag) {
+// The same round over the edges of a mesh with the neighbours taken from the
+// elements around each edge (up(1,dim), down(dim,1); NE edges per element):
+// an edge's neighbours are the other edges of its elements, which as a set
+// is the edge star star(1,dim) (in 3D the two other edges of every triangle
+// through the edge and the opposite edge of every tet through it); the rule
+// depends only on that set, so the star itself, which would need up(1,2) in
+// 3D, is not built.  Bound by the gathers around undecided edges; the walk
+// meets a neighbour once per shared element, about twice the star's reads,
+// but a split pass saves the star, which cost far more than its rounds
+// (384,000 tets, 5 split passes: up(1,2) and the star 1.9 ms of 9.5 ms).
+template <u32 NE>
+__global__ __launch_bounds__(BLOCK) void indset_round_elems(u32 n, u32 const* __restrict__ uo,
+                                                            u32 const* __restrict__ ua, u32 const* __restrict__ ud,
+                                                            u32 const* __restrict__ er,
+                                                            double const* __restrict__ good,
+                                                            u32 const* __restrict__ old, u32* __restrict__ state,
+                                                            u32* __restrict__ flag) {
   u32 i = xcd_block() * BLOCK + threadIdx.x;
   bool undecided = false;
   if (i < n) {
@@ -153,9 +158,9 @@ __global__ __launch_bounds__(BLOCK) void indset_round_tets(u32 n, u32 const* __r
       bool wait = false, out = false;
       for (u32 j = uo[i]; j < uo[i + 1] && !out; ++j) {
         u32 t = ua[j], d = ud[j];
-        for (u32 l = 0; l < 6; ++l) {
+        for (u32 l = 0; l < NE; ++l) {
           if (l == d) continue;
-          u32 o = er[6 * (size_t) t + l];
+          u32 o = er[NE * (size_t) t + l];
           u32 so = old[o];
           if (so == IN_SET) {
             out = true;
@@ -219,19 +224,19 @@ __global__ __launch_bounds__(BLOCK) void indset_round_verts(u32 n, u32 const* __
 // state alone, so the result and the round count are those of a run from
 // the start)
 static Buf<u32> indset_rounds(Mesh& m, u32 ent_dim, u32 const* filter, double const* good, u32 rounds,
-                              u32 const** last_flag, bool via_tets = false, Buf<u32>* start = nullptr,
-                              u32 start_done = 0) {
+                              u32 const** last_flag, Buf<u32>* start = nullptr, u32 start_done = 0) {
   u32 n = count(m, ent_dim);
-  // vertices: neighbours through the edges (indset_round_verts)
-  bool const via_edges = ent_dim == 0 && m.dim >= 2;
+  // vertices: neighbours through the edges (indset_round_verts); edges:
+  // through the elements (indset_round_elems)
+  bool const via_edges = ent_dim == 0 && m.dim >= 2, via_elems = ent_dim == 1 && m.dim >= 2;
   Graph empty;
-  Graph const& g = (via_tets || via_edges) ? empty : ask_star(m, ent_dim, m.dim);
-  Up const* ut = via_tets ? &ask_up(m, 1, 3) : via_edges ? &ask_up(m, 0, 1) : nullptr;
-  u32 const* er = via_tets ? ask_down(m, 3, 1) : via_edges ? ask_down(m, 1, 0) : nullptr;
+  Graph const& g = (via_elems || via_edges) ? empty : ask_star(m, ent_dim, m.dim);
+  Up const* ut = via_elems ? &ask_up(m, 1, m.dim) : via_edges ? &ask_up(m, 0, 1) : nullptr;
+  u32 const* er = via_elems ? ask_down(m, m.dim, 1) : via_edges ? ask_down(m, 1, 0) : nullptr;
   auto round = [&](u32 const* in, u32* outs, u32* fl, double bytes) {
-    if (via_tets)
-      launch_timed("indset_round", bytes, indset_round_tets, dim3(nblocks(n)), dim3(BLOCK), n, ut->offsets.get(),
-                   ut->adj.get(), ut->dirs.get(), er, good, in, outs, fl);
+    if (via_elems)
+      launch_timed("indset_round", bytes, m.dim == 3 ? indset_round_elems<6> : indset_round_elems<3>, dim3(nblocks(n)),
+                   dim3(BLOCK), n, ut->offsets.get(), ut->adj.get(), ut->dirs.get(), er, good, in, outs, fl);
     else if (via_edges)
       launch_timed("indset_round", bytes, indset_round_verts, dim3(nblocks(n)), dim3(BLOCK), n, ut->offsets.get(),
                    ut->adj.get(), ut->dirs.get(), er, good, in, outs, fl);
@@ -321,9 +326,8 @@ static Buf<u32> find_indset_bounded(Mesh& m, u32 ent_dim, u32 const* filter, dou
   return indset_rounds(m, ent_dim, filter, good, first_batch_rounds(), last_flag);
 }
 // the checked loop from the first batch's state
-static Buf<u32> find_indset_resume(Mesh& m, u32 ent_dim, double const* good, Buf<u32>&& state,
-                                   bool via_tets = false) {
-  return indset_rounds(m, ent_dim, nullptr, good, 0, nullptr, via_tets, &state, first_batch_rounds());
+static Buf<u32> find_indset_resume(Mesh& m, u32 ent_dim, double const* good, Buf<u32>&& state) {
+  return indset_rounds(m, ent_dim, nullptr, good, 0, nullptr, &state, first_batch_rounds());
 }
 
 // ------------------------------------------------------------- inherit
@@ -2958,7 +2962,7 @@ static u32 swap_common(Mesh& m, Buf<u32>& cand, double const* eq_given = nullptr
   // and all the totals (a set not settled in the first batch goes on from
   // there with the checked loop, same rounds, same result)
   u32 const* flag = nullptr;
-  Buf<u32> indset = indset_rounds(m, 1, cand.get(), q.get(), first_batch_rounds(), &flag, true);
+  Buf<u32> indset = find_indset_bounded(m, 1, cand.get(), q.get(), &flag);
   u32 dlo = m.full ? 1 : m.dim;
   Buf<u32> goffs[4], soffs[4];
   u32 tots[8];
@@ -3033,7 +3037,7 @@ static u32 swap_common(Mesh& m, Buf<u32>& cand, double const* eq_given = nullptr
   };
   offsets_and_totals();
   if (tots[0]) {  // not settled in the first batch: the checked loop from there
-    indset = find_indset_resume(m, 1, q.get(), std::move(indset), true);
+    indset = find_indset_resume(m, 1, q.get(), std::move(indset));
     flag = nullptr;
     offsets_and_totals();
   }

@@ -1,0 +1,37 @@
+"""The independent set over a mesh's edges, whose neighbours are read from
+the elements around each edge, against the oracle's, which reads the edge
+star: the smallest boxes, odd sizes, and goodness with and without ties."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+import meshlib as ML
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("dim,n", [(2, 1), (2, 7), (2, 33), (3, 1), (3, 2), (3, 7)])
+@pytest.mark.parametrize("levels", [1, 5, None])
+def test_edge_indset_through_elements(dim, n, levels):
+    libs = [ML.load("product"), ML.load("oracle")]
+    assert all(libs), "build first"
+    # goodness of one level is one chain of ties over the whole mesh
+    libs[0].dll.ohx_set_indset_max_rounds.argtypes = [C.c_uint]
+    libs[1].dll.orc_set_indset_max_rounds.argtypes = [C.c_uint]
+    libs[0].dll.ohx_set_indset_max_rounds(100000)
+    libs[1].dll.orc_set_indset_max_rounds(100000)
+    try:
+        x, c = ML.box(dim, n)
+        got = []
+        for lib in libs:
+            m = ML.Mesh(lib, dim, x, c)
+            m.derive_model_full()
+            rng = np.random.default_rng(n)
+            ne = m.count(1)
+            good = rng.random(ne) if levels is None else rng.integers(0, levels, ne).astype(float)
+            got.append(m.find_indset(1, rng.random(ne) < 0.7, good))
+        assert np.array_equal(got[0], got[1])
+    finally:
+        libs[0].dll.ohx_set_indset_max_rounds(0)
+        libs[1].dll.orc_set_indset_max_rounds(0)
