@@ -223,6 +223,12 @@ __global__ __launch_bounds__(BLOCK) void indset_round_verts(u32 n, u32 const* __
 // from that state instead of from the filter (rounds are a function of the
 // state alone, so the result and the round count are those of a run from
 // the start)
+static void note_rounds(u32 used) {
+  u32 seen = g_indset_rounds_seen.load();
+  while (used > seen && !g_indset_rounds_seen.compare_exchange_weak(seen, used)) {
+  }
+}
+
 static Buf<u32> indset_rounds(Mesh& m, u32 ent_dim, u32 const* filter, double const* good, u32 rounds,
                               u32 const** last_flag, Buf<u32>* start = nullptr, u32 start_done = 0) {
   u32 n = count(m, ent_dim);
@@ -297,9 +303,7 @@ static Buf<u32> indset_rounds(Mesh& m, u32 ent_dim, u32 const* filter, double co
       // h[r]: entities still undecided after round r of this batch
       u32 k = 0;
       while (h[k]) ++k;
-      u32 used = done + k + 1, seen = g_indset_rounds_seen.load();
-      while (used > seen && !g_indset_rounds_seen.compare_exchange_weak(seen, used)) {
-      }
+      note_rounds(done + k + 1);
       return a;
     }
   }
@@ -2187,9 +2191,8 @@ void swap_int_edges_host(u32 rs, u32 code, u32* out) {
 
 // find_edge_ring (edge_ring.cpp:12-74): ring vertices ordered by chaining
 // each tet's opposite edge (a -> b), insertion style, <= 7 entries
-__device__ inline u32 edge_ring(u32 edge, u32 const* uo, u32 const* ua, u32 const* ud, u32 const* ev,
+__device__ inline u32 edge_ring(u32 edge, u32 f, u32 e, u32 const* ua, u32 const* ud, u32 const* ev,
                                 u32 const* vt, u32* edge_v, u32* ring_v) {
-  u32 f = uo[edge], e = uo[edge + 1];
   u32 rs = e - f;
   if (rs > MAX_EDGE_SWAP || rs < 3) return rs;
   u32 const* oe = opp(3, 1);
@@ -2343,32 +2346,33 @@ __device__ inline void swap_choose(SwapLds<MT>& L, u32 g, u32 lane, bool active,
   *near0 = nz;
 }
 
+// one batch of SW_EDGES candidates, group g of the block takes list[slot];
+// returns whether the group's candidate is accepted, with its value, ring
+// size and triangulation code; settled: the group had a candidate whose
+// choice is now known
 template <bool MT, bool MIXED>
-__global__ __launch_bounds__(BLOCK, 4) void swap_quality_k(
-    u32 ncand, u32 const* __restrict__ list, u32 const* __restrict__ uo, u32 const* __restrict__ ua,
-    u32 const* __restrict__ ud, u32 const* __restrict__ ev, u32 const* __restrict__ vt,
-    double const* __restrict__ x, double const* __restrict__ mt, double const* __restrict__ eq,
-    u32* __restrict__ cand, double* __restrict__ out, u32* __restrict__ rsz, u32* __restrict__ codes,
-    u32* __restrict__ words, u32 tag, u32* __restrict__ err, ScreenStats st) {
-  __shared__ SwapLds<MT> L;
+__device__ inline bool swap_quality_batch(SwapLds<MT>& L, u32 ncand, u32 slot, u32 const* __restrict__ list,
+                                          u32 const* __restrict__ uo, u32 const* __restrict__ un,
+                                          u32 const* __restrict__ ua, u32 const* __restrict__ ud,
+                                          u32 const* __restrict__ ev, u32 const* __restrict__ vt,
+                                          double const* __restrict__ x, double const* __restrict__ mt,
+                                          double const* __restrict__ eq, u32* __restrict__ err, ScreenStats st,
+                                          u32* edge, bool* settled, double* value, u32* ring_size, u32* choice) {
   u32 const g = threadIdx.x / SW_G, lane = threadIdx.x % SW_G;
-  // the candidates, compacted: group g of the block takes one
-  u32 const slot = xcd_block() * SW_EDGES + g;
   bool active = slot < ncand;
   u32 const i = active ? list[slot] : 0u;
+  *edge = i;
+  *settled = active;
   // A: the tets around the edge
   u32 f = 0, rs = 0, e0 = 0, e1 = 0;
   double qmin = 1;
   if (active) {
     f = uo[i];
-    rs = uo[i + 1] - f;
+    rs = un ? un[i] : uo[i + 1] - f;
     e0 = ev[2 * (size_t) i];
     e1 = ev[2 * (size_t) i + 1];
     if (rs > MAX_EDGE_SWAP || rs < 3) {
-      if (lane == 0) {
-        if (rs < 3) *err = ERR_EDGE_RING;
-        cand[i] = 0;
-      }
+      if (lane == 0 && rs < 3) *err = ERR_EDGE_RING;
       active = false;
     } else if (lane < rs) {
       u32 tet = ua[f + lane], te = ud[f + lane];
@@ -2407,10 +2411,7 @@ __global__ __launch_bounds__(BLOCK, 4) void swap_quality_k(
       ra[a + 1] = ta;
       rb[a + 1] = tb;
     }
-    if (!closed) {
-      *err = ERR_EDGE_RING;
-      cand[i] = 0;
-    }
+    if (!closed) *err = ERR_EDGE_RING;
     L.rs[g] = closed ? rs : 0u;
     L.old_minq[g] = qmin;
     for (u32 a = 0; a < rs; ++a) L.ring[g][a] = ra[a];
@@ -2446,7 +2447,6 @@ __global__ __launch_bounds__(BLOCK, 4) void swap_quality_k(
     }
     wave_count(st.screened, lane == 0 && reject);
     wave_count(st.reeval, lane == 0 && active && !reject);
-    if (reject && lane == 0) cand[i] = 0;
     __syncthreads();
     double best32 = best;
     bool const valid32 = !near0;  // no triangle near zero: best32 is the FP64 choice's, rounded
@@ -2460,8 +2460,27 @@ __global__ __launch_bounds__(BLOCK, 4) void swap_quality_k(
   } else {
     swap_choose<MT, false>(L, g, lane, active, &best, &code, &near0);
   }
-  bool accept = active && best > old_minq;
-  if (active && lane == 0) {
+  *value = best;
+  *ring_size = rs;
+  *choice = code;
+  return active && best > old_minq;
+}
+
+template <bool MT, bool MIXED>
+__global__ __launch_bounds__(BLOCK, 4) void swap_quality_k(
+    u32 ncand, u32 const* __restrict__ list, u32 const* __restrict__ uo, u32 const* __restrict__ ua,
+    u32 const* __restrict__ ud, u32 const* __restrict__ ev, u32 const* __restrict__ vt,
+    double const* __restrict__ x, double const* __restrict__ mt, double const* __restrict__ eq,
+    u32* __restrict__ cand, double* __restrict__ out, u32* __restrict__ rsz, u32* __restrict__ codes,
+    u32* __restrict__ words, u32 tag, u32* __restrict__ err, ScreenStats st) {
+  __shared__ SwapLds<MT> L;
+  u32 i, rs, code;
+  bool settled;
+  double best;
+  bool const accept = swap_quality_batch<MT, MIXED>(L, ncand, xcd_block() * SW_EDGES + threadIdx.x / SW_G, list, uo,
+                                                    nullptr, ua, ud, ev, vt, x, mt, eq, err, st, &i, &settled, &best,
+                                                    &rs, &code);
+  if (settled && threadIdx.x % SW_G == 0) {
     if (accept) {
       out[i] = best;
       rsz[i] = rs;
@@ -2489,7 +2508,6 @@ struct SwapEdgesOf {
   u32* out;            // (surviving + product tets) x 6 new edge ids
   u32 const* old;      // the old tets' edges
   u32 const* soff1;    // old edge -> its index among the surviving edges
-  u32 const* goff1;    // interior edges generated per swapped edge
   u32 nsame1, nsame3;  // surviving edges, surviving tets
   u32* err;
   // the element dual carried too (dual null: not built): the old dual,
@@ -2504,6 +2522,49 @@ struct SwapEdgesOf {
 };
 
 constexpr u32 DUAL_PENDING = 0xfffffffeu;
+
+// Words of a swap run (SwapRunView::words)
+enum { RW_ACC = 0, RW_EVAL = 1, RW_AFF = 2, RW_POOL = 3, RW_FIRST = 4, RW_FLAGS = 8, RW_WORDS = 16 };
+// an edge's word in a run: its choice is known, it is accepted, then ring
+// size and triangulation code as in the swap cache; a dead or boundary edge
+// is known and rejected for good
+constexpr u32 RI_KNOWN = 1u << 31, RI_ACCEPT = 1u << 30;
+
+// The mesh of a run of swap passes (see "swap passes in place"), as slots.
+struct SwapRunView {
+  u32 nE, nF, nT, nF0;  // slots in use before the pass's products; faces at the start
+  u32 pass;             // 1, 2, ...
+  u32* ev;              // edges: vertices, class, the pass that removed it (0: alive), choice and its
+  u32* ecd;             // value, first place and length of its list in (ua, ud), product uses
+  u32* eci;
+  u32* death;
+  u32* info;
+  double* q;
+  u32* lb;
+  u32* ln;
+  u32* cnt;
+  unsigned char* sa;  // independent-set state before / after a round
+  unsigned char* sb;
+  u32* ua;  // tets around the edges and the edges' places in them, ascending per edge
+  u32* ud;
+  u32* vt;  // tets: vertices, edges, dual, class, removed
+  u32* te;
+  u32* dual;
+  u32* tcd;
+  u32* tci;
+  unsigned char* dead;
+  u32* fv;  // faces: vertices, class, the pass that made a product face (from slot nF0 on)
+  u32* fcd;
+  u32* fci;
+  u32* fbirth;
+  u32* acc;  // accepted candidates and candidates to evaluate (any order)
+  u32* eval;
+  u32* sw;   // swapped edges in order, their first products of each dimension
+  u32* o1;
+  u32* o2;
+  u32* o3;
+  u32* words;
+};
 
 // local face of a tet (vertices tv) with the vertices a, b, c
 __device__ inline u32 tet_face_of(u32 const* tv, u32 a, u32 b, u32 c) {
@@ -2540,36 +2601,71 @@ __device__ inline u32 tet_edge_between(u32 a, u32 b) {
 // edges of the old tet at that ring slot (the one holding ring vertices k
 // and k + 1), and any other is one of the new interior edges.  The cavity's
 // ring edges and spokes are staged in LDS per thread (indexed by slot).
+// RUN: thread k takes the run's k-th swapped edge, nothing is renumbered
+// (soff1, soff3 are not read), a survivor's dual entry is rewritten by the
+// product now across that face, and the products' other arrays are set up.
+template <bool RUN>
 __global__ __launch_bounds__(BLOCK) void swap_products_k(
-    u32 ne, u32 const* __restrict__ indset, u32 const* __restrict__ goff1, u32 const* __restrict__ goff2,
-    u32 const* __restrict__ goff3, u32 const* __restrict__ uo, u32 const* __restrict__ ua,
-    u32 const* __restrict__ ud, u32 const* __restrict__ ev, u32 const* __restrict__ vt,
-    u32 const* __restrict__ codes, u32* __restrict__ out1, u32* __restrict__ out2, u32* __restrict__ out3,
-    SwapEdgesOf E) {
+    u32 ne, u32 const* indset, u32 const* goff1, u32 const* goff2, u32 const* goff3, u32 const* uo, u32 const* ua,
+    u32 const* ud, u32 const* ev, u32 const* vt, u32 const* codes, u32* out1, u32* out2, u32* out3, SwapEdgesOf E,
+    SwapRunView R) {
   __shared__ u32 s_ring[MAX_EDGE_SWAP][BLOCK];
   __shared__ u32 s_spoke[2][MAX_EDGE_SWAP][BLOCK];
   __shared__ u32 s_tet[MAX_EDGE_SWAP][BLOCK];
   u32 const tid = threadIdx.x;
   u32 i = xcd_block() * BLOCK + tid;
-  if (i >= ne || !indset[i]) return;  // no barrier follows
+  if (i >= ne || (!RUN && !indset[i])) return;  // no barrier follows
+  u32 const g1 = goff1[i], g2 = goff2[i], g3 = goff3[i];
+  if (RUN) i = R.sw[i];
+  u32 const f = RUN ? R.lb[i] : uo[i], e = RUN ? f + R.ln[i] : uo[i + 1];
+  auto edge_now = [&](u32 old) { return RUN ? old : E.soff1[old]; };
   u32 edge_v[2], ring_v[MAX_EDGE_SWAP];
-  u32 rs = edge_ring(i, uo, ua, ud, ev, vt, edge_v, ring_v);
+  u32 rs = edge_ring(i, f, e, ua, ud, ev, vt, edge_v, ring_v);
   if (rs < 3 || rs > MAX_EDGE_SWAP) return;  // cannot happen for an indset edge
-  u32 const code = codes[i];
+  u32 const code = codes[i] & 0xffffu;
   u32 const tpm = k_sw_sizes[rs];
   unsigned char const* mesh = k_sw_meshes + k_sw_mesh_off[rs] + code * tpm;
   unsigned char const(*tris)[3] = k_sw_tris + k_sw_tri_off[rs];
   u32 const nint = k_sw_nint[rs];
   unsigned char const* ie = k_sw_int + k_sw_int_off[rs] + code * nint * 2;
   if (out1) {
-    u32* o = out1 + (size_t) goff1[i] * 2;
+    u32* o = out1 + (size_t) g1 * 2;
     for (u32 k = 0; k < nint; ++k) {
       o[2 * k] = ring_v[ie[2 * k]];
       o[2 * k + 1] = ring_v[ie[2 * k + 1]];
     }
   }
+  if (RUN) {
+    // the products' class (the swapped edge's) and their other arrays
+    u32 const cd = R.ecd[i], ci = R.eci ? R.eci[i] : 0u;
+    for (u32 k = 0; k < nint; ++k) {
+      u32 const n = R.nE + g1 + k;
+      R.ecd[n] = cd;
+      if (R.eci) R.eci[n] = ci;
+      R.death[n] = 0;
+      R.info[n] = cd == 3 ? 0u : RI_KNOWN;
+      R.lb[n] = 0;
+      R.ln[n] = 0;
+      R.cnt[n] = 0;
+      R.sa[n] = 0;
+      R.sb[n] = 0;
+    }
+    u32 const nf = tpm + 2 * nint;
+    for (u32 k = 0; k < nf; ++k) {
+      u32 const n = R.nF + g2 + k;
+      R.fcd[n] = cd;
+      if (R.fci) R.fci[n] = ci;
+      R.fbirth[n - R.nF0] = R.pass;
+    }
+    for (u32 k = 0; k < 2 * tpm; ++k) {
+      u32 const n = R.nT + g3 + k;
+      R.tcd[n] = cd;
+      if (R.tci) R.tci[n] = ci;
+      R.dead[n] = 0;
+    }
+  }
   if (out2) {
-    u32* o = out2 + (size_t) goff2[i] * 3;
+    u32* o = out2 + (size_t) g2 * 3;
     for (u32 k = 0; k < nint; ++k)
       for (u32 j = 0; j < 2; ++j) {
         o[k * 6 + j * 3 + 0] = ring_v[ie[2 * k]];
@@ -2580,7 +2676,6 @@ __global__ __launch_bounds__(BLOCK) void swap_products_k(
     for (u32 t = 0; t < tpm; ++t)
       for (u32 j = 0; j < 3; ++j) o[t * 3 + j] = ring_v[tris[mesh[t]][j]];
   }
-  u32 const f = uo[i], e = uo[i + 1];
   for (u32 k = 0; E.out && k < rs; ++k) {
     u32 const a = ring_v[k], b = ring_v[k + 1 < rs ? k + 1 : 0];
     u32 tet = INVALID;
@@ -2607,13 +2702,13 @@ __global__ __launch_bounds__(BLOCK) void swap_products_k(
       if (tv[c] == edge_v[1]) l1 = c;
     }
     s_tet[k][tid] = tet;
-    s_ring[k][tid] = E.soff1[te[tet_edge_between(la, lb)]];
-    s_spoke[0][k][tid] = E.soff1[te[tet_edge_between(la, l0)]];
-    s_spoke[1][k][tid] = E.soff1[te[tet_edge_between(la, l1)]];
+    s_ring[k][tid] = edge_now(te[tet_edge_between(la, lb)]);
+    s_spoke[0][k][tid] = edge_now(te[tet_edge_between(la, l0)]);
+    s_spoke[1][k][tid] = edge_now(te[tet_edge_between(la, l1)]);
   }
   if (!out3) return;
-  u32* o3 = out3 + (size_t) goff3[i] * 4;
-  u32 const first = E.nsame3 + goff3[i];
+  u32* o3 = out3 + (size_t) g3 * 4;
+  u32 const first = E.nsame3 + g3;
   for (u32 t = 0; t < tpm; ++t) {
     u32 lab[4], tv[4];  // labels: ring slot, or 8 + edge end; vertices
     for (u32 j = 0; j < 3; ++j) {
@@ -2648,7 +2743,7 @@ __global__ __launch_bounds__(BLOCK) void swap_products_k(
         } else {
           for (u32 k = 0; k < nint; ++k)
             if ((ie[2 * k] == a && ie[2 * k + 1] == b) || (ie[2 * k] == b && ie[2 * k + 1] == a))
-              id = E.nsame1 + E.goff1[i] + k;
+              id = E.nsame1 + g1 + k;
         }
         if (id == INVALID) *E.err = ERR_REFLECT_NOT_FOUND;
         eo[le] = id;
@@ -2686,7 +2781,11 @@ __global__ __launch_bounds__(BLOCK) void swap_products_k(
               u32 const o = E.old_dual[4 * (size_t) tk + lf];
               if (o == INVALID) {
                 nb = INVALID;
-              } else if (E.soff3[o] != E.soff3[o + 1]) {
+              } else if (RUN && !R.dead[o]) {
+                nb = o;
+                for (u32 q = 0; q < 4; ++q)
+                  if (E.dual[4 * (size_t) o + q] == tk) E.dual[4 * (size_t) o + q] = self;
+              } else if (!RUN && E.soff3[o] != E.soff3[o + 1]) {
                 nb = E.soff3[o];
               } else {
                 nb = DUAL_PENDING;
@@ -2716,18 +2815,21 @@ __global__ __launch_bounds__(BLOCK) void swap_products_k(
   }
 }
 
+// the product across a removed tet n's face shared with the tet from
+__device__ inline u32 swap_across(SwapEdgesOf const& E, u32 n, u32 from) {
+  for (u32 g = 0; g < 4; ++g)
+    if (E.old_dual[4 * (size_t) n + g] == from) return E.face_prod[4 * (size_t) n + g];
+  *E.err = ERR_REFLECT_NOT_FOUND;
+  return INVALID;
+}
+
 // The new dual's remaining entries: threads [0, nt_old) give a surviving
 // tet its neighbours (a surviving one renumbered, a removed one replaced by
 // the product now across that face); the ngen3 * 4 after them resolve a
 // product face whose outside tet was removed by another cavity.
 __global__ __launch_bounds__(BLOCK) void swap_dual_k(u32 nt_old, u32 ngen3, SwapEdgesOf E) {
   u32 const s = xcd_block() * BLOCK + threadIdx.x;
-  auto across = [&](u32 n, u32 from) -> u32 {  // the product across n's face shared with from
-    for (u32 g = 0; g < 4; ++g)
-      if (E.old_dual[4 * (size_t) n + g] == from) return E.face_prod[4 * (size_t) n + g];
-    *E.err = ERR_REFLECT_NOT_FOUND;
-    return INVALID;
-  };
+  auto across = [&](u32 n, u32 from) { return swap_across(E, n, from); };
   if (s < nt_old) {
     u32 const o = E.soff3[s];
     if (o == E.soff3[s + 1]) return;
@@ -2813,6 +2915,19 @@ __host__ __device__ inline u32 swap_pair_slot(unsigned long long key, u32 mask) 
   key *= 0xBF58476D1CE4E5B9ull;
   key ^= key >> 32;
   return (u32) key & mask;
+}
+
+// in the mixed mode the FP32 screen is a variant chosen online: it pays only
+// where it rejects enough candidates (most swap candidates improve their
+// cavity and need their exact FP64 value anyway)
+static Tuner& swap_tuner() {
+  static thread_local Tuner tuner("swap_quality_3d_mixed", {0, 1});
+  return tuner;
+}
+static bool swap_screen_pinned() {
+  if (!swap_tuner().forced()) return false;
+  hipEvent_t a = nullptr, b = nullptr;
+  return swap_tuner().pick(1, &a, &b) == 1;
 }
 
 // swap_common + swap_interior + swap_ents (swap.cpp:27-136)
@@ -2913,10 +3028,6 @@ static u32 swap_common(Mesh& m, Buf<u32>& cand, double const* eq_given = nullptr
                      scratch_words(), tag, dev_error_word(), sst);
       }
     };
-    // in the mixed mode the FP32 screen is a variant chosen online: it pays
-    // only where it rejects enough candidates (most swap candidates improve
-    // their cavity and need their exact FP64 value anyway)
-    static thread_local Tuner tuner("swap_quality_3d_mixed", {0, 1});
     auto run = [&](u32 screen, hipEvent_t ea, hipEvent_t eb) {
       if (screen)
         mts ? go(swap_quality_k<true, true>, "swap_quality_mixed", ea, eb)
@@ -2926,7 +3037,7 @@ static u32 swap_common(Mesh& m, Buf<u32>& cand, double const* eq_given = nullptr
             : go(swap_quality_k<false, false>, "swap_quality_f64", ea, eb);
     };
     if (g_mixed)
-      tuned(tuner, ncand, run);
+      tuned(swap_tuner(), ncand, run);
     else
       run(0, nullptr, nullptr);
   }
@@ -3092,7 +3203,6 @@ static u32 swap_common(Mesh& m, Buf<u32>& cand, double const* eq_given = nullptr
     E.out = d31.get();
     E.old = ask_down(m, 3, 1);
     E.soff1 = soffs[1].get();
-    E.goff1 = goffs[1].get();
     E.nsame1 = tots[2];
     E.nsame3 = nsame3;
     E.err = dev_error_word();
@@ -3108,9 +3218,9 @@ static u32 swap_common(Mesh& m, Buf<u32>& cand, double const* eq_given = nullptr
       E.deferred = deferred.get();
     }
   }
-  launch_timed("swap_cavity", prof_bytes, swap_products_k, dim3(nblocks(ne)), dim3(BLOCK), ne, is,
+  launch_timed("swap_cavity", prof_bytes, swap_products_k<false>, dim3(nblocks(ne)), dim3(BLOCK), ne, is,
                goffs[1].get(), goffs[2].get(), goffs[3].get(), u.offsets.get(), u.adj.get(), u.dirs.get(), ev, vt,
-               codes.get(), pouts[1], pouts[2], pouts[3], E);
+               codes.get(), pouts[1], pouts[2], pouts[3], E, SwapRunView{});
   if (E.dual) {
     hipLaunchKernelGGL(swap_dual_k, dim3(nblocks((size_t) nt_old + (size_t) ngen3 * 4)), dim3(BLOCK), 0, stream(),
                        nt_old, ngen3, E);
@@ -3224,6 +3334,972 @@ u32 swap_slivers(Mesh& m, double good_qual, u32 nlayers, double const* eq, doubl
   return swap_common(m, c, eq, cache);
 }
 
+// ------------------------------------------------- swap passes in place
+// The shape loop's consecutive swap passes (adapt.cpp:58-80) on one copy of
+// the mesh that is changed in place.  A pass through swap_common writes a
+// whole new mesh, although it changes only its cavities and the passes of a
+// run change ever fewer: on the 44^3 x 6 anisotropic box (2.2 to 4 million
+// tets) a run's passes swap 412936, 276154, ... 11, 5, 1 edges, and each
+// cost 2.4 ms of rewriting, renumbering and patching everything (all swap
+// passes of that adapt: about 650 of 1309 ms of kernel time; in place 290 of 907).  Here
+// entities keep their places: a pass marks what it removes, appends its
+// products, and rewrites the tet lists of the edges around its cavities.
+// swap_common's numbering (survivors in order, then products in the order of
+// their swapped edges) is the order of the places in use, so every comparison
+// of indices (ties in the independent set, the order of a list, where a ring
+// starts) comes out the same, and closing the gaps once, after the run's
+// last pass, gives the mesh that pass by pass rewriting gives.
+//
+// What is left per pass over the whole mesh is bound by bandwidth and small:
+// the sliver marks (a byte per tet, their layers through the dual: 17 bytes
+// read per tet and layer, the bytes gathered from L2), the edges' words (4
+// bytes each; the tets of an edge are visited only where its swap is accepted
+// or not yet known) and the states (a byte per edge).  The rest is as long as
+// the pass's candidates or cavities.  One wait of the host per pass.
+//
+// A face survives a swap pass unless it holds the swapped edge, that is,
+// both its vertices (swap.cpp:41-45), and the passes do not read faces, so
+// the faces are settled once: each removed edge's vertex pair goes into a
+// hash table with the last pass that removed it, and a face is gone if one
+// of its pairs was removed in a pass after the one that made the face.
+
+// the index for each lane with pred among those of the launch, one atomic
+// per wave; every lane of the wave must call it
+__device__ inline u32 wave_append(u32* counter, bool pred) {
+  unsigned long long const m = __ballot(pred);
+  if (!m) return 0;
+  u32 const lane = (u32) __lane_id(), leader = (u32) (__ffsll((long long) m) - 1);
+  u32 base = 0;
+  if (lane == leader) base = atomicAdd(counter, (u32) __popcll(m));
+  base = (u32) __shfl((int) base, (int) leader);
+  return base + (u32) __popcll(m & ((1ull << lane) - 1ull));
+}
+
+constexpr u32 RUN_RED_BLOCKS = 1024;
+
+// slivers (marks a byte per tet, mark.cpp:202-232) and the quality minimum
+// over the live tets but the first (the serial doubles_min starts at 1);
+// block 0 clears the pass's counters
+__global__ __launch_bounds__(BLOCK) void run_slivers_k(SwapRunView R, double const* __restrict__ tq, double good,
+                                                       unsigned char* __restrict__ marks,
+                                                       double* __restrict__ part) {
+  __shared__ double lds[BLOCK / 64];
+  if (blockIdx.x == 0 && threadIdx.x < RW_WORDS && threadIdx.x != RW_POOL && threadIdx.x != RW_FIRST)
+    R.words[threadIdx.x] = 0;
+  u32 const first = R.words[RW_FIRST];
+  double v = 1.7976931348623157e308;
+  for (u32 t = blockIdx.x * BLOCK + threadIdx.x; t < R.nT; t += gridDim.x * BLOCK) {
+    bool const live = !R.dead[t];
+    double const q = tq[t];
+    marks[t] = live && q < good ? 1 : 0;
+    if (live && t != first && q < v) v = q;
+  }
+#pragma unroll
+  for (u32 d = 32; d >= 1; d >>= 1) {
+    double o = __shfl_down(v, d, 64);
+    if (o < v) v = o;
+  }
+  if ((threadIdx.x & 63u) == 0) lds[threadIdx.x >> 6] = v;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    double r = lds[0];
+    for (u32 w = 1; w < BLOCK / 64; ++w)
+      if (lds[w] < r) r = lds[w];
+    part[blockIdx.x] = r;
+  }
+}
+
+// one layer of mesh_mark_dual_layers (mark.cpp:90-126)
+__global__ __launch_bounds__(BLOCK) void run_layer_k(u32 n, uint4 const* __restrict__ dual,
+                                                     unsigned char const* __restrict__ in,
+                                                     unsigned char* __restrict__ out) {
+  u32 const t = blockIdx.x * BLOCK + threadIdx.x;
+  if (t >= n) return;
+  unsigned char r = in[t];
+  if (!r) {
+    uint4 const d = dual[t];
+    r = ((d.x != INVALID && in[d.x]) || (d.y != INVALID && in[d.y]) || (d.z != INVALID && in[d.z]) ||
+         (d.w != INVALID && in[d.w]))
+            ? 1
+            : 0;
+  }
+  out[t] = r;
+}
+
+// the candidates: live interior edges of marked tets whose swap is accepted
+// (they enter the independent set) or not yet known (to be evaluated)
+__global__ __launch_bounds__(BLOCK) void run_candidates_k(SwapRunView R, unsigned char const* __restrict__ marks) {
+  u32 const e = blockIdx.x * BLOCK + threadIdx.x;
+  bool acc = false, ask = false;
+  if (e < R.nE) {
+    u32 const w = R.info[e];
+    if (!(w & RI_KNOWN) || (w & RI_ACCEPT)) {
+      bool in = false;
+      u32 const f = R.lb[e], n = R.ln[e];
+      for (u32 k = 0; k < n && !in; ++k) in = marks[R.ua[f + k]] != 0;
+      acc = in && (w & RI_KNOWN);
+      ask = in && !(w & RI_KNOWN);
+    }
+  }
+  u32 const a = wave_append(R.words + RW_ACC, acc), b = wave_append(R.words + RW_EVAL, ask);
+  if (acc) {
+    R.acc[a] = e;
+    R.sa[e] = UNKNOWN;
+  }
+  if (ask) R.eval[b] = e;
+}
+
+// swap qualities of the candidates to evaluate: the choice goes into the
+// edge's word, an accepted edge joins the accepted candidates
+template <bool MT, bool MIXED>
+__global__ __launch_bounds__(BLOCK, 4) void run_quality_k(SwapRunView R, double const* __restrict__ x,
+                                                          double const* __restrict__ mt,
+                                                          double const* __restrict__ tq, u32* __restrict__ err,
+                                                          ScreenStats st) {
+  __shared__ SwapLds<MT> L;
+  u32 const n = R.words[RW_EVAL];
+  u32 const group = threadIdx.x / SW_G;
+  bool const lead = threadIdx.x % SW_G == 0;
+  for (u32 base = blockIdx.x * SW_EDGES; base < n; base += gridDim.x * SW_EDGES) {
+    u32 e, rs, code;
+    bool settled;
+    double best;
+    bool const accept = swap_quality_batch<MT, MIXED>(L, n, base + group, R.eval, R.lb, R.ln, R.ua, R.ud, R.ev, R.vt,
+                                                      x, mt, tq, err, st, &e, &settled, &best, &rs, &code);
+    u32 const a = wave_append(R.words + RW_ACC, accept && lead);
+    if (settled && lead) {
+      R.info[e] = accept ? RI_KNOWN | RI_ACCEPT | (rs << 16) | code : RI_KNOWN;
+      if (accept) {
+        R.q[e] = best;
+        R.acc[a] = e;
+        R.sa[e] = UNKNOWN;
+      }
+    }
+    __syncthreads();  // the next batch reuses the staging
+  }
+}
+
+// indset_round_elems over the accepted candidates (every other edge is out,
+// in both states)
+__global__ __launch_bounds__(BLOCK) void run_round_k(SwapRunView R, unsigned char const* __restrict__ old,
+                                                     unsigned char* __restrict__ state, u32* __restrict__ flag) {
+  u32 const n = R.words[RW_ACC];
+  bool undecided = false;
+  for (u32 k = blockIdx.x * BLOCK + threadIdx.x; k < n; k += gridDim.x * BLOCK) {
+    u32 const i = R.acc[k];
+    u32 s = old[i];
+    if (s == UNKNOWN) {
+      double const myg = R.q[i];
+      bool wait = false, out = false;
+      u32 const f = R.lb[i], l = R.ln[i];
+      for (u32 j = f; j < f + l && !out; ++j) {
+        u32 const t = R.ua[j], d = R.ud[j];
+        for (u32 c = 0; c < 6; ++c) {
+          if (c == d) continue;
+          u32 const o = R.te[6 * (size_t) t + c];
+          if (o >= R.nE) continue;  // a product's edge that was not found (reported)
+          u32 const so = old[o];
+          if (so == IN_SET) {
+            out = true;
+            break;
+          }
+          if (so == NOT_IN_SET || wait) continue;
+          double const og = R.q[o];
+          if ((myg == og && o < i) || myg < og) wait = true;
+        }
+      }
+      s = out ? (u32) NOT_IN_SET : (wait ? (u32) UNKNOWN : (u32) IN_SET);
+      undecided = undecided || (!out && wait);
+    }
+    state[i] = (unsigned char) s;
+  }
+  wave_flag(flag, undecided);
+}
+
+// What a swapped edge makes and needs: itself, product edges, faces and
+// tets, and at most how many list places its surroundings' survivors take
+struct RunCount {
+  u32 v[5];
+};
+constexpr u32 RUN_PER = 8;  // edges per thread of the two counting kernels
+
+__device__ inline void run_count_edge(SwapRunView const& R, u32 e, RunCount& c, bool need) {
+  u32 const w = R.info[e], rs = (w >> 16) & 0xffu;
+  u32 const nint = k_sw_nint[rs], tpm = k_sw_sizes[rs];
+  c.v[0] += 1;
+  c.v[1] += nint;
+  c.v[2] += count_swap_ents(rs, 2, nint, tpm);
+  c.v[3] += count_swap_ents(rs, 3, nint, tpm);
+  if (!need) return;
+  u32 const f = R.lb[e], n = R.ln[e];
+  for (u32 j = f; j < f + n; ++j)
+    for (u32 k = 0; k < 6; ++k) {
+      u32 const o = R.te[6 * (size_t) R.ua[j] + k];
+      c.v[4] += o < R.nE ? R.ln[o] : 0u;
+    }
+}
+
+// exclusive prefix of c over the block's threads (first N words), totals in *tot
+template <u32 N>
+__device__ inline void run_block_scan(RunCount& c, RunCount* tot, u32 (*lds)[5]) {
+  u32 const lane = threadIdx.x & 63u, wave = threadIdx.x >> 6, nw = blockDim.x >> 6;
+#pragma unroll
+  for (u32 k = 0; k < N; ++k) {
+    u32 const mine = c.v[k];
+    u32 x = mine;
+#pragma unroll
+    for (u32 d = 1; d < 64; d <<= 1) {
+      u32 const y = (u32) __shfl_up((int) x, d, 64);
+      if (lane >= d) x += y;
+    }
+    if (lane == 63u) lds[wave][k] = x;
+    c.v[k] = x - mine;
+  }
+  __syncthreads();
+#pragma unroll
+  for (u32 k = 0; k < N; ++k) {
+    u32 off = 0, all = 0;
+    for (u32 w = 0; w < nw; ++w) {
+      if (w < wave) off += lds[w][k];
+      all += lds[w][k];
+    }
+    c.v[k] += off;
+    tot->v[k] = all;
+  }
+  __syncthreads();
+}
+
+// per block of BLOCK * RUN_PER edges: the totals of its swapped edges
+__global__ __launch_bounds__(BLOCK) void run_count_k(SwapRunView R, unsigned char const* __restrict__ state,
+                                                     RunCount* __restrict__ part) {
+  __shared__ u32 lds[BLOCK / 64][5];
+  u32 const e0 = (blockIdx.x * BLOCK + threadIdx.x) * RUN_PER;
+  RunCount c{}, tot;
+  if (e0 < R.nE) {
+    // the states are padded with zeros to a multiple of RUN_PER
+    unsigned long long const w = *reinterpret_cast<unsigned long long const*>(state + e0);
+    if (w)
+      for (u32 k = 0; k < RUN_PER; ++k)
+        if (((w >> (8 * k)) & 0xffu) == IN_SET) run_count_edge(R, e0 + k, c, true);
+  }
+  run_block_scan<5>(c, &tot, lds);
+  if (threadIdx.x == 0) part[blockIdx.x] = tot;
+}
+
+// one block: the blocks' totals become their first products, and the totals,
+// the pool's top, the set's flag and the quality minimum go to the host
+__global__ __launch_bounds__(1024) void run_offsets_k(u32 nb, RunCount* __restrict__ part, u32 npart,
+                                                      double const* __restrict__ qpart, SwapRunView R,
+                                                      u32 const* __restrict__ flag, u32* __restrict__ host,
+                                                      double* __restrict__ host_min) {
+  __shared__ u32 lds[16][5];
+  __shared__ double mins[16];
+  u32 const per = (nb + 1023) / 1024, b = threadIdx.x * per, e = b + per < nb ? b + per : nb;
+  RunCount c{}, tot;
+  for (u32 i = b; i < e; ++i)
+    for (u32 k = 0; k < 5; ++k) c.v[k] += part[i].v[k];
+  run_block_scan<5>(c, &tot, lds);
+  for (u32 i = b; i < e; ++i)
+    for (u32 k = 0; k < 4; ++k) {
+      u32 const n = part[i].v[k];
+      part[i].v[k] = c.v[k];
+      c.v[k] += n;
+    }
+  double v = 1.7976931348623157e308;
+  for (u32 i = threadIdx.x; i < npart; i += 1024)
+    if (qpart[i] < v) v = qpart[i];
+#pragma unroll
+  for (u32 d = 32; d >= 1; d >>= 1) {
+    double o = __shfl_down(v, d, 64);
+    if (o < v) v = o;
+  }
+  if ((threadIdx.x & 63u) == 0) mins[threadIdx.x >> 6] = v;
+  __syncthreads();
+  if (threadIdx.x != 0) return;
+  for (u32 w = 1; w < 16; ++w)
+    if (mins[w] < v) v = mins[w];
+  for (u32 k = 0; k < 5; ++k) host[k] = tot.v[k];
+  host[5] = R.words[RW_POOL];
+  host[6] = *flag;
+  *host_min = v;
+}
+
+// the swapped edges in order with their first products; each is removed
+// with the tets around it
+__global__ __launch_bounds__(BLOCK) void run_list_k(SwapRunView R, unsigned char const* __restrict__ state,
+                                                    RunCount const* __restrict__ part) {
+  __shared__ u32 lds[BLOCK / 64][5];
+  u32 const e0 = (blockIdx.x * BLOCK + threadIdx.x) * RUN_PER;
+  RunCount c{}, tot;
+  unsigned long long w = 0;
+  if (e0 < R.nE) w = *reinterpret_cast<unsigned long long const*>(state + e0);
+  if (w)
+    for (u32 k = 0; k < RUN_PER; ++k)
+      if (((w >> (8 * k)) & 0xffu) == IN_SET) run_count_edge(R, e0 + k, c, false);
+  run_block_scan<4>(c, &tot, lds);
+  if (!w) return;
+  RunCount const base = part[blockIdx.x];
+  for (u32 k = 0; k < 4; ++k) c.v[k] += base.v[k];
+  for (u32 k = 0; k < RUN_PER; ++k) {
+    if (((w >> (8 * k)) & 0xffu) != IN_SET) continue;
+    u32 const e = e0 + k, s = c.v[0];
+    R.sw[s] = e;
+    R.o1[s] = c.v[1];
+    R.o2[s] = c.v[2];
+    R.o3[s] = c.v[3];
+    run_count_edge(R, e, c, false);
+    R.death[e] = R.pass;
+    R.info[e] &= ~RI_ACCEPT;  // the ring size and triangulation stay for the products
+    u32 const f = R.lb[e], n = R.ln[e];
+    for (u32 j = f; j < f + n; ++j) R.dead[R.ua[j]] = 1;
+  }
+}
+
+// every use of an edge by a product tet takes a place among its edge's
+// product uses; the edge's first one puts the edge on the list of changed
+// edges
+__global__ __launch_bounds__(BLOCK) void run_touch_k(SwapRunView R, u32 nuse, u32* __restrict__ slot,
+                                                     u32* __restrict__ changed) {
+  u32 const u = blockIdx.x * BLOCK + threadIdx.x;
+  bool first = false;
+  u32 e = 0;
+  if (u < nuse) {
+    e = R.te[6 * (size_t) R.nT + u];
+    u32 const s = e != INVALID ? atomicAdd(&R.cnt[e], 1u) : 1u;
+    slot[u] = s;
+    first = s == 0;
+  }
+  u32 const a = wave_append(R.words + RW_AFF, first);
+  if (first) changed[a] = e;
+}
+
+// a changed edge's new list: a place in the pool for its surviving and its
+// product uses, the survivors copied in order; cnt is then the survivors'
+// number.  Its swap is not known any more.
+__global__ __launch_bounds__(BLOCK) void run_lists_k(SwapRunView R, u32 const* __restrict__ changed) {
+  u32 const i = blockIdx.x * BLOCK + threadIdx.x;
+  u32 const n = R.words[RW_AFF];
+  u32 e = 0, f = 0, l = 0, s = 0, len = 0;
+  if (i < n) {
+    e = changed[i];
+    f = R.lb[e];
+    l = R.ln[e];
+    for (u32 k = f; k < f + l; ++k) s += R.dead[R.ua[k]] ? 0u : 1u;
+    len = s + R.cnt[e];
+  }
+  // one atomic per wave
+  u32 const lane = (u32) __lane_id();
+  u32 x = len;
+#pragma unroll
+  for (u32 d = 1; d < 64; d <<= 1) {
+    u32 const y = (u32) __shfl_up((int) x, d, 64);
+    if (lane >= d) x += y;
+  }
+  u32 base = 0;
+  if (lane == 63u && x) base = atomicAdd(R.words + RW_POOL, x);
+  base = (u32) __shfl((int) base, 63) + x - len;
+  if (i >= n) return;
+  u32 p = base;
+  for (u32 k = f; k < f + l; ++k) {
+    u32 const t = R.ua[k];
+    if (R.dead[t]) continue;
+    R.ua[p] = t;
+    R.ud[p] = R.ud[k];
+    ++p;
+  }
+  R.lb[e] = base;
+  R.ln[e] = len;
+  R.cnt[e] = s;
+  R.info[e] = R.ecd[e] == 3 ? 0u : RI_KNOWN;
+}
+
+__global__ __launch_bounds__(BLOCK) void run_place_k(SwapRunView R, u32 nuse, u32 const* __restrict__ slot) {
+  u32 const u = blockIdx.x * BLOCK + threadIdx.x;
+  if (u >= nuse) return;
+  u32 const key = 6 * R.nT + u, e = R.te[key];
+  if (e != INVALID) R.ua[R.lb[e] + R.cnt[e] + slot[u]] = key;
+}
+
+// a changed edge's product uses in ascending order (a few: insertion sort)
+__global__ __launch_bounds__(BLOCK) void run_sort_k(SwapRunView R, u32 const* __restrict__ changed) {
+  u32 const i = blockIdx.x * BLOCK + threadIdx.x;
+  if (i >= R.words[RW_AFF]) return;
+  u32 const e = changed[i];
+  u32 const b = R.lb[e] + R.cnt[e], end = R.lb[e] + R.ln[e];
+  for (u32 k = b + 1; k < end; ++k) {
+    u32 const v = R.ua[k];
+    u32 j = k;
+    for (; j > b && R.ua[j - 1] > v; --j) R.ua[j] = R.ua[j - 1];
+    R.ua[j] = v;
+  }
+  for (u32 k = b; k < end; ++k) {
+    u32 const v = R.ua[k], t = v / 6;
+    R.ua[k] = t;
+    R.ud[k] = v - 6 * t;
+  }
+  R.cnt[e] = 0;
+}
+
+// product faces between two cavities of the pass (swap_dual_k); the accepted
+// candidates' states are cleared and the first live tet is found again
+__global__ __launch_bounds__(BLOCK) void run_settle_k(SwapRunView R, u32 n3, SwapEdgesOf E) {
+  u32 const i = blockIdx.x * BLOCK + threadIdx.x;
+  if (i < 4 * n3) {
+    u32* d = R.dual + 4 * (size_t) R.nT + i;
+    if (*d == DUAL_PENDING) {
+      u32 const key = E.deferred[i];
+      *d = swap_across(E, E.old_dual[key], key / 4);
+    }
+  }
+  u32 const n = R.words[RW_ACC];
+  for (u32 k = i; k < n; k += gridDim.x * BLOCK) {
+    u32 const e = R.acc[k];
+    R.sa[e] = 0;
+    R.sb[e] = 0;
+  }
+  if (blockIdx.x == 0 && threadIdx.x < 64) {
+    u32 f = R.words[RW_FIRST];
+    u32 const nt = R.nT + n3;
+    for (;;) {
+      u32 const t = f + threadIdx.x;
+      unsigned long long const m = __ballot(t < nt && !R.dead[t]);
+      if (m) {
+        f += (u32) (__ffsll((long long) m) - 1);
+        break;
+      }
+      f += 64;
+      if (f >= nt) break;
+    }
+    if (threadIdx.x == 0) R.words[RW_FIRST] = f;
+  }
+}
+
+// the last pass that removed each vertex pair
+__global__ __launch_bounds__(BLOCK) void run_pairs_k(SwapRunView R, u32 mask, unsigned long long* __restrict__ keys,
+                                                     u32* __restrict__ when, u32* __restrict__ err) {
+  u32 const e = blockIdx.x * BLOCK + threadIdx.x;
+  if (e >= R.nE) return;
+  u32 const p = R.death[e];
+  if (!p) return;
+  unsigned long long const key = swap_pair_key(R.ev[2 * (size_t) e], R.ev[2 * (size_t) e + 1]);
+  u32 h = swap_pair_slot(key, mask);
+  for (u32 probe = 0; probe <= mask; ++probe, h = (h + 1) & mask) {
+    unsigned long long const k = atomicCAS(&keys[h], ~0ull, key);
+    if (k == ~0ull || k == key) {
+      atomicMax(&when[h], p);
+      return;
+    }
+  }
+  *err = ERR_REFLECT_NOT_FOUND;
+}
+
+// the live entities of one dimension, renumbered into the new mesh
+struct RunOut {
+  u32 n, vpe;
+  u32 const* rank;  // n + 1
+  u32 const* v;
+  u32 const* cd;
+  u32 const* ci;
+  u32* out;
+  u32* out_cd;
+  u32* out_ci;
+  // edges: choices and values, and the lists' lengths
+  u32 const* info;
+  double const* q;
+  u32 const* ln;
+  u32* out_info;
+  double* out_q;
+  u32* out_ln;
+  // tets: edges, dual, qualities
+  u32 const* te;
+  u32 const* dual;
+  double const* tq;
+  u32 const* erank;
+  u32* out_te;
+  u32* out_dual;
+  double* out_tq;
+};
+__global__ __launch_bounds__(BLOCK) void run_out_k(RunOut a) {
+  u32 const i = blockIdx.x * BLOCK + threadIdx.x;
+  if (i >= a.n) return;
+  u32 const o = a.rank[i];
+  if (o == a.rank[i + 1]) return;
+  for (u32 j = 0; j < a.vpe; ++j) a.out[(size_t) o * a.vpe + j] = a.v[(size_t) i * a.vpe + j];
+  a.out_cd[o] = a.cd[i];
+  if (a.out_ci) a.out_ci[o] = a.ci[i];
+  if (a.out_ln) a.out_ln[o] = a.ln[i];
+  if (a.out_info) {
+    a.out_info[o] = a.info[i];
+    a.out_q[o] = a.q[i];
+  }
+  if (a.out_te) {
+    for (u32 j = 0; j < 6; ++j) a.out_te[6 * (size_t) o + j] = a.erank[a.te[6 * (size_t) i + j]];
+    for (u32 j = 0; j < 4; ++j) {
+      u32 const d = a.dual[4 * (size_t) i + j];
+      a.out_dual[4 * (size_t) o + j] = d == INVALID ? INVALID : a.rank[d];
+    }
+    a.out_tq[o] = a.tq[i];
+  }
+}
+
+// the live edges' lists in the new mesh's numbering (RUN_LG lanes an edge)
+constexpr u32 RUN_LG = 4;
+__global__ __launch_bounds__(BLOCK) void run_up_k(SwapRunView R, u32 const* __restrict__ erank,
+                                                  u32 const* __restrict__ trank, u32 const* __restrict__ off,
+                                                  u32* __restrict__ adj, u32* __restrict__ dirs) {
+  size_t const gid = (size_t) blockIdx.x * BLOCK + threadIdx.x;
+  u32 const e = (u32) (gid / RUN_LG), lane = (u32) (gid % RUN_LG);
+  if (e >= R.nE) return;
+  u32 const o = erank[e];
+  if (o == erank[e + 1]) return;
+  u32 const f = R.lb[e], n = R.ln[e], p = off[o];
+  for (u32 k = lane; k < n; k += RUN_LG) {
+    adj[p + k] = trank[R.ua[f + k]];
+    dirs[p + k] = R.ud[f + k];
+  }
+}
+
+namespace {
+struct SwapRun {
+  Mesh& m;
+  Buf<u32> ev, ecd, eci, death, info, lb, ln, cnt, ua, ud, vt, te, dual, tcd, tci, fv, fcd, fci, fbirth, face_prod;
+  Buf<u32> acc, eval, words;
+  Buf<double> q, tq, qpart;
+  Buf<unsigned char> sa, sb, dead, marks, marks2;
+  Buf<RunCount> part;
+  u32 nE = 0, nF = 0, nT = 0, nF0 = 0, aE = 0, aF = 0, aT = 0, pass = 0, pool = 0;
+  bool has_id = false;
+  bool limit_hit = false;  // the independent set reached its round limit
+  u32 got[7];
+  double min_q = 0;
+
+  explicit SwapRun(Mesh& mesh) : m(mesh) {}
+
+  template <class T>
+  static void need(Buf<T>& b, size_t used, size_t want) {
+    if (b && b.size() >= want) return;
+    Buf<T> n(want + want / 2);
+    if (b) d2d(n.get(), b.get(), used);
+    b = std::move(n);
+  }
+  static size_t room(size_t n) { return n + n / 4 + 1024; }
+  template <class T>
+  static Buf<T> taken(T const* a, size_t n, size_t cap) {
+    Buf<T> b(cap);
+    d2d(b.get(), a, n);
+    return b;
+  }
+  void clear_states(size_t from) {
+    // zero beyond the edges in use: products start out of the set, and the
+    // counting kernels read whole words
+    unsigned char *a = sa.get(), *b = sb.get();
+    u32 const n = (u32) (sa.size() - from);
+    parallel_for(n, OHX_LAMBDA(u32 i) {
+      a[from + i] = 0;
+      b[from + i] = 0;
+    });
+  }
+  void edge_room(u32 want) {
+    if (ev && info.size() >= want) return;
+    size_t const old = sa.size();
+    need(ev, 2 * (size_t) nE, 2 * (size_t) want);
+    need(ecd, nE, want);
+    if (has_id) need(eci, nE, want);
+    need(death, nE, want);
+    need(info, nE, want);
+    need(q, nE, want);
+    need(lb, nE, want);
+    need(ln, nE, want);
+    need(cnt, nE, want);
+    need(acc, nE, want);  // still read: its edges' states are cleared at the pass's end
+    eval = Buf<u32>(info.size());
+    size_t const states = (info.size() + RUN_PER) / RUN_PER * RUN_PER;
+    Buf<unsigned char> a2(states), b2(states);
+    if (old) {
+      d2d(a2.get(), sa.get(), old);
+      d2d(b2.get(), sb.get(), old);
+    }
+    sa = std::move(a2);
+    sb = std::move(b2);
+    clear_states(old);
+  }
+  void tet_room(u32 want) {
+    if (dead && dead.size() >= want) return;
+    need(vt, 4 * (size_t) nT, 4 * (size_t) want);
+    need(te, 6 * (size_t) nT, 6 * (size_t) want);
+    need(dual, 4 * (size_t) nT, 4 * (size_t) want);
+    need(tcd, nT, want);
+    if (has_id) need(tci, nT, want);
+    need(tq, nT, want);
+    need(dead, nT, want);
+    face_prod = Buf<u32>(4 * dead.size());
+    marks = Buf<unsigned char>(dead.size());
+    marks2 = Buf<unsigned char>(dead.size());
+  }
+
+  SwapRunView view() const {
+    SwapRunView R{};
+    R.nE = nE;
+    R.nF = nF;
+    R.nT = nT;
+    R.nF0 = nF0;
+    R.pass = pass;
+    R.ev = ev.get();
+    R.ecd = ecd.get();
+    R.eci = eci.get();
+    R.death = death.get();
+    R.info = info.get();
+    R.q = q.get();
+    R.lb = lb.get();
+    R.ln = ln.get();
+    R.cnt = cnt.get();
+    R.sa = sa.get();
+    R.sb = sb.get();
+    R.ua = ua.get();
+    R.ud = ud.get();
+    R.vt = vt.get();
+    R.te = te.get();
+    R.dual = dual.get();
+    R.tcd = tcd.get();
+    R.tci = tci.get();
+    R.dead = dead.get();
+    R.fv = fv.get();
+    R.fcd = fcd.get();
+    R.fci = fci.get();
+    R.fbirth = fbirth.get();
+    R.acc = acc.get();
+    R.eval = eval.get();
+    R.words = words.get();
+    return R;
+  }
+
+  // the mesh's arrays, with room for products; choices: the edges' words and
+  // values when a run on the same mesh has them already (else null)
+  void begin(double const* qualities, u32 const* known, double const* values) {
+    Up const& u = ask_up(m, 1, 3);
+    u32 const* d31 = ask_down(m, 3, 1);
+    u32 const* du = ask_dual(m);
+    has_id = find_tag(m, 0, "class_id") != nullptr;
+    nE = aE = count(m, 1);
+    nF = aF = nF0 = count(m, 2);
+    nT = aT = count(m, 3);
+    pass = 0;
+    pool = u.adj.size();
+    size_t const cE = room(nE), cF = room(nF), cT = room(nT), cL = pool + pool / 2 + 4096;
+    ev = taken(ask_down(m, 1, 0), 2 * (size_t) nE, 2 * cE);
+    ecd = taken(u32_tag(m, 1, "class_dim"), nE, cE);
+    vt = taken(ask_down(m, 3, 0), 4 * (size_t) nT, 4 * cT);
+    te = taken(d31, 6 * (size_t) nT, 6 * cT);
+    dual = taken(du, 4 * (size_t) nT, 4 * cT);
+    tcd = taken(u32_tag(m, 3, "class_dim"), nT, cT);
+    fv = taken(ask_down(m, 2, 0), 3 * (size_t) nF, 3 * cF);
+    fcd = taken(u32_tag(m, 2, "class_dim"), nF, cF);
+    if (has_id) {
+      eci = taken(u32_tag(m, 1, "class_id"), nE, cE);
+      tci = taken(u32_tag(m, 3, "class_id"), nT, cT);
+      fci = taken(u32_tag(m, 2, "class_id"), nF, cF);
+    }
+    fbirth = Buf<u32>(cF - nF);
+    tq = taken(qualities, nT, cT);
+    ua = taken(u.adj.get(), pool, cL);
+    ud = taken(u.dirs.get(), pool, cL);
+    dead = Buf<unsigned char>(cT);
+    marks = Buf<unsigned char>(cT);
+    marks2 = Buf<unsigned char>(cT);
+    face_prod = Buf<u32>(4 * cT);
+    death = Buf<u32>(cE);
+    info = Buf<u32>(cE);
+    q = Buf<double>(cE);
+    lb = Buf<u32>(cE);
+    ln = Buf<u32>(cE);
+    cnt = Buf<u32>(cE);
+    acc = Buf<u32>(cE);
+    eval = Buf<u32>(cE);
+    size_t const states = (cE + RUN_PER) / RUN_PER * RUN_PER;
+    sa = Buf<unsigned char>(states);
+    sb = Buf<unsigned char>(states);
+    qpart = Buf<double>(RUN_RED_BLOCKS);
+    words = Buf<u32>(RW_WORDS);
+    // every array's start values, one launch over the states (the edges and
+    // their room) and the tets
+    SwapRunView R = view();
+    u32 const* off = u.offsets.get();
+    u32 const p0 = pool, ns = (u32) states;
+    parallel_for(ns > nT ? ns : nT, OHX_LAMBDA(u32 i) {
+      if (i < ns) {
+        R.sa[i] = 0;
+        R.sb[i] = 0;
+      }
+      if (i < R.nE) {
+        R.death[i] = 0;
+        R.cnt[i] = 0;
+        R.lb[i] = off[i];
+        R.ln[i] = off[i + 1] - off[i];
+        R.info[i] = R.ecd[i] != 3 ? RI_KNOWN : known ? known[i] : 0u;
+        if (known) R.q[i] = values[i];
+      }
+      if (i < R.nT) R.dead[i] = 0;
+      if (i < RW_WORDS) R.words[i] = i == RW_POOL ? p0 : 0u;
+    });
+  }
+
+  // one swap pass; returns whether it changed the mesh, and sets min_q, the
+  // quality minimum of the mesh before the pass (at least good: no pass)
+  bool step(double good, u32 nlayers) {
+    {
+      // as check_index_space, from the live counts
+      size_t const star = 6 * (size_t) aF + 6 * (size_t) aT;
+      if (2 * star >= ((size_t) 1 << 32)) fail("mesh too large for 32-bit adjacency offsets", __FILE__, __LINE__);
+    }
+    make_swap_tables();
+    ++pass;
+    SwapRunView R = view();
+    u32 const rb = nblocks(nT) < RUN_RED_BLOCKS ? nblocks(nT) : RUN_RED_BLOCKS;
+    hipLaunchKernelGGL(run_slivers_k, dim3(rb), dim3(BLOCK), 0, stream(), R, tq.get(), good, marks.get(),
+                       qpart.get());
+    check_launch("run_slivers");
+    for (u32 l = 0; l < nlayers; ++l) {
+      hipLaunchKernelGGL(run_layer_k, dim3(nblocks(nT)), dim3(BLOCK), 0, stream(), nT,
+                         reinterpret_cast<uint4 const*>(dual.get()), marks.get(), marks2.get());
+      check_launch("run_layer");
+      std::swap(marks, marks2);
+    }
+    hipLaunchKernelGGL(run_candidates_k, dim3(nblocks(nE)), dim3(BLOCK), 0, stream(), R, marks.get());
+    check_launch("run_candidates");
+    evaluate(R);
+    // a first batch of rounds with no host check, as the other passes
+    u32 const first = first_batch_rounds();
+    u32 const gr = nblocks(nE) < 512 ? nblocks(nE) : 512;
+    unsigned char *a = sa.get(), *b = sb.get();
+    u32* flags = words.get() + RW_FLAGS;
+    auto round = [&](u32* fl) {
+      launch_timed("indset_round", (double) nE, run_round_k, dim3(gr), dim3(BLOCK), R, a, b, fl);
+      std::swap(a, b);
+    };
+    for (u32 r = 0; r < first; ++r) round(flags + r);
+    u32 const nb = nblocks(nE, BLOCK * RUN_PER);
+    if (!part || part.size() < nb) part = Buf<RunCount>(nb + nb / 2);
+    u32* hs = host_slot<u32>(SLOT_RUN);
+    u32* ds = dev_slot<u32>(SLOT_RUN);
+    u32 const* flag = flags + first - 1;
+    auto totals = [&] {
+      hipLaunchKernelGGL(run_count_k, dim3(nb), dim3(BLOCK), 0, stream(), R, a, part.get());
+      hipLaunchKernelGGL(run_offsets_k, dim3(1), dim3(1024), 0, stream(), nb, part.get(), rb, qpart.get(), R, flag,
+                         ds, dev_slot<double>(SLOT_RUN_MIN));
+      check_launch("run_offsets");
+      sync();
+      for (u32 k = 0; k < 7; ++k) got[k] = hs[k];
+    };
+    totals();
+    min_q = *host_slot<double>(SLOT_RUN_MIN);
+    if (min_q >= good) return false;
+    if (got[6]) {
+      // not settled in the first batch: checked batches up to the limit
+      rounds_to_the_end(round, flags);
+      flag = words.get() + RW_AFF;  // zero: settled
+      totals();
+    }
+    if (!got[0]) return false;
+    swap(R, a, nb);
+    return true;
+  }
+
+  void evaluate(SwapRunView const& R) {
+    double const* mt = metric_of(m);
+    double const* x = coords(m);
+    u32 const need = (aE + SW_EDGES - 1) / SW_EDGES;
+    dim3 const grid(need < 2048 ? (need ? need : 1) : 2048);
+    ScreenStats st = screen_stats();
+    auto go = [&](auto kernel, char const* kn) {
+      launch_timed(kn, (double) aE * 24, kernel, grid, dim3(BLOCK), R, x, mt, tq.get(), dev_error_word(), st);
+    };
+    // the FP32 screen runs only where it is pinned on: timed on live
+    // launches it lost to FP64 at every size class of the shipped table
+    if (g_mixed && swap_screen_pinned())
+      mt ? go(run_quality_k<true, true>, "swap_quality_mixed") : go(run_quality_k<false, true>, "swap_quality_mixed");
+    else
+      mt ? go(run_quality_k<true, false>, "swap_quality_f64") : go(run_quality_k<false, false>, "swap_quality_f64");
+  }
+
+  template <class F>
+  void rounds_to_the_end(F&& round, u32* flags) {
+    constexpr u32 BATCH = 8;
+    u32 const limit = g_indset_max_rounds;
+    for (u32 done = first_batch_rounds(); done < limit; done += BATCH) {
+      u32 const nr = limit - done < BATCH ? limit - done : BATCH;
+      fill(flags, nr, 0);
+      for (u32 r = 0; r < nr; ++r) round(flags + r);
+      u32 h[BATCH];
+      u32 const* fp[BATCH];
+      for (u32 r = 0; r < nr; ++r) fp[r] = flags + r;
+      read_many(fp, nr, h);
+      if (!h[nr - 1]) {
+        u32 k = 0;
+        while (h[k]) ++k;
+        note_rounds(done + k + 1);
+        return;
+      }
+    }
+    limit_hit = true;
+    fail("independent set did not converge within the round limit (indset.cpp:107-116)", __FILE__, __LINE__);
+  }
+
+  // the run's mesh, gaps closed, becomes m; eq its element qualities, and
+  // known and values (when wanted) its edges' words and values
+  void finish(Buf<double>& eq, Buf<u32>* known, Buf<double>* values) {
+    sync();  // an error of the last pass's kernels shows here, before its output is followed
+    SwapRunView R = view();
+    Buf<u32> er(nE + 1), tr(nT + 1), fr(nF + 1);
+    exscan_fn(nE, OHX_LAMBDA(u32 i) { return R.death[i] ? 0u : 1u; }, er.get());
+    exscan_fn(nT, OHX_LAMBDA(u32 i) { return R.dead[i] ? 0u : 1u; }, tr.get());
+    u32 cap = 64;
+    while (cap < 4 * (size_t) (nE - aE)) cap *= 2;
+    u32 const mask = cap - 1;
+    Buf<unsigned long long> keys(cap);
+    Buf<u32> when(cap);
+    unsigned long long* kp = keys.get();
+    u32* wp = when.get();
+    parallel_for(cap, OHX_LAMBDA(u32 i) {
+      kp[i] = ~0ull;
+      wp[i] = 0;
+    });
+    hipLaunchKernelGGL(run_pairs_k, dim3(nblocks(nE)), dim3(BLOCK), 0, stream(), R, mask, kp, wp, dev_error_word());
+    check_launch("run_pairs");
+    exscan_fn_heavy(nF, OHX_LAMBDA(u32 i) {
+      u32 const* v = R.fv + 3 * (size_t) i;
+      u32 const born = i < R.nF0 ? 0u : R.fbirth[i - R.nF0];
+      for (u32 j = 0; j < 3; ++j) {
+        unsigned long long const key = swap_pair_key(v[j], v[(j + 1) % 3]);
+        for (u32 probe = 0, h = swap_pair_slot(key, mask); probe <= mask; ++probe, h = (h + 1) & mask) {
+          unsigned long long const t = kp[h];
+          if (t == ~0ull) break;
+          if (t != key) continue;
+          if (wp[h] > born) return 0u;
+          break;
+        }
+      }
+      return 1u;
+    }, fr.get());
+    Mesh mo(3, true);
+    set_ents(mo, 0, m.counts[0], Buf<u32>());
+    mo.tags[0] = std::move(m.tags[0]);
+    u32 const alive[4] = {0, aE, aF, aT};
+    Buf<u32> lens(aE), nd31((size_t) 6 * aT), ndual((size_t) 4 * aT);
+    Buf<double> neq(aT);
+    if (known) {
+      *known = Buf<u32>(aE);
+      *values = Buf<double>(aE);
+    }
+    for (u32 d = 1; d <= 3; ++d) {
+      RunOut o{};
+      o.n = d == 1 ? nE : d == 2 ? nF : nT;
+      o.vpe = d + 1;
+      o.rank = d == 1 ? er.get() : d == 2 ? fr.get() : tr.get();
+      o.v = d == 1 ? ev.get() : d == 2 ? fv.get() : vt.get();
+      o.cd = d == 1 ? ecd.get() : d == 2 ? fcd.get() : tcd.get();
+      o.ci = !has_id ? nullptr : d == 1 ? eci.get() : d == 2 ? fci.get() : tci.get();
+      Buf<u32> verts((size_t) alive[d] * (d + 1)), cdo(alive[d]), cio;
+      if (has_id) cio = Buf<u32>(alive[d]);
+      o.out = verts.get();
+      o.out_cd = cdo.get();
+      o.out_ci = cio.get();
+      if (d == 1) {
+        o.ln = ln.get();
+        o.out_ln = lens.get();
+        if (known) {
+          o.info = info.get();
+          o.q = q.get();
+          o.out_info = known->get();
+          o.out_q = values->get();
+        }
+      }
+      if (d == 3) {
+        o.te = te.get();
+        o.dual = dual.get();
+        o.tq = tq.get();
+        o.erank = er.get();
+        o.out_te = nd31.get();
+        o.out_dual = ndual.get();
+        o.out_tq = neq.get();
+      }
+      hipLaunchKernelGGL(run_out_k, dim3(nblocks(o.n)), dim3(BLOCK), 0, stream(), o);
+      check_launch("run_out");
+      set_ents(mo, d, alive[d], std::move(verts));
+      add_tag_u32(mo, d, "class_dim", 1, std::move(cdo));
+      if (has_id) add_tag_u32(mo, d, "class_id", 1, std::move(cio));
+    }
+    auto up = std::make_unique<Up>();
+    up->offsets = exscan(lens.get(), aE);
+    up->adj = Buf<u32>((size_t) 6 * aT);
+    up->dirs = Buf<u32>((size_t) 6 * aT);
+    hipLaunchKernelGGL(run_up_k, dim3(nblocks((size_t) nE * RUN_LG)), dim3(BLOCK), 0, stream(), R, er.get(), tr.get(),
+                       up->offsets.get(), up->adj.get(), up->dirs.get());
+    check_launch("run_up");
+    mo.up[1][3] = std::move(up);
+    mo.down[3][1] = std::move(nd31);
+    mo.dual = std::move(ndual);
+    overwrite(m, std::move(mo));
+    eq = std::move(neq);
+  }
+
+  void swap(SwapRunView R, unsigned char const* state, u32 nb) {
+    u32 const ns = got[0], n1 = got[1], n2 = got[2], n3 = got[3];
+    if (6 * ((size_t) nT + n3) >= ((size_t) 1 << 32) || (size_t) got[5] + got[4] + 6 * (size_t) n3 >= ((size_t) 1 << 32))
+      fail("swap: more than 2^32 uses", __FILE__, __LINE__);
+    edge_room(nE + n1);
+    tet_room(nT + n3);
+    need(fv, 3 * (size_t) nF, 3 * ((size_t) nF + n2));
+    need(fcd, nF, (size_t) nF + n2);
+    if (has_id) need(fci, nF, (size_t) nF + n2);
+    need(fbirth, nF - nF0, (size_t) nF - nF0 + n2);
+    need(ua, got[5], (size_t) got[5] + got[4] + 6 * (size_t) n3);
+    need(ud, got[5], (size_t) got[5] + got[4] + 6 * (size_t) n3);
+    Buf<u32> lists((size_t) 4 * ns), uses((size_t) 12 * n3), deferred((size_t) 4 * n3);
+    // the states may have moved: the round's result is in sa or sb as before
+    bool const in_a = state == R.sa;
+    R = view();
+    state = in_a ? R.sa : R.sb;
+    R.sw = lists.get();
+    R.o1 = R.sw + ns;
+    R.o2 = R.o1 + ns;
+    R.o3 = R.o2 + ns;
+    u32 const nuse = 6 * n3;
+    u32 *slot = uses.get(), *changed = slot + nuse;
+    hipLaunchKernelGGL(run_list_k, dim3(nb), dim3(BLOCK), 0, stream(), R, state, part.get());
+    check_launch("run_list");
+    SwapEdgesOf E{};
+    E.out = R.te;
+    E.old = R.te;
+    E.nsame1 = nE;
+    E.nsame3 = nT;
+    E.err = dev_error_word();
+    E.dual = R.dual;
+    E.old_dual = R.dual;
+    E.face_prod = face_prod.get();
+    E.deferred = deferred.get();
+    launch_timed("swap_cavity", (double) n1 * 8 + (double) n2 * 12 + (double) n3 * 16 + (double) ns * 12,
+                 swap_products_k<true>, dim3(nblocks(ns)), dim3(BLOCK), ns, (u32 const*) nullptr, R.o1, R.o2, R.o3,
+                 (u32 const*) nullptr, R.ua, R.ud, R.ev, R.vt, R.info, R.ev + 2 * (size_t) nE,
+                 R.fv + 3 * (size_t) nF, R.vt + 4 * (size_t) nT, E, R);
+    element_qualities_into(3, n3, R.vt + 4 * (size_t) nT, coords(m), 0, metric_of(m), tq.get() + nT);
+    hipLaunchKernelGGL(run_touch_k, dim3(nblocks(nuse)), dim3(BLOCK), 0, stream(), R, nuse, slot, changed);
+    hipLaunchKernelGGL(run_lists_k, dim3(nblocks(nuse)), dim3(BLOCK), 0, stream(), R, changed);
+    hipLaunchKernelGGL(run_place_k, dim3(nblocks(nuse)), dim3(BLOCK), 0, stream(), R, nuse, slot);
+    hipLaunchKernelGGL(run_sort_k, dim3(nblocks(nuse)), dim3(BLOCK), 0, stream(), R, changed);
+    hipLaunchKernelGGL(run_settle_k, dim3(nblocks(4 * (size_t) n3)), dim3(BLOCK), 0, stream(), R, n3, E);
+    check_launch("run_settle");
+    nE += n1;
+    nF += n2;
+    nT += n3;
+    // a ring of rs tets and faces goes, 2 (rs - 2) tets come
+    u32 const ring = n3 / 2 + 2 * ns;
+    aE = aE + n1 - ns;
+    aF = aF + n2 - ring;
+    aT = aT + n3 - ring;
+  }
+};
+}  // namespace
+
 // ---------------------------------------------------------------- adapt
 // mesh_adapt (adapt.cpp:19-94)
 namespace {
@@ -3241,6 +4317,7 @@ struct Ctx {
   };
   std::vector<Timed> timed;
   std::vector<hipEvent_t> pool;
+  bool timing = false;  // the caller wants the statistics
   hipEvent_t event() {
     if (!pool.empty()) {
       hipEvent_t e = pool.back();
@@ -3250,6 +4327,25 @@ struct Ctx {
     hipEvent_t e;
     OHX_CHECK(hipEventCreate(&e));
     return e;
+  }
+  Timed start(double tin) {
+    Timed t{nullptr, nullptr, tin};
+    if (timing) {
+      t.a = event();
+      t.b = event();
+      OHX_CHECK(hipEventRecord(t.a, stream()));
+    }
+    return t;
+  }
+  void stop(Timed const& t, bool changed) {
+    if (!timing) return;
+    OHX_CHECK(hipEventRecord(t.b, stream()));
+    if (changed) {
+      timed.push_back(t);
+    } else {
+      pool.push_back(t.a);
+      pool.push_back(t.b);
+    }
   }
   void finish() {
     for (Timed& t : timed) {
@@ -3289,9 +4385,8 @@ u32 run_pass(Mesh& m, Ctx& c, Kind k, double a, double b, u32 n, double const* e
   double tin = count(m, m.dim);
   static bool const trace = std::getenv("OHX_TRACE_DERIVE") && std::getenv("OHX_TRACE_DERIVE")[0] == '1';
   if (trace) std::fprintf(stderr, "pass %s n=%.0f\n", k == REFINE ? "refine" : k == COARSEN ? "coarsen" : k == SWAP ? "swap" : "csliv", tin);
-  hipEvent_t e0 = c.event(), e1 = c.event();
-  OHX_CHECK(hipEventRecord(e0, stream()));
   u32 ok = 0;
+  Ctx::Timed const t = c.start(tin);
   if (k != SWAP) c.swap_cache.clear();
   if (k != COARSEN) c.size_codes.clear();
   switch (k) {
@@ -3300,20 +4395,74 @@ u32 run_pass(Mesh& m, Ctx& c, Kind k, double a, double b, u32 n, double const* e
     case SWAP: ok = swap_slivers(m, a, n, eq, gate, &c.swap_cache); break;
     case COARSEN_SLIVERS: ok = coarsen_slivers(m, a, n, eq); break;
   }
-  OHX_CHECK(hipEventRecord(e1, stream()));
-  if (ok)
-    c.timed.push_back(Ctx::Timed{e0, e1, tin});
-  else {
-    c.pool.push_back(e0);
-    c.pool.push_back(e1);
-  }
+  c.stop(t, ok != 0);
   return ok;
+}
+
+// the meshes the in-place swap passes serve: no element field to transfer, no
+// batch, nothing to print per pass, classified in every dimension
+bool swap_run_fits(Mesh& m) {
+  if (m.dim != 3 || !m.full || g_batch || g_verbose) return false;
+  bool const has_id = find_tag(m, 0, "class_id") != nullptr;
+  for (u32 d = 0; d <= 3; ++d)
+    for (char const* name : {"class_dim", "class_id"}) {
+      Tag* t = find_tag(m, d, name);
+      bool const wanted = name[6] == 'd' || has_id;
+      if (wanted && !(t && t->type == TagType::U32 && t->ncomps == 1)) return false;
+    }
+  for (auto& t : m.tags[3])
+    if (t->transfer == 1 || t->transfer == 2) return false;  // OSH_TRANSFER_POINTWISE, _CONSERVE
+  return true;
+}
+
+// swap passes until one changes nothing; eq: the element qualities of m,
+// before and after.  *good_now: the last one found every quality good.
+// Returns whether the operation limit was reached.
+bool swap_passes(Mesh& m, Ctx& c, double good_qual, u32 nlayers, Buf<double>& eq, bool* good_now) {
+  SwapRun run(m);
+  run.begin(eq.get(), nullptr, nullptr);
+  bool changed = false, limited = false;
+  *good_now = false;
+  for (;;) {
+    Ctx::Timed const t = c.start(run.aT);
+    bool ok;
+    try {
+      ok = run.step(good_qual, nlayers);
+    } catch (Error const&) {
+      // the round limit leaves the mesh of the passes before, as the pass
+      // through a whole mesh does
+      if (run.limit_hit && changed) run.finish(eq, nullptr, nullptr);
+      throw;
+    }
+    c.stop(t, ok);
+    if (!ok) {
+      *good_now = run.min_q >= good_qual;
+      break;
+    }
+    changed = true;
+    if (!incr_op(m, c)) {
+      limited = true;
+      break;
+    }
+    // more gaps than tets: close them, so that what each pass reads of the
+    // whole mesh stays below twice the mesh
+    if (run.nT - run.aT > run.aT) {
+      Buf<u32> known;
+      Buf<double> values;
+      run.finish(eq, &known, &values);
+      run.begin(eq.get(), known.get(), values.get());
+      changed = false;
+    }
+  }
+  if (changed) run.finish(eq, nullptr, nullptr);
+  return limited;
 }
 }  // namespace
 
 int adapt(Mesh& m, double size_floor, double good_qual, u32 nlayers, u32 max_ops, AdaptStats* st) {
   Ctx c;
   c.max_ops = max_ops;
+  c.timing = st != nullptr;
   double t0 = now_s();
   int result = 0;
   adapt_summary(m);
@@ -3330,7 +4479,17 @@ int adapt(Mesh& m, double size_floor, double good_qual, u32 nlayers, u32 max_ops
     // read them (a pass that changes nothing leaves them valid for the next)
     u32 const nel = count(m, m.dim);
     Buf<double> eq = c.swap_cache.eq ? std::move(c.swap_cache.eq) : mesh_qualities(m);
-    if (m.dim == 3) {
+    if (swap_run_fits(m)) {
+      // the minimum first, in a wait of its own: a mesh of good quality then
+      // needs none of the maps a swap pass derives
+      double const prev = nel > 1 ? min_f64(eq.get(), nel, 1) : 1.7976931348623157e308;
+      if (prev >= good_qual) break;
+      c.size_codes.clear();
+      c.swap_cache.clear();
+      bool good_now = false;
+      aborted = swap_passes(m, c, good_qual, nlayers, eq, &good_now);
+      if (aborted || good_now) break;
+    } else if (m.dim == 3) {
       // the minimum (over elements 1..n-1, as the serial doubles_min)
       // reaches the host with the swap pass's first wait instead of a wait
       // of its own: the pass's sliver marks are gated on it on the device,

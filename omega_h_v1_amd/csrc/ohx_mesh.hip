@@ -151,15 +151,20 @@ __global__ __launch_bounds__(BLOCK) void elem_min_quality_f64(u32 n, u32 begin,
   }
 }
 
-Buf<double> element_qualities(u32 dim, u32 n, u32 const* ev, double const* x, u32 nverts, double const* mt) {
-  Buf<double> q(n);
-  if (!n) return q;
+void element_qualities_into(u32 dim, u32 n, u32 const* ev, double const* x, u32 nverts, double const* mt,
+                            double* out) {
+  if (!n) return;
   // compulsory bytes: connectivity, each vertex's coordinates once, output
   double prof_bytes = (double) n * (dim + 1) * 4 + (double) nverts * 24 + (double) n * 8;
   if (dim == 3)
-    launch_timed("elem_quality_f64", prof_bytes, elem_quality_f64<3>, dim3(nblocks(n)), dim3(BLOCK), n, ev, x, mt, q.get());
+    launch_timed("elem_quality_f64", prof_bytes, elem_quality_f64<3>, dim3(nblocks(n)), dim3(BLOCK), n, ev, x, mt, out);
   else
-    launch_timed("elem_quality_f64", prof_bytes, elem_quality_f64<2>, dim3(nblocks(n)), dim3(BLOCK), n, ev, x, mt, q.get());
+    launch_timed("elem_quality_f64", prof_bytes, elem_quality_f64<2>, dim3(nblocks(n)), dim3(BLOCK), n, ev, x, mt, out);
+}
+
+Buf<double> element_qualities(u32 dim, u32 n, u32 const* ev, double const* x, u32 nverts, double const* mt) {
+  Buf<double> q(n);
+  element_qualities_into(dim, n, ev, x, nverts, mt, q.get());
   return q;
 }
 

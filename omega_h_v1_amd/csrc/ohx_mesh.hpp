@@ -81,6 +81,8 @@ u32 const* u32_tag(Mesh& m, u32 d, char const* name);
 // nverts only feeds the traffic accounting of the kernel timers
 Buf<double> element_qualities(u32 dim, u32 n, u32 const* verts_of_elems, double const* x, u32 nverts = 0,
                               double const* metric = nullptr);
+void element_qualities_into(u32 dim, u32 n, u32 const* verts_of_elems, double const* x, u32 nverts,
+                            double const* metric, double* out);
 Buf<double> mesh_qualities(Mesh& m);
 double min_element_quality(u32 dim, u32 n, u32 const* verts_of_elems, double const* x, u32 nverts = 0,
                            double const* metric = nullptr);
