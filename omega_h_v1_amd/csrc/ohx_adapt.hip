@@ -2523,49 +2523,6 @@ struct SwapEdgesOf {
 
 constexpr u32 DUAL_PENDING = 0xfffffffeu;
 
-// Words of a swap run (SwapRunView::words)
-enum { RW_ACC = 0, RW_EVAL = 1, RW_AFF = 2, RW_POOL = 3, RW_FIRST = 4, RW_FLAGS = 8, RW_WORDS = 16 };
-// an edge's word in a run: its choice is known, it is accepted, then ring
-// size and triangulation code as in the swap cache; a dead or boundary edge
-// is known and rejected for good
-constexpr u32 RI_KNOWN = 1u << 31, RI_ACCEPT = 1u << 30;
-
-// The mesh of a run of swap passes (see "swap passes in place"), as slots.
-struct SwapRunView {
-  u32 nE, nF, nT, nF0;  // slots in use before the pass's products; faces at the start
-  u32 pass;             // 1, 2, ...
-  u32* ev;              // edges: vertices, class, the pass that removed it (0: alive), choice and its
-  u32* ecd;             // value, first place and length of its list in (ua, ud), product uses
-  u32* eci;
-  u32* death;
-  u32* info;
-  double* q;
-  u32* lb;
-  u32* ln;
-  u32* cnt;
-  unsigned char* sa;  // independent-set state before / after a round
-  unsigned char* sb;
-  u32* ua;  // tets around the edges and the edges' places in them, ascending per edge
-  u32* ud;
-  u32* vt;  // tets: vertices, edges, dual, class, removed
-  u32* te;
-  u32* dual;
-  u32* tcd;
-  u32* tci;
-  unsigned char* dead;
-  u32* fv;  // faces: vertices, class, the pass that made a product face (from slot nF0 on)
-  u32* fcd;
-  u32* fci;
-  u32* fbirth;
-  u32* acc;  // accepted candidates and candidates to evaluate (any order)
-  u32* eval;
-  u32* sw;   // swapped edges in order, their first products of each dimension
-  u32* o1;
-  u32* o2;
-  u32* o3;
-  u32* words;
-};
-
 // local face of a tet (vertices tv) with the vertices a, b, c
 __device__ inline u32 tet_face_of(u32 const* tv, u32 a, u32 b, u32 c) {
   for (u32 f = 0; f < 4; ++f) {
@@ -2601,28 +2558,24 @@ __device__ inline u32 tet_edge_between(u32 a, u32 b) {
 // edges of the old tet at that ring slot (the one holding ring vertices k
 // and k + 1), and any other is one of the new interior edges.  The cavity's
 // ring edges and spokes are staged in LDS per thread (indexed by slot).
-// RUN: thread k takes the run's k-th swapped edge, nothing is renumbered
-// (soff1, soff3 are not read), a survivor's dual entry is rewritten by the
-// product now across that face, and the products' other arrays are set up.
-template <bool RUN>
 __global__ __launch_bounds__(BLOCK) void swap_products_k(
-    u32 ne, u32 const* indset, u32 const* goff1, u32 const* goff2, u32 const* goff3, u32 const* uo, u32 const* ua,
-    u32 const* ud, u32 const* ev, u32 const* vt, u32 const* codes, u32* out1, u32* out2, u32* out3, SwapEdgesOf E,
-    SwapRunView R) {
+    u32 ne, u32 const* __restrict__ indset, u32 const* __restrict__ goff1, u32 const* __restrict__ goff2,
+    u32 const* __restrict__ goff3, u32 const* __restrict__ uo, u32 const* __restrict__ ua,
+    u32 const* __restrict__ ud, u32 const* __restrict__ ev, u32 const* __restrict__ vt,
+    u32 const* __restrict__ codes, u32* __restrict__ out1, u32* __restrict__ out2, u32* __restrict__ out3,
+    SwapEdgesOf E) {
   __shared__ u32 s_ring[MAX_EDGE_SWAP][BLOCK];
   __shared__ u32 s_spoke[2][MAX_EDGE_SWAP][BLOCK];
   __shared__ u32 s_tet[MAX_EDGE_SWAP][BLOCK];
   u32 const tid = threadIdx.x;
   u32 i = xcd_block() * BLOCK + tid;
-  if (i >= ne || (!RUN && !indset[i])) return;  // no barrier follows
+  if (i >= ne || !indset[i]) return;  // no barrier follows
   u32 const g1 = goff1[i], g2 = goff2[i], g3 = goff3[i];
-  if (RUN) i = R.sw[i];
-  u32 const f = RUN ? R.lb[i] : uo[i], e = RUN ? f + R.ln[i] : uo[i + 1];
-  auto edge_now = [&](u32 old) { return RUN ? old : E.soff1[old]; };
+  u32 const f = uo[i], e = uo[i + 1];
   u32 edge_v[2], ring_v[MAX_EDGE_SWAP];
   u32 rs = edge_ring(i, f, e, ua, ud, ev, vt, edge_v, ring_v);
   if (rs < 3 || rs > MAX_EDGE_SWAP) return;  // cannot happen for an indset edge
-  u32 const code = codes[i] & 0xffffu;
+  u32 const code = codes[i];
   u32 const tpm = k_sw_sizes[rs];
   unsigned char const* mesh = k_sw_meshes + k_sw_mesh_off[rs] + code * tpm;
   unsigned char const(*tris)[3] = k_sw_tris + k_sw_tri_off[rs];
@@ -2633,35 +2586,6 @@ __global__ __launch_bounds__(BLOCK) void swap_products_k(
     for (u32 k = 0; k < nint; ++k) {
       o[2 * k] = ring_v[ie[2 * k]];
       o[2 * k + 1] = ring_v[ie[2 * k + 1]];
-    }
-  }
-  if (RUN) {
-    // the products' class (the swapped edge's) and their other arrays
-    u32 const cd = R.ecd[i], ci = R.eci ? R.eci[i] : 0u;
-    for (u32 k = 0; k < nint; ++k) {
-      u32 const n = R.nE + g1 + k;
-      R.ecd[n] = cd;
-      if (R.eci) R.eci[n] = ci;
-      R.death[n] = 0;
-      R.info[n] = cd == 3 ? 0u : RI_KNOWN;
-      R.lb[n] = 0;
-      R.ln[n] = 0;
-      R.cnt[n] = 0;
-      R.sa[n] = 0;
-      R.sb[n] = 0;
-    }
-    u32 const nf = tpm + 2 * nint;
-    for (u32 k = 0; k < nf; ++k) {
-      u32 const n = R.nF + g2 + k;
-      R.fcd[n] = cd;
-      if (R.fci) R.fci[n] = ci;
-      R.fbirth[n - R.nF0] = R.pass;
-    }
-    for (u32 k = 0; k < 2 * tpm; ++k) {
-      u32 const n = R.nT + g3 + k;
-      R.tcd[n] = cd;
-      if (R.tci) R.tci[n] = ci;
-      R.dead[n] = 0;
     }
   }
   if (out2) {
@@ -2702,9 +2626,9 @@ __global__ __launch_bounds__(BLOCK) void swap_products_k(
       if (tv[c] == edge_v[1]) l1 = c;
     }
     s_tet[k][tid] = tet;
-    s_ring[k][tid] = edge_now(te[tet_edge_between(la, lb)]);
-    s_spoke[0][k][tid] = edge_now(te[tet_edge_between(la, l0)]);
-    s_spoke[1][k][tid] = edge_now(te[tet_edge_between(la, l1)]);
+    s_ring[k][tid] = E.soff1[te[tet_edge_between(la, lb)]];
+    s_spoke[0][k][tid] = E.soff1[te[tet_edge_between(la, l0)]];
+    s_spoke[1][k][tid] = E.soff1[te[tet_edge_between(la, l1)]];
   }
   if (!out3) return;
   u32* o3 = out3 + (size_t) g3 * 4;
@@ -2781,11 +2705,7 @@ __global__ __launch_bounds__(BLOCK) void swap_products_k(
               u32 const o = E.old_dual[4 * (size_t) tk + lf];
               if (o == INVALID) {
                 nb = INVALID;
-              } else if (RUN && !R.dead[o]) {
-                nb = o;
-                for (u32 q = 0; q < 4; ++q)
-                  if (E.dual[4 * (size_t) o + q] == tk) E.dual[4 * (size_t) o + q] = self;
-              } else if (!RUN && E.soff3[o] != E.soff3[o + 1]) {
+              } else if (E.soff3[o] != E.soff3[o + 1]) {
                 nb = E.soff3[o];
               } else {
                 nb = DUAL_PENDING;
@@ -2815,21 +2735,18 @@ __global__ __launch_bounds__(BLOCK) void swap_products_k(
   }
 }
 
-// the product across a removed tet n's face shared with the tet from
-__device__ inline u32 swap_across(SwapEdgesOf const& E, u32 n, u32 from) {
-  for (u32 g = 0; g < 4; ++g)
-    if (E.old_dual[4 * (size_t) n + g] == from) return E.face_prod[4 * (size_t) n + g];
-  *E.err = ERR_REFLECT_NOT_FOUND;
-  return INVALID;
-}
-
 // The new dual's remaining entries: threads [0, nt_old) give a surviving
 // tet its neighbours (a surviving one renumbered, a removed one replaced by
 // the product now across that face); the ngen3 * 4 after them resolve a
 // product face whose outside tet was removed by another cavity.
 __global__ __launch_bounds__(BLOCK) void swap_dual_k(u32 nt_old, u32 ngen3, SwapEdgesOf E) {
   u32 const s = xcd_block() * BLOCK + threadIdx.x;
-  auto across = [&](u32 n, u32 from) { return swap_across(E, n, from); };
+  auto across = [&](u32 n, u32 from) -> u32 {  // the product across n's face shared with from
+    for (u32 g = 0; g < 4; ++g)
+      if (E.old_dual[4 * (size_t) n + g] == from) return E.face_prod[4 * (size_t) n + g];
+    *E.err = ERR_REFLECT_NOT_FOUND;
+    return INVALID;
+  };
   if (s < nt_old) {
     u32 const o = E.soff3[s];
     if (o == E.soff3[s + 1]) return;
@@ -3218,9 +3135,9 @@ static u32 swap_common(Mesh& m, Buf<u32>& cand, double const* eq_given = nullptr
       E.deferred = deferred.get();
     }
   }
-  launch_timed("swap_cavity", prof_bytes, swap_products_k<false>, dim3(nblocks(ne)), dim3(BLOCK), ne, is,
+  launch_timed("swap_cavity", prof_bytes, swap_products_k, dim3(nblocks(ne)), dim3(BLOCK), ne, is,
                goffs[1].get(), goffs[2].get(), goffs[3].get(), u.offsets.get(), u.adj.get(), u.dirs.get(), ev, vt,
-               codes.get(), pouts[1], pouts[2], pouts[3], E, SwapRunView{});
+               codes.get(), pouts[1], pouts[2], pouts[3], E);
   if (E.dual) {
     hipLaunchKernelGGL(swap_dual_k, dim3(nblocks((size_t) nt_old + (size_t) ngen3 * 4)), dim3(BLOCK), 0, stream(),
                        nt_old, ngen3, E);
@@ -3363,6 +3280,49 @@ u32 swap_slivers(Mesh& m, double good_qual, u32 nlayers, double const* eq, doubl
 // hash table with the last pass that removed it, and a face is gone if one
 // of its pairs was removed in a pass after the one that made the face.
 
+// Words of a swap run (SwapRunView::words)
+enum { RW_ACC = 0, RW_EVAL = 1, RW_AFF = 2, RW_POOL = 3, RW_FIRST = 4, RW_NEED = 5, RW_FLAGS = 8, RW_WORDS = 16 };
+// an edge's word in a run: its choice is known, it is accepted, then ring
+// size and triangulation code as in the swap cache; a dead or boundary edge
+// is known and rejected for good
+constexpr u32 RI_KNOWN = 1u << 31, RI_ACCEPT = 1u << 30;
+
+// The mesh of a run of swap passes (see "swap passes in place"), as slots.
+struct SwapRunView {
+  u32 nE, nF, nT, nF0;  // slots in use before the pass's products; faces at the start
+  u32 pass;             // 1, 2, ...
+  u32* ev;              // edges: vertices, class, the pass that removed it (0: alive), choice and its
+  u32* ecd;             // value, first place and length of its list in (ua, ud), product uses
+  u32* eci;
+  u32* death;
+  u32* info;
+  double* q;
+  u32* lb;
+  u32* ln;
+  u32* cnt;
+  unsigned char* sa;  // independent-set state before / after a round
+  unsigned char* sb;
+  u32* ua;  // tets around the edges and the edges' places in them, ascending per edge
+  u32* ud;
+  u32* vt;  // tets: vertices, edges, dual, class, removed
+  u32* te;
+  u32* dual;
+  u32* tcd;
+  u32* tci;
+  unsigned char* dead;
+  u32* fv;  // faces: vertices, class, the pass that made a product face (from slot nF0 on)
+  u32* fcd;
+  u32* fci;
+  u32* fbirth;
+  u32* acc;  // accepted candidates and candidates to evaluate (any order)
+  u32* eval;
+  u32* sw;   // swapped edges in order, their first products of each dimension
+  u32* o1;
+  u32* o2;
+  u32* o3;
+  u32* words;
+};
+
 // the index for each lane with pred among those of the launch, one atomic
 // per wave; every lane of the wave must call it
 __device__ inline u32 wave_append(u32* counter, bool pred) {
@@ -3434,9 +3394,18 @@ __global__ __launch_bounds__(BLOCK) void run_candidates_k(SwapRunView R, unsigne
   if (e < R.nE) {
     u32 const w = R.info[e];
     if (!(w & RI_KNOWN) || (w & RI_ACCEPT)) {
+      // four tets at a time, so that their loads are in flight together
       bool in = false;
       u32 const f = R.lb[e], n = R.ln[e];
-      for (u32 k = 0; k < n && !in; ++k) in = marks[R.ua[f + k]] != 0;
+      for (u32 k = 0; k < n && !in; k += 4) {
+        u32 t[4];
+#pragma unroll
+        for (u32 j = 0; j < 4; ++j) t[j] = R.ua[f + (k + j < n ? k + j : k)];
+        u32 any = 0;
+#pragma unroll
+        for (u32 j = 0; j < 4; ++j) any |= marks[t[j]];
+        in = any != 0;
+      }
       acc = in && (w & RI_KNOWN);
       ask = in && !(w & RI_KNOWN);
     }
@@ -3493,19 +3462,20 @@ __global__ __launch_bounds__(BLOCK) void run_round_k(SwapRunView R, unsigned cha
       bool wait = false, out = false;
       u32 const f = R.lb[i], l = R.ln[i];
       for (u32 j = f; j < f + l && !out; ++j) {
-        u32 const t = R.ua[j], d = R.ud[j];
+        // a tet's edges and their states in two round trips
+        u32 const t = R.ua[j];
+        u32 o[6], so[6];
+#pragma unroll
+        for (u32 c = 0; c < 6; ++c) o[c] = R.te[6 * (size_t) t + c];
+#pragma unroll
+        for (u32 c = 0; c < 6; ++c)  // (INVALID: a product's edge that was not found, reported)
+          so[c] = o[c] == i || o[c] >= R.nE ? (u32) NOT_IN_SET : old[o[c]];
+#pragma unroll
         for (u32 c = 0; c < 6; ++c) {
-          if (c == d) continue;
-          u32 const o = R.te[6 * (size_t) t + c];
-          if (o >= R.nE) continue;  // a product's edge that was not found (reported)
-          u32 const so = old[o];
-          if (so == IN_SET) {
-            out = true;
-            break;
-          }
-          if (so == NOT_IN_SET || wait) continue;
-          double const og = R.q[o];
-          if ((myg == og && o < i) || myg < og) wait = true;
+          if (so[c] == IN_SET) out = true;
+          if (so[c] != UNKNOWN || wait) continue;
+          double const og = R.q[o[c]];
+          if ((myg == og && o[c] < i) || myg < og) wait = true;
         }
       }
       s = out ? (u32) NOT_IN_SET : (wait ? (u32) UNKNOWN : (u32) IN_SET);
@@ -3516,35 +3486,26 @@ __global__ __launch_bounds__(BLOCK) void run_round_k(SwapRunView R, unsigned cha
   wave_flag(flag, undecided);
 }
 
-// What a swapped edge makes and needs: itself, product edges, faces and
-// tets, and at most how many list places its surroundings' survivors take
+// What a swapped edge makes: itself, product edges, faces and tets
 struct RunCount {
-  u32 v[5];
+  u32 v[4];
 };
 constexpr u32 RUN_PER = 8;  // edges per thread of the two counting kernels
 
-__device__ inline void run_count_edge(SwapRunView const& R, u32 e, RunCount& c, bool need) {
+__device__ inline void run_count_edge(SwapRunView const& R, u32 e, RunCount& c) {
   u32 const w = R.info[e], rs = (w >> 16) & 0xffu;
   u32 const nint = k_sw_nint[rs], tpm = k_sw_sizes[rs];
   c.v[0] += 1;
   c.v[1] += nint;
   c.v[2] += count_swap_ents(rs, 2, nint, tpm);
   c.v[3] += count_swap_ents(rs, 3, nint, tpm);
-  if (!need) return;
-  u32 const f = R.lb[e], n = R.ln[e];
-  for (u32 j = f; j < f + n; ++j)
-    for (u32 k = 0; k < 6; ++k) {
-      u32 const o = R.te[6 * (size_t) R.ua[j] + k];
-      c.v[4] += o < R.nE ? R.ln[o] : 0u;
-    }
 }
 
-// exclusive prefix of c over the block's threads (first N words), totals in *tot
-template <u32 N>
-__device__ inline void run_block_scan(RunCount& c, RunCount* tot, u32 (*lds)[5]) {
+// exclusive prefix of c over the block's threads, totals in *tot
+__device__ inline void run_block_scan(RunCount& c, RunCount* tot, u32 (*lds)[4]) {
   u32 const lane = threadIdx.x & 63u, wave = threadIdx.x >> 6, nw = blockDim.x >> 6;
 #pragma unroll
-  for (u32 k = 0; k < N; ++k) {
+  for (u32 k = 0; k < 4; ++k) {
     u32 const mine = c.v[k];
     u32 x = mine;
 #pragma unroll
@@ -3557,7 +3518,7 @@ __device__ inline void run_block_scan(RunCount& c, RunCount* tot, u32 (*lds)[5])
   }
   __syncthreads();
 #pragma unroll
-  for (u32 k = 0; k < N; ++k) {
+  for (u32 k = 0; k < 4; ++k) {
     u32 off = 0, all = 0;
     for (u32 w = 0; w < nw; ++w) {
       if (w < wave) off += lds[w][k];
@@ -3572,7 +3533,7 @@ __device__ inline void run_block_scan(RunCount& c, RunCount* tot, u32 (*lds)[5])
 // per block of BLOCK * RUN_PER edges: the totals of its swapped edges
 __global__ __launch_bounds__(BLOCK) void run_count_k(SwapRunView R, unsigned char const* __restrict__ state,
                                                      RunCount* __restrict__ part) {
-  __shared__ u32 lds[BLOCK / 64][5];
+  __shared__ u32 lds[BLOCK / 64][4];
   u32 const e0 = (blockIdx.x * BLOCK + threadIdx.x) * RUN_PER;
   RunCount c{}, tot;
   if (e0 < R.nE) {
@@ -3580,9 +3541,9 @@ __global__ __launch_bounds__(BLOCK) void run_count_k(SwapRunView R, unsigned cha
     unsigned long long const w = *reinterpret_cast<unsigned long long const*>(state + e0);
     if (w)
       for (u32 k = 0; k < RUN_PER; ++k)
-        if (((w >> (8 * k)) & 0xffu) == IN_SET) run_count_edge(R, e0 + k, c, true);
+        if (((w >> (8 * k)) & 0xffu) == IN_SET) run_count_edge(R, e0 + k, c);
   }
-  run_block_scan<5>(c, &tot, lds);
+  run_block_scan(c, &tot, lds);
   if (threadIdx.x == 0) part[blockIdx.x] = tot;
 }
 
@@ -3592,13 +3553,13 @@ __global__ __launch_bounds__(1024) void run_offsets_k(u32 nb, RunCount* __restri
                                                       double const* __restrict__ qpart, SwapRunView R,
                                                       u32 const* __restrict__ flag, u32* __restrict__ host,
                                                       double* __restrict__ host_min) {
-  __shared__ u32 lds[16][5];
+  __shared__ u32 lds[16][4];
   __shared__ double mins[16];
   u32 const per = (nb + 1023) / 1024, b = threadIdx.x * per, e = b + per < nb ? b + per : nb;
   RunCount c{}, tot;
   for (u32 i = b; i < e; ++i)
-    for (u32 k = 0; k < 5; ++k) c.v[k] += part[i].v[k];
-  run_block_scan<5>(c, &tot, lds);
+    for (u32 k = 0; k < 4; ++k) c.v[k] += part[i].v[k];
+  run_block_scan(c, &tot, lds);
   for (u32 i = b; i < e; ++i)
     for (u32 k = 0; k < 4; ++k) {
       u32 const n = part[i].v[k];
@@ -3618,9 +3579,9 @@ __global__ __launch_bounds__(1024) void run_offsets_k(u32 nb, RunCount* __restri
   if (threadIdx.x != 0) return;
   for (u32 w = 1; w < 16; ++w)
     if (mins[w] < v) v = mins[w];
-  for (u32 k = 0; k < 5; ++k) host[k] = tot.v[k];
-  host[5] = R.words[RW_POOL];
-  host[6] = *flag;
+  for (u32 k = 0; k < 4; ++k) host[k] = tot.v[k];
+  host[4] = R.words[RW_POOL];
+  host[5] = *flag;
   *host_min = v;
 }
 
@@ -3628,15 +3589,15 @@ __global__ __launch_bounds__(1024) void run_offsets_k(u32 nb, RunCount* __restri
 // with the tets around it
 __global__ __launch_bounds__(BLOCK) void run_list_k(SwapRunView R, unsigned char const* __restrict__ state,
                                                     RunCount const* __restrict__ part) {
-  __shared__ u32 lds[BLOCK / 64][5];
+  __shared__ u32 lds[BLOCK / 64][4];
   u32 const e0 = (blockIdx.x * BLOCK + threadIdx.x) * RUN_PER;
   RunCount c{}, tot;
   unsigned long long w = 0;
   if (e0 < R.nE) w = *reinterpret_cast<unsigned long long const*>(state + e0);
   if (w)
     for (u32 k = 0; k < RUN_PER; ++k)
-      if (((w >> (8 * k)) & 0xffu) == IN_SET) run_count_edge(R, e0 + k, c, false);
-  run_block_scan<4>(c, &tot, lds);
+      if (((w >> (8 * k)) & 0xffu) == IN_SET) run_count_edge(R, e0 + k, c);
+  run_block_scan(c, &tot, lds);
   if (!w) return;
   RunCount const base = part[blockIdx.x];
   for (u32 k = 0; k < 4; ++k) c.v[k] += base.v[k];
@@ -3647,12 +3608,204 @@ __global__ __launch_bounds__(BLOCK) void run_list_k(SwapRunView R, unsigned char
     R.o1[s] = c.v[1];
     R.o2[s] = c.v[2];
     R.o3[s] = c.v[3];
-    run_count_edge(R, e, c, false);
+    run_count_edge(R, e, c);
     R.death[e] = R.pass;
     R.info[e] &= ~RI_ACCEPT;  // the ring size and triangulation stay for the products
     u32 const f = R.lb[e], n = R.ln[e];
     for (u32 j = f; j < f + n; ++j) R.dead[R.ua[j]] = 1;
   }
+}
+
+// The products of the pass's cavities (swap_products_k's, unnumbered), RUN_G
+// lanes per swapped edge: lane j reads the edge's j-th tet, the lanes chain
+// the ring together (edge_ring.cpp:12-74 follows each tet's opposite edge a
+// -> b from the first tet; here the lane whose a is the current b is found by
+// ballot), and each writes an edge, faces and a tet with its edges and dual.
+// A thread per cavity took 99 us on the 21^3 x 6 anisotropic box whether a
+// pass had 60,000 cavities or one: a serial chain of its loads and of the
+// products' bookkeeping, which a cavity's lanes now share.
+constexpr u32 RUN_G = 16;
+struct RunCavity {
+  // by ring slot k: the vertex, the tet around (k, k + 1), its ring edge, the
+  // edges from the vertex to the swapped edge's ends, and where the ends are
+  // in the tet
+  u32 ring[8], tet[8], redge[8], spoke[2][8], loc[8];
+};
+// local vertices of a tet's edge d, the edge opposite, the face opposite a
+// local vertex (k_r_e_v, k_o_r_e, k_r_f_v), a digit each
+__device__ inline u32 tet_ev0(u32 d) { return (0x210210u >> (4 * d)) & 3u; }
+__device__ inline u32 tet_ev1(u32 d) { return (0x333021u >> (4 * d)) & 3u; }
+__device__ inline u32 tet_oe(u32 d) { return (0x021435u >> (4 * d)) & 7u; }
+__device__ inline u32 tet_face_without(u32 v) { return (0x0132u >> (4 * v)) & 3u; }
+__device__ inline u32 tet_edge_of(u32 a, u32 b) {
+  return a == 3 ? 3 + b : b == 3 ? 3 + a : a + b == 1 ? 0u : a + b == 3 ? 1u : 2u;
+}
+
+__global__ __launch_bounds__(BLOCK) void run_products_k(SwapRunView R, u32 ns, u32* __restrict__ face_prod,
+                                                        u32* __restrict__ deferred, u32* __restrict__ err) {
+  __shared__ RunCavity cavities[BLOCK / RUN_G];
+  u32 const g = threadIdx.x / RUN_G, lane = threadIdx.x % RUN_G;
+  RunCavity& C = cavities[g];
+  u32 const s = blockIdx.x * (BLOCK / RUN_G) + g;
+  u32 e = 0, f = 0, rs = 0, ends[2] = {0, 0}, code = 0, g1 = 0, g2 = 0, g3 = 0, cd = 0, ci = 0;
+  if (s < ns) {
+    e = R.sw[s];
+    f = R.lb[e];
+    rs = R.ln[e];
+    ends[0] = R.ev[2 * (size_t) e];
+    ends[1] = R.ev[2 * (size_t) e + 1];
+    code = R.info[e] & 0xffffu;
+    g1 = R.o1[s];
+    g2 = R.o2[s];
+    g3 = R.o3[s];
+    cd = R.ecd[e];
+    if (R.eci) ci = R.eci[e];
+    if (rs < 3 || rs > MAX_EDGE_SWAP) rs = 0;  // cannot happen for an accepted edge
+  }
+  // the edge's tets
+  u32 a = INVALID, b = INVALID, t = 0, redge = 0, sp0 = 0, sp1 = 0, loc = 0;
+  if (lane < rs) {
+    t = R.ua[f + lane];
+    u32 const d = R.ud[f + lane];
+    u32 v[4], le[6];
+#pragma unroll
+    for (u32 k = 0; k < 4; ++k) v[k] = R.vt[4 * (size_t) t + k];
+#pragma unroll
+    for (u32 k = 0; k < 6; ++k) le[k] = R.te[6 * (size_t) t + k];
+    auto vert = [&](u32 l) { return l == 0 ? v[0] : l == 1 ? v[1] : l == 2 ? v[2] : v[3]; };
+    auto edge = [&](u32 l) { return l == 0 ? le[0] : l == 1 ? le[1] : l == 2 ? le[2] : l == 3 ? le[3] : l == 4 ? le[4] : le[5]; };
+    u32 const o = tet_oe(d);
+    bool const turned = vert(tet_ev0(d)) != ends[0];
+    u32 const l0 = turned ? tet_ev1(d) : tet_ev0(d), l1 = turned ? tet_ev0(d) : tet_ev1(d);
+    u32 const la = turned ? tet_ev1(o) : tet_ev0(o), lb = turned ? tet_ev0(o) : tet_ev1(o);
+    a = vert(la);
+    b = vert(lb);
+    redge = edge(o);
+    sp0 = edge(tet_edge_of(la, l0));
+    sp1 = edge(tet_edge_of(la, l1));
+    loc = l0 | (l1 << 2);
+  }
+  // the ring: each lane's slot
+  u32 const shift = (threadIdx.x & 63u) & ~(RUN_G - 1u);
+  u32 slot = lane == 0 ? 0u : INVALID, cur = 0;
+  for (u32 k = 1; k < MAX_EDGE_SWAP; ++k) {
+    u32 const want = (u32) __shfl((int) b, (int) cur, (int) RUN_G);
+    u32 const m = (u32) (__ballot(lane < rs && a == want) >> shift) & ((1u << RUN_G) - 1u);
+    cur = m ? (u32) (__ffs((int) m) - 1) : 0u;
+    if (m && k < rs && lane == cur) slot = k;
+  }
+  if (lane < rs) {
+    if (slot == INVALID) {
+      *err = ERR_EDGE_RING;  // cannot happen: the ring closed when it was evaluated
+      slot = lane;
+    }
+    C.ring[slot] = a;
+    C.tet[slot] = t;
+    C.redge[slot] = redge;
+    C.spoke[0][slot] = sp0;
+    C.spoke[1][slot] = sp1;
+    C.loc[slot] = loc;
+  }
+  __syncthreads();
+  if (!rs) return;  // no barrier follows
+  u32 const tpm = k_sw_sizes[rs], nint = k_sw_nint[rs];
+  unsigned char const* mesh = k_sw_meshes + k_sw_mesh_off[rs] + code * tpm;
+  unsigned char const(*tris)[3] = k_sw_tris + k_sw_tri_off[rs];
+  unsigned char const* ie = k_sw_int + k_sw_int_off[rs] + code * nint * 2;
+  if (lane < nint) {
+    u32 const n = R.nE + g1 + lane;
+    R.ev[2 * (size_t) n] = C.ring[ie[2 * lane]];
+    R.ev[2 * (size_t) n + 1] = C.ring[ie[2 * lane + 1]];
+    R.ecd[n] = cd;
+    if (R.eci) R.eci[n] = ci;
+    R.death[n] = 0;
+    R.info[n] = cd == 3 ? 0u : RI_KNOWN;
+    R.lb[n] = 0;
+    R.ln[n] = 0;
+    R.cnt[n] = 0;
+    R.sa[n] = 0;
+    R.sb[n] = 0;
+  }
+  u32 const nf = tpm + 2 * nint;  // at most 13: a lane each
+  if (lane < nf) {
+    u32 const n = R.nF + g2 + lane;
+    u32* o = R.fv + 3 * (size_t) n;
+    if (lane < 2 * nint) {
+      o[0] = C.ring[ie[2 * (lane / 2)]];
+      o[1] = C.ring[ie[2 * (lane / 2) + 1]];
+      o[2] = ends[lane & 1u];
+    } else {
+      for (u32 j = 0; j < 3; ++j) o[j] = C.ring[tris[mesh[lane - 2 * nint]][j]];
+    }
+    R.fcd[n] = cd;
+    if (R.fci) R.fci[n] = ci;
+    R.fbirth[n - R.nF0] = R.pass;
+  }
+  if (lane >= 2 * tpm) return;  // at most 10 tets
+  // the tet of triangle p and edge end 1, then with its first two corners
+  // exchanged and edge end 0
+  u32 const p = lane / 2, j = lane & 1u, x = 1 - j;
+  u32 const first = R.nT + g3, self = first + lane;
+  u32 lab[3] = {tris[mesh[p]][j], tris[mesh[p]][1 - j], tris[mesh[p]][2]};
+  for (u32 k = 0; k < 3; ++k) R.vt[4 * (size_t) self + k] = C.ring[lab[k]];
+  R.vt[4 * (size_t) self + 3] = ends[x];
+  R.tcd[self] = cd;
+  if (R.tci) R.tci[self] = ci;
+  R.dead[self] = 0;
+  // adjacent ring slots: the slot their ring edge and tet have, else INVALID
+  auto beside = [&](u32 u, u32 v) {
+    return u + 1 == v || u == v + rs - 1 ? u : v + 1 == u || v == u + rs - 1 ? v : INVALID;
+  };
+#pragma unroll
+  for (u32 k = 0; k < 3; ++k) {
+    // edges 0-1, 1-2, 2-0 and the faces on them (1, 2, 3); spokes 3, 4, 5
+    u32 const u = lab[k], v = lab[(k + 1) % 3], r = beside(u, v);
+    u32 id = INVALID, across = INVALID;
+    if (r != INVALID) {
+      id = C.redge[r];
+      u32 const tk = C.tet[r], lf = tet_face_without((C.loc[r] >> (2 * (1 - x))) & 3u);
+      size_t const key = 4 * (size_t) tk + lf;
+      face_prod[key] = self;
+      u32 const o = R.dual[key];
+      if (o != INVALID && !R.dead[o]) {
+        across = o;
+        for (u32 q = 0; q < 4; ++q)
+          if (R.dual[4 * (size_t) o + q] == tk) R.dual[4 * (size_t) o + q] = self;
+      } else if (o != INVALID) {
+        across = DUAL_PENDING;  // another cavity's: known once its products are written
+        deferred[4 * (size_t) (g3 + lane) + 1 + k] = (u32) key;
+      }
+    } else {
+      for (u32 q = 0; q < nint; ++q)
+        if ((ie[2 * q] == u && ie[2 * q + 1] == v) || (ie[2 * q] == v && ie[2 * q + 1] == u)) id = R.nE + g1 + q;
+      for (u32 t2 = 0; t2 < tpm; ++t2) {
+        if (t2 == p) continue;
+        unsigned char const* tr = tris[mesh[t2]];
+        if ((tr[0] == u || tr[1] == u || tr[2] == u) && (tr[0] == v || tr[1] == v || tr[2] == v))
+          across = first + 2 * t2 + j;
+      }
+      if (across == INVALID) *err = ERR_REFLECT_NOT_FOUND;
+    }
+    if (id == INVALID) *err = ERR_REFLECT_NOT_FOUND;
+    R.te[6 * (size_t) self + k] = id;
+    R.te[6 * (size_t) self + 3 + k] = C.spoke[x][u];
+    R.dual[4 * (size_t) self + 1 + k] = across;
+  }
+  R.dual[4 * (size_t) self] = first + 2 * p + x;  // the twin: the same triangle, the other end
+}
+
+// at most how many list places the surviving uses of the changed edges take
+__global__ __launch_bounds__(BLOCK) void run_need_k(SwapRunView R, u32 ns, u32* __restrict__ out) {
+  u32 const s = blockIdx.x * BLOCK + threadIdx.x;
+  u32 n = 0;
+  if (s < ns) {
+    u32 const e = R.sw[s], f = R.lb[e], l = R.ln[e];
+    for (u32 j = f; j < f + l; ++j)
+      for (u32 k = 0; k < 6; ++k) n += R.ln[R.te[6 * (size_t) R.ua[j] + k]];
+  }
+#pragma unroll
+  for (u32 d = 32; d >= 1; d >>= 1) n += (u32) __shfl_down((int) n, d, 64);
+  if ((threadIdx.x & 63u) == 0 && n) atomicAdd(out, n);
 }
 
 // every use of an edge by a product tet takes a place among its edge's
@@ -3680,11 +3833,22 @@ __global__ __launch_bounds__(BLOCK) void run_lists_k(SwapRunView R, u32 const* _
   u32 const i = blockIdx.x * BLOCK + threadIdx.x;
   u32 const n = R.words[RW_AFF];
   u32 e = 0, f = 0, l = 0, s = 0, len = 0;
+  // the first RUN_L uses in registers, their loads in flight together
+  constexpr u32 RUN_L = 8;
+  u32 t[RUN_L];
+  bool live[RUN_L];
   if (i < n) {
     e = changed[i];
     f = R.lb[e];
     l = R.ln[e];
-    for (u32 k = f; k < f + l; ++k) s += R.dead[R.ua[k]] ? 0u : 1u;
+#pragma unroll
+    for (u32 k = 0; k < RUN_L; ++k) t[k] = k < l ? R.ua[f + k] : INVALID;
+#pragma unroll
+    for (u32 k = 0; k < RUN_L; ++k) {
+      live[k] = t[k] != INVALID && !R.dead[t[k]];
+      s += live[k] ? 1u : 0u;
+    }
+    for (u32 k = f + RUN_L; k < f + l; ++k) s += R.dead[R.ua[k]] ? 0u : 1u;
     len = s + R.cnt[e];
   }
   // one atomic per wave
@@ -3700,10 +3864,17 @@ __global__ __launch_bounds__(BLOCK) void run_lists_k(SwapRunView R, u32 const* _
   base = (u32) __shfl((int) base, 63) + x - len;
   if (i >= n) return;
   u32 p = base;
-  for (u32 k = f; k < f + l; ++k) {
-    u32 const t = R.ua[k];
-    if (R.dead[t]) continue;
-    R.ua[p] = t;
+#pragma unroll
+  for (u32 k = 0; k < RUN_L; ++k)
+    if (live[k]) {
+      R.ua[p] = t[k];
+      R.ud[p] = R.ud[f + k];
+      ++p;
+    }
+  for (u32 k = f + RUN_L; k < f + l; ++k) {
+    u32 const v = R.ua[k];
+    if (R.dead[v]) continue;
+    R.ua[p] = v;
     R.ud[p] = R.ud[k];
     ++p;
   }
@@ -3742,13 +3913,18 @@ __global__ __launch_bounds__(BLOCK) void run_sort_k(SwapRunView R, u32 const* __
 
 // product faces between two cavities of the pass (swap_dual_k); the accepted
 // candidates' states are cleared and the first live tet is found again
-__global__ __launch_bounds__(BLOCK) void run_settle_k(SwapRunView R, u32 n3, SwapEdgesOf E) {
+__global__ __launch_bounds__(BLOCK) void run_settle_k(SwapRunView R, u32 n3, u32 const* __restrict__ face_prod,
+                                                      u32 const* __restrict__ deferred, u32* __restrict__ err) {
   u32 const i = blockIdx.x * BLOCK + threadIdx.x;
   if (i < 4 * n3) {
     u32* d = R.dual + 4 * (size_t) R.nT + i;
     if (*d == DUAL_PENDING) {
-      u32 const key = E.deferred[i];
-      *d = swap_across(E, E.old_dual[key], key / 4);
+      u32 const key = deferred[i], n = R.dual[key];
+      u32 r = INVALID;
+      for (u32 g = 0; g < 4; ++g)
+        if (R.dual[4 * (size_t) n + g] == key / 4) r = face_prod[4 * (size_t) n + g];
+      if (r == INVALID) *err = ERR_REFLECT_NOT_FOUND;
+      *d = r;
     }
   }
   u32 const n = R.words[RW_ACC];
@@ -3870,7 +4046,7 @@ struct SwapRun {
   u32 nE = 0, nF = 0, nT = 0, nF0 = 0, aE = 0, aF = 0, aT = 0, pass = 0, pool = 0;
   bool has_id = false;
   bool limit_hit = false;  // the independent set reached its round limit
-  u32 got[7];
+  u32 got[6];
   double min_q = 0;
 
   explicit SwapRun(Mesh& mesh) : m(mesh) {}
@@ -3985,7 +4161,7 @@ struct SwapRun {
     nT = aT = count(m, 3);
     pass = 0;
     pool = u.adj.size();
-    size_t const cE = room(nE), cF = room(nF), cT = room(nT), cL = pool + pool / 2 + 4096;
+    size_t const cE = room(nE), cF = room(nF), cT = room(nT), cL = 2 * (size_t) pool + pool / 4 + 4096;
     ev = taken(ask_down(m, 1, 0), 2 * (size_t) nE, 2 * cE);
     ecd = taken(u32_tag(m, 1, "class_dim"), nE, cE);
     vt = taken(ask_down(m, 3, 0), 4 * (size_t) nT, 4 * cT);
@@ -4088,12 +4264,12 @@ struct SwapRun {
                          ds, dev_slot<double>(SLOT_RUN_MIN));
       check_launch("run_offsets");
       sync();
-      for (u32 k = 0; k < 7; ++k) got[k] = hs[k];
+      for (u32 k = 0; k < 6; ++k) got[k] = hs[k];
     };
     totals();
     min_q = *host_slot<double>(SLOT_RUN_MIN);
     if (min_q >= good) return false;
-    if (got[6]) {
+    if (got[5]) {
       // not settled in the first batch: checked batches up to the limit
       rounds_to_the_end(round, flags);
       flag = words.get() + RW_AFF;  // zero: settled
@@ -4244,16 +4420,13 @@ struct SwapRun {
 
   void swap(SwapRunView R, unsigned char const* state, u32 nb) {
     u32 const ns = got[0], n1 = got[1], n2 = got[2], n3 = got[3];
-    if (6 * ((size_t) nT + n3) >= ((size_t) 1 << 32) || (size_t) got[5] + got[4] + 6 * (size_t) n3 >= ((size_t) 1 << 32))
-      fail("swap: more than 2^32 uses", __FILE__, __LINE__);
+    if (6 * ((size_t) nT + n3) >= ((size_t) 1 << 32)) fail("swap: more than 2^32 uses", __FILE__, __LINE__);
     edge_room(nE + n1);
     tet_room(nT + n3);
     need(fv, 3 * (size_t) nF, 3 * ((size_t) nF + n2));
     need(fcd, nF, (size_t) nF + n2);
     if (has_id) need(fci, nF, (size_t) nF + n2);
     need(fbirth, nF - nF0, (size_t) nF - nF0 + n2);
-    need(ua, got[5], (size_t) got[5] + got[4] + 6 * (size_t) n3);
-    need(ud, got[5], (size_t) got[5] + got[4] + 6 * (size_t) n3);
     Buf<u32> lists((size_t) 4 * ns), uses((size_t) 12 * n3), deferred((size_t) 4 * n3);
     // the states may have moved: the round's result is in sa or sb as before
     bool const in_a = state == R.sa;
@@ -4267,26 +4440,34 @@ struct SwapRun {
     u32 *slot = uses.get(), *changed = slot + nuse;
     hipLaunchKernelGGL(run_list_k, dim3(nb), dim3(BLOCK), 0, stream(), R, state, part.get());
     check_launch("run_list");
-    SwapEdgesOf E{};
-    E.out = R.te;
-    E.old = R.te;
-    E.nsame1 = nE;
-    E.nsame3 = nT;
-    E.err = dev_error_word();
-    E.dual = R.dual;
-    E.old_dual = R.dual;
-    E.face_prod = face_prod.get();
-    E.deferred = deferred.get();
+    // the changed edges' lists: their product uses, and no more surviving
+    // uses than all lists have; only where the pool has not that much room
+    // left are the lists around the cavities counted (one more wait)
+    u32 const used = got[4];
+    if (ua.size() < (size_t) used + 6 * (size_t) aT + nuse) {
+      u32* word = words.get() + RW_NEED;
+      hipLaunchKernelGGL(run_need_k, dim3(nblocks(ns)), dim3(BLOCK), 0, stream(), R, ns, word);
+      check_launch("run_need");
+      u32 const* wp = word;
+      u32 bound;
+      read_many(&wp, 1, &bound);
+      size_t const want = (size_t) used + bound + nuse;
+      if (want >= ((size_t) 1 << 32)) fail("swap: more than 2^32 uses", __FILE__, __LINE__);
+      need(ua, used, want);
+      need(ud, used, want);
+      R.ua = ua.get();
+      R.ud = ud.get();
+    }
     launch_timed("swap_cavity", (double) n1 * 8 + (double) n2 * 12 + (double) n3 * 16 + (double) ns * 12,
-                 swap_products_k<true>, dim3(nblocks(ns)), dim3(BLOCK), ns, (u32 const*) nullptr, R.o1, R.o2, R.o3,
-                 (u32 const*) nullptr, R.ua, R.ud, R.ev, R.vt, R.info, R.ev + 2 * (size_t) nE,
-                 R.fv + 3 * (size_t) nF, R.vt + 4 * (size_t) nT, E, R);
+                 run_products_k, dim3(nblocks((size_t) ns * RUN_G)), dim3(BLOCK), R, ns, face_prod.get(),
+                 deferred.get(), dev_error_word());
     element_qualities_into(3, n3, R.vt + 4 * (size_t) nT, coords(m), 0, metric_of(m), tq.get() + nT);
     hipLaunchKernelGGL(run_touch_k, dim3(nblocks(nuse)), dim3(BLOCK), 0, stream(), R, nuse, slot, changed);
     hipLaunchKernelGGL(run_lists_k, dim3(nblocks(nuse)), dim3(BLOCK), 0, stream(), R, changed);
     hipLaunchKernelGGL(run_place_k, dim3(nblocks(nuse)), dim3(BLOCK), 0, stream(), R, nuse, slot);
     hipLaunchKernelGGL(run_sort_k, dim3(nblocks(nuse)), dim3(BLOCK), 0, stream(), R, changed);
-    hipLaunchKernelGGL(run_settle_k, dim3(nblocks(4 * (size_t) n3)), dim3(BLOCK), 0, stream(), R, n3, E);
+    hipLaunchKernelGGL(run_settle_k, dim3(nblocks(4 * (size_t) n3)), dim3(BLOCK), 0, stream(), R, n3,
+                       face_prod.get(), deferred.get(), dev_error_word());
     check_launch("run_settle");
     nE += n1;
     nF += n2;
