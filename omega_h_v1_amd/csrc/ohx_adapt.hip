@@ -3323,16 +3323,42 @@ struct SwapRunView {
   u32* words;
 };
 
-// the index for each lane with pred among those of the launch, one atomic
-// per wave; every lane of the wave must call it
-__device__ inline u32 wave_append(u32* counter, bool pred) {
-  unsigned long long const m = __ballot(pred);
-  if (!m) return 0;
-  u32 const lane = (u32) __lane_id(), leader = (u32) (__ffsll((long long) m) - 1);
-  u32 base = 0;
-  if (lane == leader) base = atomicAdd(counter, (u32) __popcll(m));
-  base = (u32) __shfl((int) base, (int) leader);
-  return base + (u32) __popcll(m & ((1ull << lane) - 1ull));
+// Appending to a run's lists: blocks of RUN_AB threads, RUN_AI items each, one
+// atomic per block and list.  Same-address atomics retire about one per 12 ns
+// on this part, so one per wave held these kernels up (candidates of 3.7
+// million edges 149 us against 45 us with one per 4096 edges).
+constexpr u32 RUN_AB = 1024, RUN_AI = 4, RUN_AT = RUN_AB * RUN_AI;
+// exclusive prefix of c over the block, the block's sum in *total; every
+// thread of the block must call it
+__device__ inline u32 run_block_prefix(u32 c, u32* lds, u32* total) {
+  u32 const lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+  u32 x = c;
+#pragma unroll
+  for (u32 d = 1; d < 64; d <<= 1) {
+    u32 const y = (u32) __shfl_up((int) x, d, 64);
+    if (lane >= d) x += y;
+  }
+  if (lane == 63u) lds[wave] = x;
+  __syncthreads();
+  u32 off = 0, all = 0;
+  for (u32 w = 0; w < RUN_AB / 64; ++w) {
+    u32 const v = lds[w];
+    if (w < wave) off += v;
+    all += v;
+  }
+  __syncthreads();
+  *total = all;
+  return off + x - c;
+}
+// the first list place of this thread's c items
+__device__ inline u32 run_append(u32* counter, u32 c, u32* lds) {
+  u32 total;
+  u32 const p = run_block_prefix(c, lds, &total);
+  if (threadIdx.x == 0) lds[0] = total ? atomicAdd(counter, total) : 0u;
+  __syncthreads();
+  u32 const base = lds[0];
+  __syncthreads();
+  return base + p;
 }
 
 constexpr u32 RUN_RED_BLOCKS = 1024;
@@ -3388,38 +3414,41 @@ __global__ __launch_bounds__(BLOCK) void run_layer_k(u32 n, uint4 const* __restr
 
 // the candidates: live interior edges of marked tets whose swap is accepted
 // (they enter the independent set) or not yet known (to be evaluated)
-__global__ __launch_bounds__(BLOCK) void run_candidates_k(SwapRunView R, unsigned char const* __restrict__ marks) {
-  u32 const e = blockIdx.x * BLOCK + threadIdx.x;
-  bool acc = false, ask = false;
-  if (e < R.nE) {
+__global__ __launch_bounds__(RUN_AB) void run_candidates_k(SwapRunView R, unsigned char const* __restrict__ marks) {
+  __shared__ u32 lds[RUN_AB / 64];
+  u32 const e0 = blockIdx.x * RUN_AT + threadIdx.x;
+  u32 acc = 0, ask = 0;  // bits: this thread's edges e0 + k RUN_AB
+  for (u32 k = 0; k < RUN_AI; ++k) {
+    u32 const e = e0 + k * RUN_AB;
+    if (e >= R.nE) break;
     u32 const w = R.info[e];
-    if (!(w & RI_KNOWN) || (w & RI_ACCEPT)) {
-      // four tets at a time, so that their loads are in flight together
-      bool in = false;
-      u32 const f = R.lb[e], n = R.ln[e];
-      for (u32 k = 0; k < n && !in; k += 4) {
-        u32 t[4];
-#pragma unroll
-        for (u32 j = 0; j < 4; ++j) t[j] = R.ua[f + (k + j < n ? k + j : k)];
-        u32 any = 0;
-#pragma unroll
-        for (u32 j = 0; j < 4; ++j) any |= marks[t[j]];
-        in = any != 0;
-      }
-      acc = in && (w & RI_KNOWN);
-      ask = in && !(w & RI_KNOWN);
+    if ((w & RI_KNOWN) && !(w & RI_ACCEPT)) continue;
+    bool in = false;
+    u32 const f = R.lb[e], n = R.ln[e];
+    for (u32 j = 0; j < n && !in; ++j) in = marks[R.ua[f + j]] != 0;
+    if (in) (w & RI_KNOWN ? acc : ask) |= 1u << k;
+  }
+  // both lists' places in one prefix (a block has at most 4096 of each)
+  u32 total;
+  u32 const p = run_block_prefix((u32) __popc(acc) | ((u32) __popc(ask) << 16), lds, &total);
+  if (threadIdx.x == 0) {
+    lds[0] = (total & 0xffffu) ? atomicAdd(R.words + RW_ACC, total & 0xffffu) : 0u;
+    lds[1] = (total >> 16) ? atomicAdd(R.words + RW_EVAL, total >> 16) : 0u;
+  }
+  __syncthreads();
+  u32 a = lds[0] + (p & 0xffffu), b = lds[1] + (p >> 16);
+  for (u32 k = 0; k < RUN_AI; ++k) {
+    u32 const e = e0 + k * RUN_AB;
+    if ((acc >> k) & 1u) {
+      R.acc[a++] = e;
+      R.sa[e] = UNKNOWN;
     }
+    if ((ask >> k) & 1u) R.eval[b++] = e;
   }
-  u32 const a = wave_append(R.words + RW_ACC, acc), b = wave_append(R.words + RW_EVAL, ask);
-  if (acc) {
-    R.acc[a] = e;
-    R.sa[e] = UNKNOWN;
-  }
-  if (ask) R.eval[b] = e;
 }
 
 // swap qualities of the candidates to evaluate: the choice goes into the
-// edge's word, an accepted edge joins the accepted candidates
+// edge's word
 template <bool MT, bool MIXED>
 __global__ __launch_bounds__(BLOCK, 4) void run_quality_k(SwapRunView R, double const* __restrict__ x,
                                                           double const* __restrict__ mt,
@@ -3435,16 +3464,35 @@ __global__ __launch_bounds__(BLOCK, 4) void run_quality_k(SwapRunView R, double 
     double best;
     bool const accept = swap_quality_batch<MT, MIXED>(L, n, base + group, R.eval, R.lb, R.ln, R.ua, R.ud, R.ev, R.vt,
                                                       x, mt, tq, err, st, &e, &settled, &best, &rs, &code);
-    u32 const a = wave_append(R.words + RW_ACC, accept && lead);
     if (settled && lead) {
       R.info[e] = accept ? RI_KNOWN | RI_ACCEPT | (rs << 16) | code : RI_KNOWN;
-      if (accept) {
-        R.q[e] = best;
-        R.acc[a] = e;
-        R.sa[e] = UNKNOWN;
-      }
+      if (accept) R.q[e] = best;
     }
     __syncthreads();  // the next batch reuses the staging
+  }
+}
+
+// the evaluated candidates that are accepted join the accepted ones
+__global__ __launch_bounds__(RUN_AB) void run_accept_k(SwapRunView R) {
+  __shared__ u32 lds[RUN_AB / 64];
+  u32 const n = R.words[RW_EVAL];
+  for (u32 base = blockIdx.x * RUN_AT; base < n; base += gridDim.x * RUN_AT) {
+    u32 e[RUN_AI], in = 0;
+#pragma unroll
+    for (u32 k = 0; k < RUN_AI; ++k) {
+      u32 const i = base + k * RUN_AB + threadIdx.x;
+      e[k] = i < n ? R.eval[i] : INVALID;
+    }
+#pragma unroll
+    for (u32 k = 0; k < RUN_AI; ++k)
+      if (e[k] != INVALID && (R.info[e[k]] & RI_ACCEPT)) in |= 1u << k;
+    u32 a = run_append(R.words + RW_ACC, (u32) __popc(in), lds);
+#pragma unroll
+    for (u32 k = 0; k < RUN_AI; ++k)
+      if ((in >> k) & 1u) {
+        R.acc[a++] = e[k];
+        R.sa[e[k]] = UNKNOWN;
+      }
   }
 }
 
@@ -3811,26 +3859,36 @@ __global__ __launch_bounds__(BLOCK) void run_need_k(SwapRunView R, u32 ns, u32* 
 // every use of an edge by a product tet takes a place among its edge's
 // product uses; the edge's first one puts the edge on the list of changed
 // edges
-__global__ __launch_bounds__(BLOCK) void run_touch_k(SwapRunView R, u32 nuse, u32* __restrict__ slot,
-                                                     u32* __restrict__ changed) {
-  u32 const u = blockIdx.x * BLOCK + threadIdx.x;
-  bool first = false;
-  u32 e = 0;
-  if (u < nuse) {
-    e = R.te[6 * (size_t) R.nT + u];
-    u32 const s = e != INVALID ? atomicAdd(&R.cnt[e], 1u) : 1u;
-    slot[u] = s;
-    first = s == 0;
+__global__ __launch_bounds__(RUN_AB) void run_touch_k(SwapRunView R, u32 nuse, u32* __restrict__ slot,
+                                                      u32* __restrict__ changed) {
+  __shared__ u32 lds[RUN_AB / 64];
+  u32 const u0 = blockIdx.x * RUN_AT + threadIdx.x;
+  u32 e[RUN_AI], first = 0;
+#pragma unroll
+  for (u32 k = 0; k < RUN_AI; ++k) {
+    u32 const u = u0 + k * RUN_AB;
+    e[k] = u < nuse ? R.te[6 * (size_t) R.nT + u] : INVALID;
   }
-  u32 const a = wave_append(R.words + RW_AFF, first);
-  if (first) changed[a] = e;
+#pragma unroll
+  for (u32 k = 0; k < RUN_AI; ++k) {
+    u32 const u = u0 + k * RUN_AB;
+    if (u >= nuse) continue;
+    u32 const s = e[k] != INVALID ? atomicAdd(&R.cnt[e[k]], 1u) : 1u;
+    slot[u] = s;
+    if (s == 0) first |= 1u << k;
+  }
+  u32 a = run_append(R.words + RW_AFF, (u32) __popc(first), lds);
+#pragma unroll
+  for (u32 k = 0; k < RUN_AI; ++k)
+    if ((first >> k) & 1u) changed[a++] = e[k];
 }
 
 // a changed edge's new list: a place in the pool for its surviving and its
 // product uses, the survivors copied in order; cnt is then the survivors'
 // number.  Its swap is not known any more.
-__global__ __launch_bounds__(BLOCK) void run_lists_k(SwapRunView R, u32 const* __restrict__ changed) {
-  u32 const i = blockIdx.x * BLOCK + threadIdx.x;
+__global__ __launch_bounds__(RUN_AB) void run_lists_k(SwapRunView R, u32 const* __restrict__ changed) {
+  __shared__ u32 lds[RUN_AB / 64];
+  u32 const i = blockIdx.x * RUN_AB + threadIdx.x;
   u32 const n = R.words[RW_AFF];
   u32 e = 0, f = 0, l = 0, s = 0, len = 0;
   // the first RUN_L uses in registers, their loads in flight together
@@ -3851,17 +3909,7 @@ __global__ __launch_bounds__(BLOCK) void run_lists_k(SwapRunView R, u32 const* _
     for (u32 k = f + RUN_L; k < f + l; ++k) s += R.dead[R.ua[k]] ? 0u : 1u;
     len = s + R.cnt[e];
   }
-  // one atomic per wave
-  u32 const lane = (u32) __lane_id();
-  u32 x = len;
-#pragma unroll
-  for (u32 d = 1; d < 64; d <<= 1) {
-    u32 const y = (u32) __shfl_up((int) x, d, 64);
-    if (lane >= d) x += y;
-  }
-  u32 base = 0;
-  if (lane == 63u && x) base = atomicAdd(R.words + RW_POOL, x);
-  base = (u32) __shfl((int) base, 63) + x - len;
+  u32 const base = run_append(R.words + RW_POOL, len, lds);
   if (i >= n) return;
   u32 p = base;
 #pragma unroll
@@ -4240,7 +4288,7 @@ struct SwapRun {
       check_launch("run_layer");
       std::swap(marks, marks2);
     }
-    hipLaunchKernelGGL(run_candidates_k, dim3(nblocks(nE)), dim3(BLOCK), 0, stream(), R, marks.get());
+    hipLaunchKernelGGL(run_candidates_k, dim3(nblocks(nE, RUN_AT)), dim3(RUN_AB), 0, stream(), R, marks.get());
     check_launch("run_candidates");
     evaluate(R);
     // a first batch of rounds with no host check, as the other passes
@@ -4295,6 +4343,9 @@ struct SwapRun {
       mt ? go(run_quality_k<true, true>, "swap_quality_mixed") : go(run_quality_k<false, true>, "swap_quality_mixed");
     else
       mt ? go(run_quality_k<true, false>, "swap_quality_f64") : go(run_quality_k<false, false>, "swap_quality_f64");
+    u32 const ab = nblocks(aE, RUN_AT);
+    hipLaunchKernelGGL(run_accept_k, dim3(ab < 256 ? ab : 256), dim3(RUN_AB), 0, stream(), R);
+    check_launch("run_accept");
   }
 
   template <class F>
@@ -4462,8 +4513,8 @@ struct SwapRun {
                  run_products_k, dim3(nblocks((size_t) ns * RUN_G)), dim3(BLOCK), R, ns, face_prod.get(),
                  deferred.get(), dev_error_word());
     element_qualities_into(3, n3, R.vt + 4 * (size_t) nT, coords(m), 0, metric_of(m), tq.get() + nT);
-    hipLaunchKernelGGL(run_touch_k, dim3(nblocks(nuse)), dim3(BLOCK), 0, stream(), R, nuse, slot, changed);
-    hipLaunchKernelGGL(run_lists_k, dim3(nblocks(nuse)), dim3(BLOCK), 0, stream(), R, changed);
+    hipLaunchKernelGGL(run_touch_k, dim3(nblocks(nuse, RUN_AT)), dim3(RUN_AB), 0, stream(), R, nuse, slot, changed);
+    hipLaunchKernelGGL(run_lists_k, dim3(nblocks(nuse, RUN_AB)), dim3(RUN_AB), 0, stream(), R, changed);
     hipLaunchKernelGGL(run_place_k, dim3(nblocks(nuse)), dim3(BLOCK), 0, stream(), R, nuse, slot);
     hipLaunchKernelGGL(run_sort_k, dim3(nblocks(nuse)), dim3(BLOCK), 0, stream(), R, changed);
     hipLaunchKernelGGL(run_settle_k, dim3(nblocks(4 * (size_t) n3)), dim3(BLOCK), 0, stream(), R, n3,
