@@ -977,6 +977,13 @@ __device__ inline double group_min(double v) {
 // of the vertices that need exact values.
 enum CqMode : u32 { CQ_F64 = 0, CQ_SCREEN = 1, CQ_CERTIFIED = 2, CQ_FORCE = 3 };
 __host__ __device__ inline u32 inexact_bit(u32 d) { return 4u << d; }
+// further bits of a code word: the direction's quality is known from an
+// earlier pass (accepted), and it was measured in this one and rejected
+__host__ __device__ inline u32 known_bit(u32 d) { return 16u << d; }
+__host__ __device__ inline u32 rejected_bit(u32 d) { return 64u << d; }
+// SizeCodeCache::known: accepted (1 << d), rejected, inexact
+__host__ __device__ inline u32 was_rejected(u32 d) { return 4u << d; }
+__host__ __device__ inline u32 was_inexact(u32 d) { return 16u << d; }
 
 template <u32 DIM, bool F32>
 __device__ inline double collapse_elem_q(u32 e, u32 dir, u32 gen, V3 const& pg, Sym const& mg,
@@ -1080,7 +1087,7 @@ __global__ __launch_bounds__(BLOCK) void coarsen_quality_f64(CqArgs A) {
     bool accept = MODE == CQ_CERTIFIED && !nan && minq32 > qual_floor + (double) SCREEN_MARGIN;
     if (lane == 0) wave_count(st.screened, reject || accept);
     if (reject) {
-      if (lane == 0) atomicAnd(&codes[i], ~((1u << j) | inexact_bit(j)));
+      if (lane == 0) atomicXor(&codes[i], (1u << j) | rejected_bit(j));
       return;
     }
     if (accept) {
@@ -1114,7 +1121,9 @@ __global__ __launch_bounds__(BLOCK) void coarsen_quality_f64(CqArgs A) {
     note_max_err(st.max_err, (float) (d < 0 ? -d : d));
   }
   if ((minq < qual_floor) || (eq && (minq <= old_minq))) {
-    atomicAnd(&codes[i], ~((1u << j) | inexact_bit(j)));
+    // the direction's bit is set and its rejected bit is not, and the
+    // inexact bit is set exactly where an FP32 value is measured again
+    atomicXor(&codes[i], (1u << j) | rejected_bit(j) | (MODE == CQ_FORCE ? inexact_bit(j) : 0u));
   } else {
     out[2 * (size_t) i + j] = minq;
     if (MODE == CQ_FORCE) atomicAnd(&codes[i], ~inexact_bit(j));
@@ -1217,22 +1226,58 @@ __global__ __launch_bounds__(BLOCK) void coarsen_size_code_f64(u32 n, u32 const*
 }
 
 // size codes carried to a collapse pass's new mesh: threads [0, ne_old)
-// give a surviving edge its old code; the next ngen measure a product edge
-__global__ __launch_bounds__(BLOCK) void carry_size_codes_k(u32 ne_old, u32 ngen, u32 nsame,
-                                                            u32 const* __restrict__ soff,
-                                                            u32 const* __restrict__ old_codes,
-                                                            u32 const* __restrict__ ev, double const* __restrict__ x,
-                                                            double const* __restrict__ h,
-                                                            double const* __restrict__ mt, double floor_,
-                                                            u32* __restrict__ codes) {
+// give a surviving edge its old code; the next ngen measure a product edge.
+// A surviving edge's direction whose collapsing vertex kept all its elements
+// and gained none also keeps what is known of its quality: the quality reads
+// those elements, their vertices and the target's position, and a collapse
+// moves no vertex.
+struct CarryCodes {
+  u32 ne_old, ngen, nsame;
+  u32 const* soff;
+  u32 const* old_codes;
+  u32 const* ev;  // the new mesh's
+  double const* x;
+  double const* h;
+  double const* mt;
+  double floor_;
+  u32* codes;
+  u32 const* now;        // the pass's code words
+  u32 const* old_known;  // or null
+  double const* q;
+  u32 const* old_ev;
+  u32 const* vsoff;
+  u32 const* full;  // per new vertex (UpPatchCounts)
+  u32 const* cnt;
+  u32 const* cnt_s;
+  u32* known;
+  double* new_q;
+};
+__global__ __launch_bounds__(BLOCK) void carry_size_codes_k(CarryCodes a) {
   u32 t = xcd_block() * BLOCK + threadIdx.x;
-  if (t < ne_old) {
-    u32 o = soff[t];
-    if (o != soff[t + 1]) codes[o] = old_codes[t];
-  } else if (t - ne_old < ngen) {
-    u32 i = nsame + (t - ne_old);
-    double sz = edge_size(ev[2 * i], ev[2 * i + 1], x, h, mt);
-    codes[i] = (sz < floor_) ? (u32) COLLAPSE_BOTH : (u32) DONT_COLLAPSE;
+  if (t < a.ne_old) {
+    u32 o = a.soff[t];
+    if (o == a.soff[t + 1]) return;
+    a.codes[o] = a.old_codes[t];
+    u32 const c = a.now[t], was = a.old_known ? a.old_known[t] : 0u;
+    u32 k = 0;
+    for (u32 d = 0; d < 2; ++d) {
+      u32 b = was & ((1u << d) | was_rejected(d) | was_inexact(d));
+      if (collapses(c, d))
+        b = (1u << d) | ((c & inexact_bit(d)) ? was_inexact(d) : 0u);
+      else if (c & rejected_bit(d))
+        b = was_rejected(d);
+      if (!b) continue;
+      u32 const v = a.vsoff[a.old_ev[2 * (size_t) t + d]];
+      if (!a.full[v] || a.cnt[v] != a.cnt_s[v]) continue;
+      k |= b;
+      if (b & (1u << d)) a.new_q[2 * (size_t) o + d] = a.q[2 * (size_t) t + d];
+    }
+    a.known[o] = k;
+  } else if (t - a.ne_old < a.ngen) {
+    u32 i = a.nsame + (t - a.ne_old);
+    double sz = edge_size(a.ev[2 * i], a.ev[2 * i + 1], a.x, a.h, a.mt);
+    a.codes[i] = (sz < a.floor_) ? (u32) COLLAPSE_BOTH : (u32) DONT_COLLAPSE;
+    a.known[i] = 0;
   }
 }
 
@@ -1618,9 +1663,12 @@ static u32 coarsen_common(Mesh& m, Buf<u32>& codes, double qual_floor, bool requ
   // The list is the uses of up(0,1) that collapse, in use order, so one
   // flat scan over the uses numbers them (no per-vertex loop), and a
   // vertex's first direction is the scan at its first use.
-  u32 ncand;
-  Buf<u32> clist, voff;
+  // Where the loop carries known qualities, only the directions without one
+  // are measured: a second list, from a second scan before the same read.
+  u32 ncand, neval;
+  Buf<u32> clist, elist, voff;
   u32 const nv0 = count(m, 0);
+  bool const some_known = sizes && sizes->known;
   {
     Up const& uv = ask_up(m, 0, 1);
     u32 const* uo = uv.offsets.get();
@@ -1628,16 +1676,35 @@ static u32 coarsen_common(Mesh& m, Buf<u32>& codes, double qual_floor, bool requ
     u32 const* ud = uv.dirs.get();
     u32 const* cp = codes.get();
     u32 const nuse = 2 * ne;
-    Buf<u32> uoff(nuse + 1);
-    ncand = exscan_fn_total(nuse, OHX_LAMBDA(u32 k) { return collapses(cp[ua[k]], ud[k]); }, uoff.get());
+    Buf<u32> uoff(nuse + 1), eoff;
+    auto listed = OHX_LAMBDA(u32 k) { return collapses(cp[ua[k]], ud[k]); };
+    if (some_known) {
+      eoff = Buf<u32>(nuse + 1);
+      exscan_fn(nuse, listed, uoff.get());
+      exscan_fn(nuse, OHX_LAMBDA(u32 k) {
+        u32 const c = cp[ua[k]], d = ud[k];
+        return collapses(c, d) && !(c & known_bit(d)) ? 1u : 0u;
+      }, eoff.get());
+      u32 const* ptrs[2] = {uoff.get() + nuse, eoff.get() + nuse};
+      u32 n[2];
+      read_many(ptrs, 2, n);
+      ncand = n[0];
+      neval = n[1];
+    } else {
+      ncand = neval = exscan_fn_total(nuse, listed, uoff.get());
+    }
     if (!ncand) return 0;
     clist = Buf<u32>(ncand);
+    if (some_known) elist = Buf<u32>(neval);
     voff = Buf<u32>(nv0 + 1);
     u32 const* uf = uoff.get();
+    u32 const* ef = eoff.get();
     u32* cl = clist.get();
+    u32* el = elist.get();
     u32* vo = voff.get();
     parallel_for(nuse > nv0 ? nuse : nv0 + 1, OHX_LAMBDA(u32 k) {
       if (k < nuse && uf[k] != uf[k + 1]) cl[uf[k]] = 2 * ua[k] + ud[k];
+      if (ef && k < nuse && ef[k] != ef[k + 1]) el[ef[k]] = 2 * ua[k] + ud[k];
       if (k <= nv0) vo[k] = uf[uo[k]];
     });
   }
@@ -1652,7 +1719,7 @@ static u32 coarsen_common(Mesh& m, Buf<u32>& codes, double qual_floor, bool requ
     if (!eq_given) eq = element_qualities(dim, count(m, dim), vel, coords(m), count(m, 0), metric_of(m));
     eqp = eq_given ? eq_given : eq.get();
   }
-  Buf<double> cq((size_t) 2 * ne);
+  Buf<double> cq = some_known ? std::move(sizes->q) : Buf<double>((size_t) 2 * ne);
   Buf<u32> cand;
   Buf<double> vq;
   {
@@ -1671,11 +1738,11 @@ static u32 coarsen_common(Mesh& m, Buf<u32>& codes, double qual_floor, bool requ
          Tuner("coarsen_quality_3d_mixed", {33, 34, 36, 40, 17, 18, 20, 24}),
          Tuner("coarsen_quality_3d_mixed_small", {1, 2, 4, 8})}};
     constexpr u32 CQ_CERTIFIED_MIN = 4096;
-    bool const big = ncand >= CQ_CERTIFIED_MIN || tuners[dim == 3][1].forced();
+    bool const big = neval >= CQ_CERTIFIED_MIN || tuners[dim == 3][1].forced();
     Tuner& tuner = tuners[dim == 3][g_mixed ? (big ? 1 : 2) : 0];
     CqArgs a{};
-    a.ncand = ncand;
-    a.list = clist.get();
+    a.ncand = neval;
+    a.list = some_known ? elist.get() : clist.get();
     a.ev = ev;
     a.uo = ue.offsets.get();
     a.ua = ue.adj.get();
@@ -1699,13 +1766,17 @@ static u32 coarsen_common(Mesh& m, Buf<u32>& codes, double qual_floor, bool requ
     Up const& uv = ask_up(m, 0, 1);
     cand = Buf<u32>(nv);
     vq = Buf<double>(nv);
-    tuned(tuner, ncand, [&](u32 var, hipEvent_t ea, hipEvent_t eb) {
+    auto measure = [&](u32 var, hipEvent_t ea, hipEvent_t eb) {
       u32 g = var & 15u;
       u32 mode = (var & 32u) ? (u32) CQ_CERTIFIED : (var & 16u) ? (u32) CQ_SCREEN : (u32) CQ_F64;
-      bool const certified = mode == CQ_CERTIFIED && !require_better;
+      bool const measures32 = mode == CQ_CERTIFIED && !require_better;
+      if (sizes && measures32) sizes->inexact = true;
+      // FP32 values may also come from an earlier pass
+      bool const certified = measures32 || (sizes && sizes->inexact);
       if (ea) OHX_CHECK(hipEventRecord(ea, stream()));
-      dim == 3 ? cq_launch_mode<3>(mode, g, a, prof_bytes, nullptr, nullptr)
-               : cq_launch_mode<2>(mode, g, a, prof_bytes, nullptr, nullptr);
+      if (neval)
+        dim == 3 ? cq_launch_mode<3>(mode, g, a, prof_bytes, nullptr, nullptr)
+                 : cq_launch_mode<2>(mode, g, a, prof_bytes, nullptr, nullptr);
       Buf<u32> vinex, vmark;
       if (certified) vinex = Buf<u32>(nv);
       auto to_vert = [&] {
@@ -1726,13 +1797,19 @@ static u32 coarsen_common(Mesh& m, Buf<u32>& codes, double qual_floor, bool requ
                            vmark.get());
         check_launch("coarsen_certify");
         CqArgs f = a;
+        f.ncand = ncand;
+        f.list = clist.get();
         f.vmark = vmark.get();
         dim == 3 ? cq_launch_mode<3>(CQ_FORCE, g, f, prof_bytes, nullptr, nullptr)
                  : cq_launch_mode<2>(CQ_FORCE, g, f, prof_bytes, nullptr, nullptr);
         to_vert();
       }
       if (eb) OHX_CHECK(hipEventRecord(eb, stream()));
-    });
+    };
+    if (neval)
+      tuned(tuner, neval, measure);
+    else
+      measure(1, nullptr, nullptr);
   }
   // no host check here: if the quality check left no collapse, the
   // candidates below are empty, the independent set settles at once and the
@@ -1879,8 +1956,10 @@ static u32 coarsen_common(Mesh& m, Buf<u32>& codes, double qual_floor, bool requ
   }
   if (g_batch) batch_note_changed(m, 0, indset.get());
   cand.release();
-  codes.release();
-  cq.release();
+  if (!sizes) {
+    codes.release();
+    cq.release();
+  }
   vq.release();
   u32 total = got[1];
   if (!total) return 0;
@@ -1979,23 +2058,49 @@ static u32 coarsen_common(Mesh& m, Buf<u32>& codes, double qual_floor, bool requ
       if (side_maps[h][l]) mo.down[h][l] = std::move(side_maps[h][l]);
   // the vertices' upward adjacencies this pass read (to edges, to
   // elements), carried too (vertices survive or are removed, none is new)
+  UpPatchCounts elems;  // which vertices kept their elements
   auto carry_up = [&](u32 h) {
     if (!m.up[0][h]) return;
     mo.up[0][h] = up_patch(h_down_deg[h][0], *m.up[0][h], m.counts[0], soff.get(), nv_out, 0, plan[h].esoff.get(),
-                           got[2 + 2 * (h - 1) + 1], got[2 + 2 * (h - 1)], mo.down[h][0].get());
+                           got[2 + 2 * (h - 1) + 1], got[2 + 2 * (h - 1)], mo.down[h][0].get(),
+                           h == dim && sizes ? &elems : nullptr);
   };
   carry_up(1);
   carry_up(dim);
   if (sizes && sizes->ne == m.counts[1]) {
-    // the new mesh's size codes: survivors' carried, products measured
-    u32 const ne_old = m.counts[1], ngen1 = got[2], nsame1 = got[3];
-    Buf<u32> nc((size_t) nsame1 + ngen1);
-    hipLaunchKernelGGL(carry_size_codes_k, dim3(nblocks((size_t) ne_old + ngen1)), dim3(BLOCK), 0, stream(), ne_old,
-                       ngen1, nsame1, plan[1].esoff.get(), sizes->codes.get(), mo.down[1][0].get(), coords(mo),
-                       size_of(mo), metric_of(mo), size_floor, nc.get());
+    // the new mesh's size codes: survivors' carried, products measured;
+    // and what is known of the survivors' qualities
+    u32 const ne_old = m.counts[1], ngen1 = got[2], nsame1 = got[3], ne_new = nsame1 + ngen1;
+    Buf<u32> nc(ne_new), nk(ne_new);
+    Buf<double> nq((size_t) 2 * ne_new);
+    CarryCodes a{};
+    a.ne_old = ne_old;
+    a.ngen = ngen1;
+    a.nsame = nsame1;
+    a.soff = plan[1].esoff.get();
+    a.old_codes = sizes->codes.get();
+    a.ev = mo.down[1][0].get();
+    a.x = coords(mo);
+    a.h = size_of(mo);
+    a.mt = metric_of(mo);
+    a.floor_ = size_floor;
+    a.codes = nc.get();
+    a.now = codes.get();
+    a.old_known = sizes->known.get();
+    a.q = cq.get();
+    a.old_ev = ev;
+    a.vsoff = soff.get();
+    a.full = elems.full.get();
+    a.cnt = elems.cnt.get();
+    a.cnt_s = elems.cnt_s.get();
+    a.known = nk.get();
+    a.new_q = nq.get();
+    hipLaunchKernelGGL(carry_size_codes_k, dim3(nblocks((size_t) ne_old + ngen1)), dim3(BLOCK), 0, stream(), a);
     check_launch("carry_size_codes");
-    sizes->ne = nsame1 + ngen1;
+    sizes->ne = ne_new;
     sizes->codes = std::move(nc);
+    sizes->known = std::move(nk);
+    sizes->q = std::move(nq);
   } else if (sizes) {
     sizes->clear();
   }
@@ -2017,13 +2122,21 @@ u32 coarsen_by_size(Mesh& m, double qual_floor, double size_floor, SizeCodeCache
   if (cache && cache->ne != ne) cache->clear();
   if (ne && cache && cache->ne) {
     // the codes carried from the pass before (the pass consumes its copy)
+    // -- without the directions known to be rejected, the accepted ones
+    // marked so that they are not measured again
     u32* c = codes.get();
     u32 const* cc = cache->codes.get();
+    u32 const* kn = cache->known.get();
     u32* words = scratch_words();
     parallel_for(ne, OHX_LAMBDA(u32 i) {
-      u32 const v = cc[i];
+      u32 v = cc[i];
+      u32 const k = kn && v ? kn[i] : 0u;
+      for (u32 d = 0; d < 2; ++d) {
+        if (k & was_rejected(d)) v = dont_collapse(v, d);
+        if (k & (1u << d)) v |= known_bit(d) | ((k & was_inexact(d)) ? inexact_bit(d) : 0u);
+      }
       c[i] = v;
-      wave_flag_value(words + W_ANY, v != 0, tag);
+      wave_flag_value(words + W_ANY, (v & (u32) COLLAPSE_BOTH) != 0, tag);
     });
   } else if (ne) {
     double prof_bytes = (double) ne * 12 + (double) count(m, 0) * 32;

@@ -15,12 +15,22 @@ void uniformly_refine(Mesh& m);
 // mesh: a surviving edge keeps its vertices, their coordinates and the
 // metric, so its code (its length against the floor) stays what it was;
 // only the product edges of a pass are measured again.
+// What the collapse-by-size loop carries from pass to pass: the edges' size
+// codes, and what is known of their collapse qualities (per edge and
+// direction: accepted with its value, and whether that is an FP32 value, or
+// rejected), which stands as long as the collapsing vertex keeps its elements
 struct SizeCodeCache {
   u32 ne = 0;  // edges of the mesh it describes (0: empty)
   Buf<u32> codes;
+  Buf<u32> known;  // null: nothing known yet
+  Buf<double> q;
+  bool inexact = false;  // some values are FP32
   void clear() {
     ne = 0;
     codes.release();
+    known.release();
+    q.release();
+    inexact = false;
   }
 };
 u32 coarsen_by_size(Mesh& m, double qual_floor, double size_floor, SizeCodeCache* cache = nullptr);
