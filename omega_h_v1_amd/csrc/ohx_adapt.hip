@@ -334,6 +334,11 @@ static Buf<u32> find_indset_resume(Mesh& m, u32 ent_dim, double const* good, Buf
   return indset_rounds(m, ent_dim, nullptr, good, 0, nullptr, &state, first_batch_rounds());
 }
 
+struct UpPatchCounts;
+static std::unique_ptr<Up> up_patch(u32 deg, Up const& old, u32 nl_old, u32 const* soff_l, u32 nsame_l,
+                                    u32 ngen_l, u32 const* soff_h, u32 nsame_h, u32 ngen_h, u32 const* dn,
+                                    UpPatchCounts* keep = nullptr);
+
 // ------------------------------------------------------------- inherit
 // Class tags (class_dim, class_id) of products come from the entity they
 // were made from (inherit.cpp:14-232); the fused output kernels of each
@@ -579,6 +584,13 @@ static void refine_verts(Mesh& m, Mesh& mo, u32 const* gen_off, u32 nsplit) {
   check_launch("refine_vertex_tags");
 }
 
+// whether the mesh has element fields that the passes transfer
+static bool has_element_transfer(Mesh& m) {
+  for (auto& t : m.tags[m.dim])
+    if (t->transfer == 1 || t->transfer == 2) return true;  // OSH_TRANSFER_POINTWISE, _CONSERVE
+  return false;
+}
+
 static u32 prods_per_dom(u32 dom_dim, u32 src_dim, u32 prod_dim) {  // refine_topology.cpp:110-121
   if (prod_dim == 0) return (dom_dim == src_dim) ? 1 : 0;
   u32 base_dim = prod_dim - 1;
@@ -587,57 +599,161 @@ static u32 prods_per_dom(u32 dom_dim, u32 src_dim, u32 prod_dim) {  // refine_to
   return h_down_deg[src_dim][opp_dim];
 }
 
-// Arguments of the fused refine product kernel (one prod dimension).
+// Arguments of the fused refine product kernel.
 struct RefineArgs {
-  u32 dim, pd;
+  u32 dim;
   u32 nv;
   u32 n[4];                // entity counts
   u32 const* off[4];       // split offsets of domains of each dim (off[1] = edge split offsets)
   u32 const* verts_of[4];  // down(d, 0)
   u32 const* edges_of[4];  // down(d, 1), d >= 2
-  u32 const* soff;         // survivor offsets of dim pd (pd >= 1)
-  u32 ppd[4];              // products per splitting domain of dim d
-  u32 go[4];               // output base of the products of domains of dim d
-  u32 seg[5];              // index space: [survivors | doms of d = 1..3]
-  u32* out_verts;          // pd >= 1
+  u32 const* faces_of;     // down(3, 2), when maps are carried
   u32 const* cd[4];        // class_dim / class_id per dim (may be null)
   u32 const* ci[4];
-  u32* out_cd;
-  u32* out_ci;
+  struct Prod {            // one product dimension
+    u32 block0;            // its first block
+    u32 ppd[4];            // products per splitting domain of dim d
+    u32 go[4];             // output base of the products of domains of dim d
+    u32 seg[4];            // index space: [survivors | doms of d = 1..3]
+    u32* out_verts;        // pd >= 1
+    u32* out_cd;
+    u32* out_ci;
+    u32* out_edges;        // the new down(pd, 1), pd >= 2, when carried
+    u32* out_faces;        // the new down(3, 2), when carried
+    u32* soff;             // survivor offsets of dim pd, when wanted
+  } p[4];
 };
 
-// refine_ents (refine_common.cpp:64-129) for one product dimension, fused:
-// survivors keep their vertices and class (inherit.cpp:104-138); every
-// splitting domain (split_to_domain, splits_to_domains.cpp:13-56: along its
-// first split edge) emits its products (refine_domain_entity,
-// refine_topology.cpp:26-107: the base opposite each of the edge's
-// opposite-dim entities + the new vertex), classified like the domain.
+// local vertices of a tet's edge d (of a triangle's for d < 3), its opposite
+// edge, the face opposite a local vertex, the edge between two local vertices
+// (k_r_e_v, k_f_e_v, k_o_r_e, k_o_r_v), a digit each
+__device__ inline u32 tet_ev0(u32 d) { return (0x210210u >> (4 * d)) & 3u; }
+__device__ inline u32 tet_ev1(u32 d) { return (0x333021u >> (4 * d)) & 3u; }
+__device__ inline u32 tet_oe(u32 d) { return (0x021435u >> (4 * d)) & 7u; }
+__device__ inline u32 tet_face_without(u32 v) { return (0x0132u >> (4 * v)) & 3u; }
+__device__ inline u32 tet_edge_of(u32 a, u32 b) {
+  return a == 3 ? 3 + b : b == 3 ? 3 + a : a + b == 1 ? 0u : a + b == 3 ? 1u : 2u;
+}
+
+// The sides of the entities a split pass makes, without looking them up.  A
+// domain entity has one split edge (the set's edges share no element), at
+// vertex v, with ends p and q.  A side of a product without v is a side of
+// the domain that keeps one end, so it survives; one with v and the end E
+// is the half, on E's side, of the domain's side on both ends; one with v
+// and no end is what the domain's side on both ends and the others makes
+// inside.
+struct RefineSides {
+  RefineArgs const& a;
+  __device__ u32 survivor(u32 d, u32 i) const { return i - a.off[d][i]; }
+  // the half of split edge e without vertex x; of split face f (its split
+  // edge e)
+  __device__ u32 half_edge(u32 e, u32 x) const {
+    return a.p[1].go[1] + 2 * a.off[1][e] + (a.verts_of[1][2 * (size_t) e] == x ? 0u : 1u);
+  }
+  __device__ u32 half_face(u32 f, u32 e, u32 x) const {
+    u32 const* fe = a.edges_of[2] + 3 * (size_t) f;
+    u32 const k = fe[0] == e ? 0u : fe[1] == e ? 1u : 2u;
+    return a.p[2].go[2] + 2 * a.off[2][f] + (a.verts_of[2][3 * (size_t) f + k] == x ? 0u : 1u);
+  }
+  __device__ u32 inner_edge(u32 f) const { return a.p[1].go[2] + a.off[2][f]; }
+  __device__ u32 inner_face(u32 t) const { return a.p[2].go[3] + a.off[3][t]; }
+
+  // product j of triangle i, split edge dir: (b0, b1, v) with the edge b0 b1
+  // opposite the end that goes
+  __device__ void tri(u32 i, u32 dir, u32 j, u32 const* vd, u32* out) const {
+    u32 const* e = a.edges_of[2] + 3 * (size_t) i;
+    u32 const ends[2] = {tet_ev0(dir), tet_ev1(dir)};
+    u32 const gone = ends[j], kept = ends[1 - j];
+    u32 const opp_e = (gone + 1) % 3, b0 = opp_e, b1 = (opp_e + 1) % 3;
+    u32 const half = half_edge(e[dir], vd[gone]), inner = inner_edge(i);
+    out[0] = survivor(1, e[opp_e]);
+    out[1] = b1 == kept ? half : inner;
+    out[2] = b0 == kept ? half : inner;
+  }
+  // the face a split tet makes inside: (c0, c1, v) on the edge opposite
+  __device__ void tet_inner(u32 i, u32 dir, u32* out) const {
+    u32 const* e = a.edges_of[3] + 6 * (size_t) i;
+    u32 const* f = a.faces_of + 4 * (size_t) i;
+    u32 const o = tet_oe(dir), c0 = tet_ev0(o), c1 = tet_ev1(o);
+    out[0] = survivor(1, e[o]);
+    // the face on both ends and c is the one without the other
+    out[1] = inner_edge(f[tet_face_without(c0)]);
+    out[2] = inner_edge(f[tet_face_without(c1)]);
+  }
+  // product j of tet i: (b0, b1, b2, v) with the face b0 b1 b2 opposite the
+  // end that goes
+  __device__ void tet(u32 i, u32 dir, u32 j, u32 const* vd, u32* oe, u32* of) const {
+    u32 const* e = a.edges_of[3] + 6 * (size_t) i;
+    u32 const* f = a.faces_of + 4 * (size_t) i;
+    u32 const p = tet_ev0(dir), q = tet_ev1(dir);
+    u32 const gone = j == 0 ? p : q, kept = j == 0 ? q : p;
+    u32 const base = tet_face_without(gone);
+    u32 const* b = k_r_f_v[base];
+    u32 const x = vd[gone], half = half_edge(e[dir], x), inner = inner_face(i);
+    // the face on both ends and local vertex s
+    auto on = [&](u32 s) { return f[tet_face_without(6 - p - q - s)]; };
+    for (u32 k = 0; k < 3; ++k) {
+      u32 const u = b[k], w = b[(k + 1) % 3];
+      oe[k] = survivor(1, e[tet_edge_of(u, w)]);
+      oe[3 + k] = u == kept ? half : inner_edge(on(u));
+      // the face of v and the edge u w: local faces 1, 2, 3 are on the
+      // base's edges 0-1, 1-2, 2-0
+      of[1 + k] = u == kept ? half_face(on(w), e[dir], x) : w == kept ? half_face(on(u), e[dir], x) : inner;
+    }
+    of[0] = survivor(2, f[base]);
+  }
+};
+
+// refine_ents (refine_common.cpp:64-129), every product dimension in one
+// launch (a range of blocks each): survivors keep their vertices and class
+// (inherit.cpp:104-138); every splitting domain (split_to_domain,
+// splits_to_domains.cpp:13-56: along its first split edge) emits its products
+// (refine_domain_entity, refine_topology.cpp:26-107: the base opposite each
+// of the edge's opposite-dim entities + the new vertex), classified like the
+// domain.  With maps carried, survivors and products also get their sides
+// (RefineSides): looking them up again in hash tables and counting the
+// elements around the edges anew cost 2.6 of 6.9 ms of the kernel time of
+// refining 384,000 tets to 1.76 million.
 __global__ __launch_bounds__(BLOCK) void refine_products(RefineArgs a) {
-  u32 t = xcd_block() * BLOCK + threadIdx.x;
-  if (t >= a.seg[4]) return;
-  u32 pd = a.pd;
-  if (t < a.seg[0]) {
+  u32 pd = 0;
+  while (pd < a.dim && blockIdx.x >= a.p[pd + 1].block0) ++pd;
+  RefineArgs::Prod const& P = a.p[pd];
+  u32 const t = (blockIdx.x - P.block0) * BLOCK + threadIdx.x;
+  if (t >= P.seg[3]) return;
+  RefineSides const S{a};
+  if (t < P.seg[0]) {
     u32 i = t, o;
     if (pd == 0) {
       o = i;
     } else {
       u32 const* of = a.off[pd];
+      o = i - of[i];
+      if (P.soff) {
+        P.soff[i] = o;
+        if (i + 1 == P.seg[0]) P.soff[i + 1] = i + 1 - of[i + 1];
+      }
       if (of[i] != of[i + 1]) return;
-      o = a.soff[i];
-      for (u32 k = 0; k <= pd; ++k) a.out_verts[(size_t) o * (pd + 1) + k] = a.verts_of[pd][(size_t) i * (pd + 1) + k];
+      for (u32 k = 0; k <= pd; ++k) P.out_verts[(size_t) o * (pd + 1) + k] = a.verts_of[pd][(size_t) i * (pd + 1) + k];
+      if (P.out_edges) {
+        u32 const ne = pd == 3 ? 6u : 3u;
+        for (u32 k = 0; k < ne; ++k)
+          P.out_edges[(size_t) o * ne + k] = S.survivor(1, a.edges_of[pd][(size_t) i * ne + k]);
+      }
+      if (P.out_faces)
+        for (u32 k = 0; k < 4; ++k) P.out_faces[4 * (size_t) o + k] = S.survivor(2, a.faces_of[4 * (size_t) i + k]);
     }
-    if (a.out_cd) a.out_cd[o] = a.cd[pd][i];
-    if (a.out_ci) a.out_ci[o] = a.ci[pd][i];
+    if (P.out_cd) P.out_cd[o] = a.cd[pd][i];
+    if (P.out_ci) P.out_ci[o] = a.ci[pd][i];
     return;
   }
   u32 d = 1;
-  while (t >= a.seg[d]) ++d;
-  u32 i = t - a.seg[d - 1];
+  while (t >= P.seg[d]) ++d;
+  u32 i = t - P.seg[d - 1];
   u32 const* of = a.off[d];
   u32 k0 = of[i];
   if (k0 == of[i + 1]) return;
-  u32 ppd = a.ppd[d];
-  u32 o = a.go[d] + k0 * ppd;
+  u32 ppd = P.ppd[d];
+  u32 o = P.go[d] + k0 * ppd;
   if (pd > 0) {
     // the domain's first split edge: its local index and new vertex
     u32 dir = 0, edge = i;
@@ -659,14 +775,23 @@ __global__ __launch_bounds__(BLOCK) void refine_products(RefineArgs a) {
     u32 const* vd = a.verts_of[d] + (size_t) i * (d + 1);
     for (u32 j = 0; j < ppd; ++j) {
       u32 const* bv = canon(d, pd - 1, 0, bo[os[j]]);
-      u32* q = a.out_verts + (size_t) (o + j) * (pd + 1);
+      u32* q = P.out_verts + (size_t) (o + j) * (pd + 1);
       for (u32 k = 0; k < pd; ++k) q[k] = vd[bv[k]];
       q[pd] = vert;
+      if (P.out_edges) {
+        u32* e = P.out_edges + (size_t) (o + j) * (pd == 3 ? 6 : 3);
+        if (pd == 3)
+          S.tet(i, dir, j, vd, e, P.out_faces + 4 * (size_t) (o + j));
+        else if (d == 3)
+          S.tet_inner(i, dir, e);
+        else
+          S.tri(i, dir, j, vd, e);
+      }
     }
   }
   for (u32 j = 0; j < ppd; ++j) {
-    if (a.out_cd) a.out_cd[o + j] = a.cd[d][i];
-    if (a.out_ci) a.out_ci[o + j] = a.ci[d][i];
+    if (P.out_cd) P.out_cd[o + j] = a.cd[d][i];
+    if (P.out_ci) P.out_ci[o + j] = a.ci[d][i];
   }
 }
 
@@ -688,70 +813,95 @@ static void refine_dom_offsets(Mesh& m, u32 const* gen_off, Buf<u32>* off) {
   }
 }
 
-// nsplit[d]: splitting domains of dimension d (from the offsets' totals)
-static void refine_ents(Mesh& m, Mesh& mo, u32 const* gen_off, Buf<u32>* off, u32 const* nsplit) {
+// nsplit[d]: splitting domains of dimension d (from the offsets' totals);
+// carry: the new mesh gets the maps the next split pass reads
+static void refine_ents(Mesh& m, Mesh& mo, u32 const* gen_off, Buf<u32>* off, u32 const* nsplit, bool carry) {
   OHX_REQUIRE(m.full, "refine needs a full-topology mesh");
   u32 dim = m.dim;
-  RefineArgs base{};
-  base.dim = dim;
-  base.nv = count(m, 0);
-  base.off[1] = gen_off;  // an edge splits iff it is in the independent set
+  RefineArgs a{};
+  a.dim = dim;
+  a.nv = count(m, 0);
+  a.off[1] = gen_off;  // an edge splits iff it is in the independent set
   for (u32 d = 0; d <= dim; ++d) {
-    base.n[d] = count(m, d);
-    base.verts_of[d] = d ? ask_down(m, d, 0) : nullptr;
+    a.n[d] = count(m, d);
+    a.verts_of[d] = d ? ask_down(m, d, 0) : nullptr;
   }
   for (u32 d = 2; d <= dim; ++d) {
-    base.edges_of[d] = ask_down(m, d, 1);
-    base.off[d] = off[d].get();
+    a.edges_of[d] = ask_down(m, d, 1);
+    a.off[d] = off[d].get();
   }
+  if (carry && dim == 3) a.faces_of = ask_down(m, 3, 2);
   bool has_class = find_tag(m, 0, "class_dim") != nullptr;
   bool has_id = find_tag(m, 0, "class_id") != nullptr;
   if (has_class)
     for (u32 d = 0; d <= dim; ++d) {
-      base.cd[d] = u32_tag(m, d, "class_dim");
-      base.ci[d] = has_id ? u32_tag(m, d, "class_id") : nullptr;
+      a.cd[d] = u32_tag(m, d, "class_dim");
+      a.ci[d] = has_id ? u32_tag(m, d, "class_id") : nullptr;
     }
+  bool const transfers = has_element_transfer(m);
+  Buf<u32> verts[4], cdo[4], cio[4], edges[4], faces, soff[4];
+  u32 total[4], nsame[4], blocks = 0;
   for (u32 pd = 0; pd <= dim; ++pd) {
-    RefineArgs a = base;
-    a.pd = pd;
-    u32 nsurv = base.n[pd] - (pd ? nsplit[pd] : 0);
-    Buf<u32> soff;
-    if (pd) soff = negate_offsets(base.off[pd], base.n[pd]);
-    a.soff = soff.get();
-    u32 total = nsurv;
-    a.seg[0] = base.n[pd];
+    RefineArgs::Prod& P = a.p[pd];
+    nsame[pd] = a.n[pd] - (pd ? nsplit[pd] : 0);
+    total[pd] = nsame[pd];
+    P.block0 = blocks;
+    P.seg[0] = a.n[pd];
     for (u32 d = 1; d <= 3; ++d) {
       bool live = d <= dim && d >= (pd > 1 ? pd : 1);
-      a.ppd[d] = live ? prods_per_dom(d, 1, pd) : 0;
-      a.go[d] = total;
-      total += a.ppd[d] * nsplit[d];
-      a.seg[d] = a.seg[d - 1] + ((live && a.ppd[d]) ? base.n[d] : 0);
+      P.ppd[d] = live ? prods_per_dom(d, 1, pd) : 0;
+      P.go[d] = total[pd];
+      total[pd] += P.ppd[d] * nsplit[d];
+      P.seg[d] = P.seg[d - 1] + ((live && P.ppd[d]) ? a.n[d] : 0);
     }
-    a.seg[4] = a.seg[3];
-    Buf<u32> verts, cdo, cio;
+    blocks += nblocks(P.seg[3]);
     if (pd) {
-      verts = Buf<u32>((size_t) total * (pd + 1));
-      a.out_verts = verts.get();
+      verts[pd] = Buf<u32>((size_t) total[pd] * (pd + 1));
+      P.out_verts = verts[pd].get();
     }
     if (has_class) {
-      cdo = Buf<u32>(total);
-      a.out_cd = cdo.get();
+      cdo[pd] = Buf<u32>(total[pd]);
+      P.out_cd = cdo[pd].get();
       if (has_id) {
-        cio = Buf<u32>(total);
-        a.out_ci = cio.get();
+        cio[pd] = Buf<u32>(total[pd]);
+        P.out_ci = cio[pd].get();
       }
     }
-    if (a.seg[4]) {
-      hipLaunchKernelGGL(refine_products, dim3(nblocks(a.seg[4])), dim3(BLOCK), 0, stream(), a);
-      check_launch("refine_products");
+    if (carry && pd >= 2) {
+      edges[pd] = Buf<u32>((size_t) total[pd] * (pd == 3 ? 6 : 3));
+      P.out_edges = edges[pd].get();
     }
-    if (pd) set_ents(mo, pd, total, std::move(verts));
-    if (has_class) {
-      add_tag_u32(mo, pd, "class_dim", 1, std::move(cdo));
-      if (has_id) add_tag_u32(mo, pd, "class_id", 1, std::move(cio));
+    if (carry && pd == 3) {
+      faces = Buf<u32>((size_t) total[pd] * 4);
+      P.out_faces = faces.get();
     }
-    if (pd == dim) refine_transfer(m, mo, soff.get(), base.off[dim], a.ppd[dim], a.go[dim], total);
+    if ((carry && pd == 1) || (pd == dim && (carry || transfers))) {
+      soff[pd] = Buf<u32>((size_t) a.n[pd] + 1);
+      P.soff = soff[pd].get();
+    }
   }
+  for (u32 pd = dim + 1; pd < 4; ++pd) a.p[pd].block0 = blocks;
+  if (blocks) {
+    hipLaunchKernelGGL(refine_products, dim3(blocks), dim3(BLOCK), 0, stream(), a);
+    check_launch("refine_products");
+  }
+  for (u32 pd = 0; pd <= dim; ++pd) {
+    if (pd) set_ents(mo, pd, total[pd], std::move(verts[pd]));
+    if (has_class) {
+      add_tag_u32(mo, pd, "class_dim", 1, std::move(cdo[pd]));
+      if (has_id) add_tag_u32(mo, pd, "class_id", 1, std::move(cio[pd]));
+    }
+  }
+  if (transfers)
+    refine_transfer(m, mo, soff[dim].get(), a.off[dim], a.p[dim].ppd[dim], a.p[dim].go[dim], total[dim]);
+  if (!carry) return;
+  // the elements around the edges from the old ones: survivors of both
+  // dimensions come first and the products are numbered after them
+  mo.up[1][dim] = up_patch(h_down_deg[dim][1], ask_up(m, 1, dim), a.n[1], soff[1].get(), nsame[1],
+                           total[1] - nsame[1], soff[dim].get(), nsame[dim], total[dim] - nsame[dim],
+                           edges[dim].get());
+  for (u32 d = 2; d <= dim; ++d) mo.down[d][1] = std::move(edges[d]);
+  if (dim == 3) mo.down[3][2] = std::move(faces);
 }
 
 static void say(char const* verb, u32 n, u32 d) {
@@ -775,7 +925,7 @@ static void check_index_space(Mesh& m) {
 }
 
 static u32 refine_common(Mesh& m, Buf<u32>& cand, double qual_floor, bool require_better,
-                         double const* qfe = nullptr) {
+                         double const* qfe = nullptr, bool carry = false) {
   check_index_space(m);
   u32 ns = count(m, 1), dim = m.dim;
   Buf<double> q = refine_qualities(m, cand.get(), qual_floor, require_better, qfe);
@@ -810,13 +960,15 @@ static u32 refine_common(Mesh& m, Buf<u32>& cand, double qual_floor, bool requir
   u32 nsplit[4] = {0, total, got[2], got[3]};
   Mesh mo(m.dim, m.full);
   refine_verts(m, mo, gen_off.get(), total);
-  refine_ents(m, mo, gen_off.get(), off, nsplit);
+  // maps are carried through mesh_adapt's loop of split passes, and where the
+  // mesh has the map that only the carrying reads
+  refine_ents(m, mo, gen_off.get(), off, nsplit, carry || (dim == 3 && m.down[3][2]));
   say("split", total, 1);
   overwrite(m, std::move(mo));
   return 1;
 }
 
-u32 refine_by_size(Mesh& m, double qual_floor) {
+u32 refine_by_size(Mesh& m, double qual_floor, bool carry) {
   u32 ne = count(m, 1);
   double const* h = size_of(m);
   double const* mt = metric_of(m);
@@ -833,7 +985,7 @@ u32 refine_by_size(Mesh& m, double qual_floor) {
     Buf<double> qfe = batch_floors(m, 1);
     return refine_common(m, cand, qual_floor, false, qfe.get());
   }
-  return refine_common(m, cand, qual_floor, false);
+  return refine_common(m, cand, qual_floor, false, nullptr, carry);
 }
 
 void uniformly_refine(Mesh& m) {
@@ -1586,7 +1738,7 @@ struct UpPatchCounts {
 // new down(h,l) (its product rows are read)
 static std::unique_ptr<Up> up_patch(u32 deg, Up const& old, u32 nl_old, u32 const* soff_l, u32 nsame_l,
                                     u32 ngen_l, u32 const* soff_h, u32 nsame_h, u32 ngen_h, u32 const* dn,
-                                    UpPatchCounts* keep = nullptr) {
+                                    UpPatchCounts* keep) {
   u32 const nl = nsame_l + ngen_l, nuse = (nsame_h + ngen_h) * deg, nprod = ngen_h * deg;
   auto up = std::make_unique<Up>();
   up->offsets = Buf<u32>(nl + 1);
@@ -3792,16 +3944,6 @@ struct RunCavity {
   // in the tet
   u32 ring[8], tet[8], redge[8], spoke[2][8], loc[8];
 };
-// local vertices of a tet's edge d, the edge opposite, the face opposite a
-// local vertex (k_r_e_v, k_o_r_e, k_r_f_v), a digit each
-__device__ inline u32 tet_ev0(u32 d) { return (0x210210u >> (4 * d)) & 3u; }
-__device__ inline u32 tet_ev1(u32 d) { return (0x333021u >> (4 * d)) & 3u; }
-__device__ inline u32 tet_oe(u32 d) { return (0x021435u >> (4 * d)) & 7u; }
-__device__ inline u32 tet_face_without(u32 v) { return (0x0132u >> (4 * v)) & 3u; }
-__device__ inline u32 tet_edge_of(u32 a, u32 b) {
-  return a == 3 ? 3 + b : b == 3 ? 3 + a : a + b == 1 ? 0u : a + b == 3 ? 1u : 2u;
-}
-
 __global__ __launch_bounds__(BLOCK) void run_products_k(SwapRunView R, u32 ns, u32* __restrict__ face_prod,
                                                         u32* __restrict__ deferred, u32* __restrict__ err) {
   __shared__ RunCavity cavities[BLOCK / RUN_G];
@@ -4735,7 +4877,7 @@ u32 run_pass(Mesh& m, Ctx& c, Kind k, double a, double b, u32 n, double const* e
   if (k != SWAP) c.swap_cache.clear();
   if (k != COARSEN) c.size_codes.clear();
   switch (k) {
-    case REFINE: ok = refine_by_size(m, a); break;
+    case REFINE: ok = refine_by_size(m, a, true); break;
     case COARSEN: ok = coarsen_by_size(m, a, b, &c.size_codes); break;
     case SWAP: ok = swap_slivers(m, a, n, eq, gate, &c.swap_cache); break;
     case COARSEN_SLIVERS: ok = coarsen_slivers(m, a, n, eq); break;
@@ -4755,9 +4897,7 @@ bool swap_run_fits(Mesh& m) {
       bool const wanted = name[6] == 'd' || has_id;
       if (wanted && !(t && t->type == TagType::U32 && t->ncomps == 1)) return false;
     }
-  for (auto& t : m.tags[3])
-    if (t->transfer == 1 || t->transfer == 2) return false;  // OSH_TRANSFER_POINTWISE, _CONSERVE
-  return true;
+  return !has_element_transfer(m);
 }
 
 // swap passes until one changes nothing; eq: the element qualities of m,

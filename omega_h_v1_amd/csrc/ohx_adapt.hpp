@@ -9,7 +9,8 @@ namespace ohx {
 
 Buf<u32> find_indset(Mesh& m, u32 ent_dim, u32 const* filter, double const* goodness);
 
-u32 refine_by_size(Mesh& m, double qual_floor);
+// carry: the new mesh also gets the maps the next split pass reads
+u32 refine_by_size(Mesh& m, double qual_floor, bool carry = false);
 void uniformly_refine(Mesh& m);
 // The size codes of the collapse-by-size loop, per edge of the current
 // mesh: a surviving edge keeps its vertices, their coordinates and the
