@@ -329,6 +329,13 @@ static Buf<u32> find_indset_bounded(Mesh& m, u32 ent_dim, u32 const* filter, dou
                                     u32 const** last_flag) {
   return indset_rounds(m, ent_dim, filter, good, first_batch_rounds(), last_flag);
 }
+// the same from states that are set up already (UNKNOWN or NOT_IN_SET, the
+// round flags cleared): the kernels that decide the candidates write them
+static Buf<u32> find_indset_from(Mesh& m, u32 ent_dim, Buf<u32>&& state, double const* good,
+                                 u32 const** last_flag) {
+  return indset_rounds(m, ent_dim, nullptr, good, first_batch_rounds(), last_flag, &state);
+}
+constexpr u32 INDSET_FLAGS = 8;
 // the checked loop from the first batch's state
 static Buf<u32> find_indset_resume(Mesh& m, u32 ent_dim, double const* good, Buf<u32>&& state) {
   return indset_rounds(m, ent_dim, nullptr, good, 0, nullptr, &state, first_batch_rounds());
@@ -346,7 +353,9 @@ static std::unique_ptr<Up> up_patch(u32 deg, Up const& old, u32 nl_old, u32 cons
 
 // --------------------------------------------------------------- refine
 // Worst child quality of every candidate edge split
-// (refine_qualities.cpp:16-82); rejected candidates are cleared.
+// (refine_qualities.cpp:16-82); rejected candidates are cleared, the others
+// become UNKNOWN: cand is then the independent set's first state, and the
+// flags of its rounds are cleared on the way.
 template <u32 DIM, bool MIXED>
 __global__ __launch_bounds__(BLOCK) void refine_quality_f64(
     u32 ns, u32 const* __restrict__ vs, u32 const* __restrict__ uo, u32 const* __restrict__ ua,
@@ -355,6 +364,7 @@ __global__ __launch_bounds__(BLOCK) void refine_quality_f64(
     double const* __restrict__ qfe, u32* __restrict__ cand, double* __restrict__ out, u32* __restrict__ words, u32 tag,
     u32* __restrict__ err, ScreenStats st) {
   u32 i = xcd_block() * BLOCK + threadIdx.x;
+  if (i < INDSET_FLAGS) words[W_FLAGS + i] = 0;
   if (i >= ns || !cand[i]) return;
   // one floor for the mesh, or its component's in a batch
   double const qual_floor = qfe ? qfe[i] : qual_floor_all;
@@ -450,6 +460,7 @@ __global__ __launch_bounds__(BLOCK) void refine_quality_f64(
     cand[i] = 0;
   else {
     out[i] = minq;
+    cand[i] = UNKNOWN;
     wave_flag_value(words + W_ANY, true, tag);
   }
 }
@@ -795,24 +806,6 @@ __global__ __launch_bounds__(BLOCK) void refine_products(RefineArgs a) {
   }
 }
 
-// offsets of the splitting domains of each dimension d >= 2 (a domain
-// splits iff one of its edges does), enqueued without reading their totals
-static void refine_dom_offsets(Mesh& m, u32 const* gen_off, Buf<u32>* off) {
-  for (u32 d = 2; d <= m.dim; ++d) {
-    u32 n = count(m, d);
-    u32 const* ed = ask_down(m, d, 1);
-    u32 spd = h_down_deg[d][1];
-    off[d] = Buf<u32>(n + 1);
-    exscan_fn_heavy(n, OHX_LAMBDA(u32 i) {
-      for (u32 j = 0; j < spd; ++j) {
-        u32 e = ed[(size_t) i * spd + j];
-        if (gen_off[e] != gen_off[e + 1]) return 1u;
-      }
-      return 0u;
-    }, off[d].get());
-  }
-}
-
 // nsplit[d]: splitting domains of dimension d (from the offsets' totals);
 // carry: the new mesh gets the maps the next split pass reads
 static void refine_ents(Mesh& m, Mesh& mo, u32 const* gen_off, Buf<u32>* off, u32 const* nsplit, bool carry) {
@@ -934,30 +927,55 @@ static u32 refine_common(Mesh& m, Buf<u32>& cand, double qual_floor, bool requir
   // convergence flag and the totals (a candidate-free call ends with an
   // empty set and returns 0)
   u32 const* flag = nullptr;
-  Buf<u32> indset = find_indset_bounded(m, 1, cand.get(), q.get(), &flag);
+  Buf<u32> indset = find_indset_from(m, 1, std::move(cand), q.get(), &flag);
   Buf<u32> gen_off(ns + 1);
-  Buf<u32> off[4];
-  u32 got[4];
+  Buf<u32> off[4], splits[4];
+  u32 got[3] = {0, 0, 0}, open = 0;
   auto offsets_and_totals = [&] {
-    exscan(indset.get(), ns, gen_off.get());
-    refine_dom_offsets(m, gen_off.get(), off);
-    u32 const* ptrs[4] = {flag, gen_off.get() + ns, dim >= 2 ? off[2].get() + count(m, 2) : nullptr,
-                          dim >= 3 ? off[3].get() + count(m, 3) : nullptr};
-    read_many(ptrs, 4, got);
+    // a face or tet splits iff one of its edges does: both dimensions'
+    // flags in one launch, then every scan in one
+    scan_detail::ScanJobs J{};
+    scan_job(J, ns, indset.get(), IN_SET, gen_off.get());
+    u32 n[4] = {0, 0, 0, 0};
+    u32 const* ed[4] = {nullptr, nullptr, nullptr, nullptr};
+    for (u32 d = 2; d <= dim; ++d) {
+      n[d] = count(m, d);
+      ed[d] = ask_down(m, d, 1);
+      off[d] = Buf<u32>(n[d] + 1);
+      splits[d] = Buf<u32>(n[d]);
+      scan_job(J, n[d], splits[d].get(), 1, off[d].get());
+    }
+    u32 const* is = indset.get();
+    u32 const n2 = n[2], n3 = n[3];
+    u32 const *e2 = ed[2], *e3 = ed[3];
+    u32 *s2 = splits[2].get(), *s3 = splits[3].get();
+    parallel_for(n2 > n3 ? n2 : n3, OHX_LAMBDA(u32 i) {
+      if (i < n2) {
+        u32 const* e = e2 + 3 * (size_t) i;
+        s2[i] = is[e[0]] == IN_SET || is[e[1]] == IN_SET || is[e[2]] == IN_SET ? 1u : 0u;
+      }
+      if (i < n3) {
+        u32 const* e = e3 + 6 * (size_t) i;
+        u32 any = 0;
+#pragma unroll
+        for (u32 j = 0; j < 6; ++j) any |= is[e[j]] == IN_SET ? 1u : 0u;
+        s3[i] = any;
+      }
+    });
+    exscan_jobs(J, flag, got, &open);
   };
   offsets_and_totals();
-  if (got[0]) {  // not settled in the first batch: the checked loop from there
+  if (open) {  // not settled in the first batch: the checked loop from there
     indset = find_indset_resume(m, 1, q.get(), std::move(indset));
     flag = nullptr;
     offsets_and_totals();
   }
   if (g_batch) batch_note_changed(m, 1, indset.get());
-  cand.release();
   q.release();
   indset.release();
-  u32 total = got[1];
+  u32 total = got[0];
   if (!total) return 0;
-  u32 nsplit[4] = {0, total, got[2], got[3]};
+  u32 nsplit[4] = {0, total, got[1], got[2]};
   Mesh mo(m.dim, m.full);
   refine_verts(m, mo, gen_off.get(), total);
   // maps are carried through mesh_adapt's loop of split passes, and where the
@@ -1284,13 +1302,16 @@ __global__ __launch_bounds__(BLOCK) void coarsen_quality_f64(CqArgs A) {
 
 // collapse_to_vert (collapses_to_verts.cpp:13-42): whether each vertex
 // collapses and the best goodness of its collapse directions; inex (when
-// given) says whether that goodness is an FP32 value
+// given) says whether that goodness is an FP32 value.  cand is the
+// independent set's first state, and the flags of its rounds are cleared.
 __global__ __launch_bounds__(BLOCK) void collapse_to_vert_k(u32 nv, u32 const* __restrict__ uo,
                                                             u32 const* __restrict__ ua, u32 const* __restrict__ ud,
                                                             u32 const* __restrict__ cd, double const* __restrict__ q,
                                                             u32 const* __restrict__ vo, u32* __restrict__ cand,
-                                                            double* __restrict__ vq, u32* __restrict__ inex) {
+                                                            double* __restrict__ vq, u32* __restrict__ inex,
+                                                            u32* __restrict__ flags) {
   u32 i = xcd_block() * BLOCK + threadIdx.x;
+  if (i < INDSET_FLAGS) flags[i] = 0;
   if (i >= nv) return;
   double maxq = 0;
   u32 is = 0, mi = 0;
@@ -1311,7 +1332,7 @@ __global__ __launch_bounds__(BLOCK) void collapse_to_vert_k(u32 nv, u32 const* _
       mi = (c & inexact_bit(d)) ? 1u : 0u;
     }
   }
-  cand[i] = is;
+  cand[i] = is ? (u32) UNKNOWN : (u32) NOT_IN_SET;
   vq[i] = is ? maxq : 0.0;
   if (inex) inex[i] = mi;
 }
@@ -1433,10 +1454,8 @@ __global__ __launch_bounds__(BLOCK) void carry_size_codes_k(CarryCodes a) {
   }
 }
 
-// tags_subset (subset.cpp:15-43): every tag of the surviving vertices,
-// one thread per old vertex, all tags in one launch
-__global__ __launch_bounds__(BLOCK) void subset_tags(u32 n, u32 const* __restrict__ soff, TagList L) {
-  u32 i = xcd_block() * BLOCK + threadIdx.x;
+// tags_subset (subset.cpp:15-43): every tag of old vertex i if it survives
+__device__ inline void subset_tags(u32 i, u32 n, u32 const* __restrict__ soff, TagList const& L) {
   if (i >= n) return;
   u32 o = soff[i];
   if (o == soff[i + 1]) return;
@@ -1526,8 +1545,24 @@ __device__ inline u32 coarsen_product_side(u32 d, u32 c, u32 gd, u32 const* row,
 // setup_coarsen class inheritance (inherit.cpp:140-156), fused: survivors
 // first, then the entities rebuilt on the collapse target (the base
 // opposite the collapsing vertex, then the target), vertex ids renumbered.
-__global__ __launch_bounds__(BLOCK) void coarsen_outputs(CoarsenArgs a) {
-  u32 i = xcd_block() * BLOCK + threadIdx.x;
+// Every dimension and the vertices' tags in one launch, a range of blocks
+// each: the elements first, which take longest.
+struct CoarsenOutputs {
+  CoarsenArgs a[3];
+  u32 block0[4];  // first blocks of a[0..2] and of the vertices
+  u32 nv;
+  u32 const* soff;
+  TagList tags;
+};
+__global__ __launch_bounds__(BLOCK) void coarsen_outputs(CoarsenOutputs O) {
+  if (blockIdx.x >= O.block0[3]) {
+    subset_tags((blockIdx.x - O.block0[3]) * BLOCK + threadIdx.x, O.nv, O.soff, O.tags);
+    return;
+  }
+  u32 part = 0;
+  while (part < 2 && blockIdx.x >= O.block0[part + 1]) ++part;
+  CoarsenArgs const& a = O.a[part];
+  u32 i = (blockIdx.x - O.block0[part]) * BLOCK + threadIdx.x;
   if (i >= a.n) return;
   u32 d = a.d, vpe = d + 1;
   u32 const* v = a.vent + (size_t) i * vpe;
@@ -1935,7 +1970,7 @@ static u32 coarsen_common(Mesh& m, Buf<u32>& codes, double qual_floor, bool requ
         if (!nv) return;
         hipLaunchKernelGGL(collapse_to_vert_k, dim3(nblocks(nv)), dim3(BLOCK), 0, stream(), nv, uv.offsets.get(),
                            uv.adj.get(), uv.dirs.get(), codes.get(), cq.get(), voff.get(), cand.get(), vq.get(),
-                           certified ? vinex.get() : nullptr);
+                           certified ? vinex.get() : nullptr, scratch_words() + W_FLAGS);
         check_launch("collapse_to_vert");
       };
       to_vert();
@@ -1972,25 +2007,27 @@ static u32 coarsen_common(Mesh& m, Buf<u32>& codes, double qual_floor, bool requ
   // a first batch of indset rounds, the collapse destinations and the
   // vertex offsets, then one read of the convergence flag and the total
   u32 const* flag = nullptr;
-  Buf<u32> indset = find_indset_bounded(m, 0, cand.get(), vq.get(), &flag);
+  Buf<u32> indset = find_indset_from(m, 0, std::move(cand), vq.get(), &flag);
   Buf<u32> gvv(nv);
-  Buf<u32> goff(nv + 1);
   // coarsen_all_ents (coarsen_common.cpp:91-107), top dimension first.
   // Phase 1 decides every dimension's survivors and products on the device
   // (a dimension's fused sides feed the next lower one, no host decision
-  // needed), right after the destinations; one read then brings the set's
-  // convergence flag, the collapse count and all the totals; phase 2
-  // writes the outputs.
+  // needed), right after the destinations; one launch scans them all and one
+  // read then brings the set's convergence flag, the collapse count and all
+  // the totals; phase 2 writes the outputs.
   bool has_class = find_tag(m, 0, "class_dim") != nullptr;
   bool has_id = find_tag(m, 0, "class_id") != nullptr;
-  Buf<u32> fused[4], fused_to[4];
+  bool const transfers = has_element_transfer(m);
+  Buf<u32> fused_to[4], goff, soff(nv + 1);
   struct DimPlan {
-    Buf<u32> gv, gd, egoff, esoff;
+    Buf<u32> gv, gd, egoff, esoff, fate;
   };
   DimPlan plan[4];
-  u32 got[10];
+  u32 got[scan_detail::MAX_JOBS], open = 0;
+  enum Fate : u32 { REMOVED = 0, SAME = 1, REBUILT = 2 };
   auto dest_and_total = [&] {
-    // vertex_dest (collapses_to_verts.cpp:72-135)
+    // vertex_dest (collapses_to_verts.cpp:72-135); the sides' fusions are
+    // cleared on the way
     u32 const* uo = uv.offsets.get();
     u32 const* ua = uv.adj.get();
     u32 const* ud = uv.dirs.get();
@@ -2001,7 +2038,14 @@ static u32 coarsen_common(Mesh& m, Buf<u32>& codes, double qual_floor, bool requ
     u32* g = gvv.get();
     u32* err = dev_error_word();
     u32 const* fl = flag;
-    parallel_for(nv, OHX_LAMBDA(u32 i) {
+    u32 const nf1 = dim >= 2 ? count(m, 1) : 0, nf2 = dim == 3 ? count(m, 2) : 0;
+    for (u32 d = 1; d < dim; ++d) fused_to[d] = Buf<u32>(count(m, d));
+    u32 *ft1 = fused_to[1].get(), *ft2 = fused_to[2].get();
+    u32 const nmost = nf2 > nf1 ? nf2 : nf1;
+    parallel_for(nmost > nv ? nmost : nv, OHX_LAMBDA(u32 i) {
+      if (i < nf1) ft1[i] = INVALID;
+      if (i < nf2) ft2[i] = INVALID;
+      if (i >= nv) return;
       if (!is[i] || (fl && *fl)) {  // not in the set, or the set is not settled yet
         g[i] = INVALID;
         return;
@@ -2023,120 +2067,104 @@ static u32 coarsen_common(Mesh& m, Buf<u32>& codes, double qual_floor, bool requ
       g[i] = gv;
     });
     // coarsen_interior (coarsen_common.cpp:191-219)
-    exscan(indset.get(), nv, goff.get());
+    scan_detail::ScanJobs J{};
+    scan_job(J, nv, is, NOT_IN_SET, soff.get());
     for (u32 dd = 0; dd < dim; ++dd) {
       u32 d = dim - dd;
       u32 n = count(m, d);
       u32 const* vent = ask_down(m, d, 0);
       u32 const* sent = ask_down(m, d, d - 1);
-      u32 nsd = count(m, d - 1);
-      fused[d - 1] = filled(nsd, 0);
-      if (d >= 2) fused_to[d - 1] = Buf<u32>(nsd);
       u32 vpe = d + 1, spe = h_down_deg[d][d - 1];
-      Buf<u32> will(n), gv(n), gd(n), same(n);
+      DimPlan& pl = plan[d];
+      pl.gv = Buf<u32>(n);
+      pl.gd = Buf<u32>(n);
+      pl.fate = Buf<u32>(n);
+      pl.egoff = Buf<u32>(n + 1);
+      pl.esoff = Buf<u32>(n + 1);
       {
         // collapse_to_ent (collapses_to_ents.cpp:11-82); also marks the
         // entities with no collapsing vertex, which survive unchanged, and
         // notes for each fused side the side it merges into (the one
         // opposite the collapsing vertex), which the maps carried to the
         // new mesh read
-        u32 const* go = goff.get();
-        u32 const* g = gvv.get();
-        u32 const* fe = fused[d] ? fused[d].get() : nullptr;
-        u32* fs = fused[d - 1].get();
+        u32 const* fe = fused_to[d].get();  // null for elements
         u32* ft = d >= 2 ? fused_to[d - 1].get() : nullptr;
-        u32* wl = will.get();
-        u32* gvp = gv.get();
-        u32* gdp = gd.get();
-        u32* smp = same.get();
+        u32* wl = pl.fate.get();
+        u32* gvp = pl.gv.get();
+        u32* gdp = pl.gd.get();
         parallel_for(n, OHX_LAMBDA(u32 i) {
           u32 const* v = vent + (size_t) i * vpe;
           u32 col = INVALID, dir = INVALID;
           for (u32 j = 0; j < vpe; ++j)
-            if (go[v[j]] != go[v[j] + 1]) {
+            if (is[v[j]]) {
               col = v[j];
               dir = j;
             }
-          u32 w = 0, gvv_ = 0, gd_ = 0;
+          u32 w = SAME;
           if (dir != INVALID) {
+            w = REMOVED;
             u32 target = g[col];
             u32 gdir = INVALID;
             for (u32 j = 0; j < vpe; ++j)
               if (v[j] == target) gdir = j;
             if (gdir != INVALID) {
-              u32 const side = sent[(size_t) i * spe + opp(d, 0)[gdir]];
-              fs[side] = 1;
-              if (ft) ft[side] = sent[(size_t) i * spe + opp(d, 0)[dir]];
-            } else if (!(fe && fe[i])) {
-              w = 1;
-              gvv_ = target;
-              gd_ = dir;
+              if (ft) ft[sent[(size_t) i * spe + opp(d, 0)[gdir]]] = sent[(size_t) i * spe + opp(d, 0)[dir]];
+            } else if (!(fe && fe[i] != INVALID)) {
+              w = REBUILT;
+              gvp[i] = target;
+              gdp[i] = dir;
             }
           }
           wl[i] = w;
-          gvp[i] = gvv_;
-          gdp[i] = gd_;
-          smp[i] = dir == INVALID ? 1u : 0u;
         });
       }
-      Buf<u32> egoff(n + 1), esoff(n + 1);
-      {
-        u32 const* wl = will.get();
-        u32 const* smp = same.get();
-        exscan_fn(n, OHX_LAMBDA(u32 i) { return wl[i]; }, egoff.get());
-        exscan_fn(n, OHX_LAMBDA(u32 i) { return smp[i]; }, esoff.get());
-      }
-      same.release();
-      plan[d] = DimPlan{std::move(gv), std::move(gd), std::move(egoff), std::move(esoff)};
     }
-    u32 const* ptrs[10];
-    u32 k = 0;
-    ptrs[k++] = flag;
-    ptrs[k++] = goff.get() + nv;
     for (u32 d = 1; d <= dim; ++d) {
-      u32 n = count(m, d);
-      ptrs[k++] = plan[d].egoff.get() + n;
-      ptrs[k++] = plan[d].esoff.get() + n;
+      u32 const n = count(m, d);
+      scan_job(J, n, plan[d].fate.get(), REBUILT, plan[d].egoff.get());
+      scan_job(J, n, plan[d].fate.get(), SAME, plan[d].esoff.get());
     }
-    read_many(ptrs, k, got);
+    if (transfers) {  // the only reader of the collapsing vertices' own numbering
+      goff = Buf<u32>(nv + 1);
+      scan_job(J, nv, is, IN_SET, goff.get());
+    }
+    exscan_jobs(J, flag, got, &open);
   };
+  // got: surviving vertices, then per dimension the rebuilt and the same
   dest_and_total();
-  if (got[0]) {  // not settled in the first batch: the checked loop from there
+  if (open) {  // not settled in the first batch: the checked loop from there
     indset = find_indset_resume(m, 0, vq.get(), std::move(indset));
     flag = nullptr;
     dest_and_total();
   }
   if (g_batch) batch_note_changed(m, 0, indset.get());
-  cand.release();
   if (!sizes) {
     codes.release();
     cq.release();
   }
   vq.release();
-  u32 total = got[1];
+  u32 const nv_out = got[0], total = nv - nv_out;
   if (!total) return 0;
   indset.release();
-  Buf<u32> soff = negate_offsets(goff.get(), nv);
-  u32 nv_out = nv - total;
+  auto const rebuilt = [&](u32 d) { return got[1 + 2 * (d - 1)]; };
+  auto const same = [&](u32 d) { return got[2 + 2 * (d - 1)]; };
   Mesh mo(dim, m.full);
   set_ents(mo, 0, nv_out, Buf<u32>());
-  {
-    // tags_subset (subset.cpp:15-43): every vertex tag, one launch
-    TagList L;
-    for (auto& tp : m.tags[0]) {
-      Tag& t = *tp;
-      void* dst;
-      if (t.type == TagType::F64)
-        dst = add_tag_f64(mo, 0, t.name.c_str(), t.ncomps, Buf<double>((size_t) nv_out * t.ncomps), t.transfer).f.get();
-      else
-        dst = add_tag_u32(mo, 0, t.name.c_str(), t.ncomps, Buf<u32>((size_t) nv_out * t.ncomps), t.transfer).u.get();
-      tag_list_add(L, t, dst);
-    }
-    if (L.n) {
-      hipLaunchKernelGGL(subset_tags, dim3(nblocks(nv)), dim3(BLOCK), 0, stream(), nv, soff.get(), L);
-      check_launch("subset_tags");
-    }
+  CoarsenOutputs out{};
+  out.nv = nv;
+  out.soff = soff.get();
+  // tags_subset (subset.cpp:15-43): every vertex tag
+  for (auto& tp : m.tags[0]) {
+    Tag& t = *tp;
+    void* dst;
+    if (t.type == TagType::F64)
+      dst = add_tag_f64(mo, 0, t.name.c_str(), t.ncomps, Buf<double>((size_t) nv_out * t.ncomps), t.transfer).f.get();
+    else
+      dst = add_tag_u32(mo, 0, t.name.c_str(), t.ncomps, Buf<u32>((size_t) nv_out * t.ncomps), t.transfer).u.get();
+    tag_list_add(out.tags, t, dst);
   }
+  double out_bytes = 0;
+  u32 blocks = 0;
   // the maps this pass read and the next collapse pass reads again,
   // carried to the new mesh instead of derived again: each entity's sides
   // (down(d, d-1)) here, the vertices' upward adjacencies below.  The tets'
@@ -2149,11 +2177,13 @@ static u32 coarsen_common(Mesh& m, Buf<u32>& codes, double qual_floor, bool requ
     u32 d = dim - dd;
     u32 n = count(m, d);
     u32 vpe = d + 1;
-    u32 ngen = got[2 + 2 * (d - 1)], nsame = got[2 + 2 * (d - 1) + 1];
+    u32 ngen = rebuilt(d), nsame = same(d);
     DimPlan& pl = plan[d];
     Buf<u32> vout((size_t) (nsame + ngen) * vpe);
     Buf<u32> cdo, cio;
-    CoarsenArgs a{};
+    CoarsenArgs& a = out.a[dd];
+    out.block0[dd] = blocks;
+    blocks += nblocks(n);
     auto carry_sides = [&](u32 l, CoarsenSides& cs) {
       u32 const ns = simplex_sides(d, l);
       side_maps[d][l] = Buf<u32>((size_t) (nsame + ngen) * ns);
@@ -2162,7 +2192,7 @@ static u32 coarsen_common(Mesh& m, Buf<u32>& codes, double qual_floor, bool requ
       cs.soff = plan[l].esoff.get();
       cs.egoff = plan[l].egoff.get();
       cs.fused_to = fused_to[l].get();
-      cs.nsame = got[2 + 2 * (l - 1) + 1];
+      cs.nsame = same(l);
       cs.l = l;
       cs.nold = m.counts[l];
       cs.err = dev_error_word();
@@ -2196,15 +2226,17 @@ static u32 coarsen_common(Mesh& m, Buf<u32>& codes, double qual_floor, bool requ
     // direction, class tags in and out, and the carried sides (old ids in,
     // new ids gathered and written)
     u32 const ns = (a.sides.out ? simplex_sides(d, d - 1) : 0u) + (a.edges.out ? 6u : 0u);
-    launch_timed("coarsen_outputs", (double) n * (vpe * 12 + 32 + ns * 12), coarsen_outputs, dim3(nblocks(n)),
-                 dim3(BLOCK), a);
+    out_bytes += (double) n * (vpe * 12 + 32 + ns * 12);
     set_ents(mo, d, nsame + ngen, std::move(vout));
     if (has_class) {
       add_tag_u32(mo, d, "class_dim", 1, std::move(cdo));
       if (has_id) add_tag_u32(mo, d, "class_id", 1, std::move(cio));
     }
-    if (d == dim) coarsen_transfer(m, mo, goff.get(), total, pl.egoff.get(), pl.esoff.get(), nsame, ngen);
   }
+  for (u32 k = dim; k < 4; ++k) out.block0[k] = blocks;
+  launch_timed("coarsen_outputs", out_bytes, coarsen_outputs, dim3(blocks + nblocks(nv)), dim3(BLOCK), out);
+  if (transfers)
+    coarsen_transfer(m, mo, goff.get(), total, plan[dim].egoff.get(), plan[dim].esoff.get(), same(dim), rebuilt(dim));
   for (u32 h = 2; h <= dim; ++h)
     for (u32 l = 1; l < h; ++l)
       if (side_maps[h][l]) mo.down[h][l] = std::move(side_maps[h][l]);
@@ -2214,15 +2246,14 @@ static u32 coarsen_common(Mesh& m, Buf<u32>& codes, double qual_floor, bool requ
   auto carry_up = [&](u32 h) {
     if (!m.up[0][h]) return;
     mo.up[0][h] = up_patch(h_down_deg[h][0], *m.up[0][h], m.counts[0], soff.get(), nv_out, 0, plan[h].esoff.get(),
-                           got[2 + 2 * (h - 1) + 1], got[2 + 2 * (h - 1)], mo.down[h][0].get(),
-                           h == dim && sizes ? &elems : nullptr);
+                           same(h), rebuilt(h), mo.down[h][0].get(), h == dim && sizes ? &elems : nullptr);
   };
   carry_up(1);
   carry_up(dim);
   if (sizes && sizes->ne == m.counts[1]) {
     // the new mesh's size codes: survivors' carried, products measured;
     // and what is known of the survivors' qualities
-    u32 const ne_old = m.counts[1], ngen1 = got[2], nsame1 = got[3], ne_new = nsame1 + ngen1;
+    u32 const ne_old = m.counts[1], ngen1 = rebuilt(1), nsame1 = same(1), ne_new = nsame1 + ngen1;
     Buf<u32> nc(ne_new), nk(ne_new);
     Buf<double> nq((size_t) 2 * ne_new);
     CarryCodes a{};
@@ -2257,8 +2288,8 @@ static u32 coarsen_common(Mesh& m, Buf<u32>& codes, double qual_floor, bool requ
     sizes->clear();
   }
   if (require_better && dim == 3 && m.up[1][3] && mo.down[3][1])
-    mo.up[1][3] = up_patch(6, *m.up[1][3], m.counts[1], plan[1].esoff.get(), got[3], got[2], plan[3].esoff.get(),
-                           got[7], got[6], mo.down[3][1].get());
+    mo.up[1][3] = up_patch(6, *m.up[1][3], m.counts[1], plan[1].esoff.get(), same(1), rebuilt(1),
+                           plan[3].esoff.get(), same(3), rebuilt(3), mo.down[3][1].get());
   say("collapsed", total, 1);
   overwrite(m, std::move(mo));
   return 1;

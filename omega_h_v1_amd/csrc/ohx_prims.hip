@@ -208,15 +208,6 @@ Buf<double> copy_f64(double const* a, u32 n) {
   return b;
 }
 
-Buf<u32> negate_offsets(u32 const* offs, u32 n) {
-  // offsets of 0/1 flags: the items before i without a product number
-  // i - offs[i], so no scan is needed
-  Buf<u32> o(n + 1);
-  u32* op = o.get();
-  parallel_for(n + 1, OHX_LAMBDA(u32 i) { op[i] = i - offs[i]; });
-  return o;
-}
-
 Buf<u32> scale(u32 const* a, u32 n, u32 s) {
   Buf<u32> b(n);
   u32* p = b.get();

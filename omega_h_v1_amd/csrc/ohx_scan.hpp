@@ -64,40 +64,23 @@ __device__ inline u64 pack(u32 epoch, u32 inclusive, u32 v) {
 
 __device__ inline u32 pad(u32 i) { return i + (i >> 5); }
 
-template <u32 SCAN_I, u32 LB, bool TICKET, class F>
-__global__ __launch_bounds__(SCAN_T) void scan_fn_kernel(u32 n, F f, u32 ntiles, u32* __restrict__ out,
-                                                         u64* __restrict__ tiles, u32* __restrict__ ticket,
-                                                         u32 epoch, u32* __restrict__ host_total,
-                                                         u32* __restrict__ err) {
+// LDS of a tile's scan
+template <u32 SCAN_I>
+struct TileLds {
+  u32 tile[SCAN_T * SCAN_I + SCAN_T * SCAN_I / 32];
+  u32 w[SCAN_T / 64];
+  u32 prefix;
+};
+
+// tile t of ntiles of a scan whose tile words start at tiles
+template <u32 SCAN_I, u32 LB, class F>
+__device__ inline void scan_tile(TileLds<SCAN_I>& lds, u32 n, F f, u32 t, u32 ntiles, u32* __restrict__ out,
+                                 u64* __restrict__ tiles, u32 epoch, u32* __restrict__ host_total,
+                                 u32* __restrict__ err) {
   constexpr u32 SCAN_TILE = SCAN_T * SCAN_I;
-  __shared__ u32 tile[SCAN_TILE + SCAN_TILE / 32];
-  __shared__ u32 lds_w[SCAN_T / 64];
-  __shared__ u32 s_prefix;
-  __shared__ u32 s_tile;
-  // Which tile a block scans.  With one host thread (one stream of scans)
-  // the tile is the block index: workgroups are dispatched in index order
-  // within each XCD, so the lowest-numbered resident block always finds
-  // every earlier tile finished or on an XCD with free slots, and the
-  // look-back cannot wait on a block that is never scheduled.  That
-  // argument does not cover scans of other streams holding the free slots,
-  // so with several host threads (TICKET) a block takes its tile from a
-  // fetch-add ticket: tiles are then claimed only by resident blocks, in
-  // order, and the lowest unfinished tile always belongs to a running block
-  // whose predecessors are all done, whatever else occupies the GPU.  (The
-  // ticket costs one same-address atomic per block, which retire one per
-  // ~12 ns on this part, so the single-stream path does without it.)  The
-  // block that draws the last ticket clears the word for the next scan of
-  // the stream.  The spin stays bounded regardless.
-  u32 t = blockIdx.x;
-  if (TICKET) {
-    if (threadIdx.x == 0) {
-      u32 k = atomicAdd(ticket, 1u);
-      if (k == ntiles - 1) __hip_atomic_store(ticket, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      s_tile = k;
-    }
-    __syncthreads();
-    t = s_tile;
-  }
+  u32* const tile = lds.tile;
+  u32* const lds_w = lds.w;
+  u32& s_prefix = lds.prefix;
   u32 base = t * SCAN_TILE;
 #pragma unroll
   for (u32 k = 0; k < SCAN_I; ++k) {
@@ -204,6 +187,74 @@ __global__ __launch_bounds__(SCAN_T) void scan_fn_kernel(u32 n, F f, u32 ntiles,
   if (t == 0 && threadIdx.x == 0) out[0] = 0;
 }
 
+// Which tile a block scans.  With one host thread (one stream of scans)
+// the tile is the block index: workgroups are dispatched in index order
+// within each XCD, so the lowest-numbered resident block always finds
+// every earlier tile finished or on an XCD with free slots, and the
+// look-back cannot wait on a block that is never scheduled.  That
+// argument does not cover scans of other streams holding the free slots,
+// so with several host threads (TICKET) a block takes its tile from a
+// fetch-add ticket: tiles are then claimed only by resident blocks, in
+// order, and the lowest unfinished tile always belongs to a running block
+// whose predecessors are all done, whatever else occupies the GPU.  (The
+// ticket costs one same-address atomic per block, which retire one per
+// ~12 ns on this part, so the single-stream path does without it.)  The
+// block that draws the last ticket clears the word for the next scan of
+// the stream.  The spin stays bounded regardless.
+template <bool TICKET>
+__device__ inline u32 take_tile(u32 ntiles, u32* ticket) {
+  __shared__ u32 s_tile;
+  if (!TICKET) return blockIdx.x;
+  if (threadIdx.x == 0) {
+    u32 k = atomicAdd(ticket, 1u);
+    if (k == ntiles - 1) __hip_atomic_store(ticket, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    s_tile = k;
+  }
+  __syncthreads();
+  return s_tile;
+}
+
+template <u32 SCAN_I, u32 LB, bool TICKET, class F>
+__global__ __launch_bounds__(SCAN_T) void scan_fn_kernel(u32 n, F f, u32 ntiles, u32* __restrict__ out,
+                                                         u64* __restrict__ tiles, u32* __restrict__ ticket,
+                                                         u32 epoch, u32* __restrict__ host_total,
+                                                         u32* __restrict__ err) {
+  __shared__ TileLds<SCAN_I> lds;
+  u32 const t = take_tile<TICKET>(ntiles, ticket);
+  scan_tile<SCAN_I, LB>(lds, n, f, t, ntiles, out, tiles, epoch, host_total, err);
+}
+
+// One of the scans of a launch: out[i + 1] - out[i] = (in[i] == key), or
+// in[i] itself for a key of JOB_SUM
+constexpr u32 JOB_SUM = 0xffffffffu;
+constexpr u32 MAX_JOBS = 8;
+struct ScanJobs {
+  u32 njobs;
+  struct Job {
+    u32 n, key, tile0;
+    u32 const* in;
+    u32* out;
+  } j[MAX_JOBS];
+};
+template <u32 SCAN_I, u32 LB, bool TICKET>
+__global__ __launch_bounds__(SCAN_T) void scan_jobs_kernel(ScanJobs J, u32 ntiles, u64* __restrict__ tiles,
+                                                           u32* __restrict__ ticket, u32 epoch,
+                                                           u32 const* __restrict__ flag, u32* __restrict__ host,
+                                                           u32* __restrict__ err) {
+  __shared__ TileLds<SCAN_I> lds;
+  u32 const t = take_tile<TICKET>(ntiles, ticket);
+  if (t == 0 && threadIdx.x == 0) host[2 * MAX_JOBS] = flag ? *flag : 0u;
+  u32 k = 0;
+  while (k + 1 < J.njobs && t >= J.j[k + 1].tile0) ++k;
+  ScanJobs::Job const& job = J.j[k];
+  u32 const* const in = job.in;
+  u32 const key = job.key;
+  u32 const t0 = job.tile0, nt = (k + 1 < J.njobs ? J.j[k + 1].tile0 : ntiles) - t0;
+  scan_tile<SCAN_I, LB>(
+      lds, job.n, [in, key](u32 i) { return key == JOB_SUM ? in[i] : in[i] == key ? 1u : 0u; }, t - t0, nt, job.out,
+      tiles + t0, epoch, host + 2 * k, err);
+}
+
 }  // namespace scan_detail
 
 template <u32 I, u32 LB, bool TICKET, class F>
@@ -246,6 +297,45 @@ void exscan_fn(u32 n, F f, u32* out, u32* host_total_dev = nullptr) {
     else
       exscan_launch<16, 1>(n, f, out, host_total_dev, ea, eb);
   });
+}
+
+// Several scans in one launch, with the host's read of their totals: a pass
+// decides on a handful of offset arrays at once, and on meshes of up to a few
+// hundred thousand entities each scan of its own is a launch's latency (a
+// collapse pass's seven scans and the gather of their totals took 60 us at
+// 130,000 triangles, one launch 9 us).  Each scan's tiles are consecutive, in
+// launch order, and look back only over its own, so the argument for the
+// single scan's progress holds.  totals[k] gets job k's, *flag_out the word
+// flag points to (one synchronisation).
+inline void exscan_jobs(scan_detail::ScanJobs& J, u32 const* flag, u32* totals, u32* flag_out) {
+  using namespace scan_detail;
+  size_t all = 0;
+  for (u32 k = 0; k < J.njobs; ++k) all += J.j[k].n;
+  bool const big = all >= ((size_t) 1 << 21);  // as the tuned single scans: 16 items a thread from 2^21 on
+  u32 const tile = SCAN_T * (big ? 16 : 4);
+  u32 nt = 0;
+  for (u32 k = 0; k < J.njobs; ++k) {
+    J.j[k].tile0 = nt;
+    nt += J.j[k].n ? (J.j[k].n + tile - 1) / tile : 1;
+  }
+  ScanTiles st = scan_tiles_for(nt);
+  u32* host = dev_slot<u32>(SLOT_JOBS);
+  auto go = [&](auto kernel) {
+    launch_timed("scan", (double) all * 8, kernel, dim3(nt), dim3(SCAN_T), J, nt, st.tiles, st.ticket, st.epoch, flag,
+                 host, dev_error_word());
+  };
+  if (scan_concurrent())
+    big ? go(scan_jobs_kernel<16, 1, true>) : go(scan_jobs_kernel<4, 4, true>);
+  else
+    big ? go(scan_jobs_kernel<16, 1, false>) : go(scan_jobs_kernel<4, 4, false>);
+  sync();
+  u32 const* h = host_slot<u32>(SLOT_JOBS);
+  for (u32 k = 0; k < J.njobs; ++k) totals[k] = h[2 * k];
+  if (flag_out) *flag_out = h[2 * MAX_JOBS];
+}
+inline void scan_job(scan_detail::ScanJobs& J, u32 n, u32 const* in, u32 key, u32* out) {
+  OHX_REQUIRE(J.njobs < scan_detail::MAX_JOBS, "too many scans in one launch");
+  J.j[J.njobs++] = {n, key, 0, in, out};
 }
 
 // as exscan_fn and returns the total (one synchronisation)

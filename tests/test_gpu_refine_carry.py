@@ -38,3 +38,20 @@ def test_split_passes_carry_maps(dim, n, h, jitter, ops):
             assert np.array_equal(a.down(high, low), fresh.down(high, low)), (high, low)
     for p, q in zip(a.up(1, dim), fresh.up(1, dim)):
         assert np.array_equal(p, q)
+
+
+def test_split_and_collapse_with_large_scans():
+    """A split and a collapse pass whose offset scans together pass 2^21
+    items, where the launch takes 16 items a thread."""
+    got = []
+    for which in ("product", "oracle"):
+        lib = ML.load(which)
+        m = P.make_mesh(lib, 3, 44)
+        assert sum(m.counts()[1:]) >= 1 << 21
+        x = m.coords().reshape(-1, 3)
+        # large sizes on one side, small ones on the other
+        m.add_field(0, "adapt_size", np.where(x[:, 0] < 0.9, 4.0, 0.8) / 44)
+        m.last = (m.refine_by_size(0.2), m.coarsen_by_size(0.2, 1.0 / 3.0))
+        got.append(m)
+    assert got[0].last == got[1].last == (1, 1)
+    assert P.diff_states(*got) is None
