@@ -2592,8 +2592,10 @@ __device__ inline u32 edge_ring(u32 edge, u32 f, u32 e, u32 const* ua, u32 const
 //   B. lane 0 chains the pairs into the ring (edge_ring.cpp:12-74);
 //   C. lane j stages ring vertex j (or edge vertex j - ring size): its
 //      coordinates and metric;
-//   D. lane l measures unique triangles l, l + SW_G, ...: the two tets it
-//      forms with the edge's ends, as choose_edge_swap does;
+//   D. two neighbouring lanes measure a unique triangle: the two tets it
+//      forms with the edge's ends, as choose_edge_swap does (a ring of 4 has
+//      4 triangles: its 8 tets take the group's 8 lanes once; with both of a
+//      triangle's tets on one lane half the lanes waited);
 //   E. lane l takes triangulations l, l + SW_G, ...: the running minimum of
 //      its triangles, stopped at the first negative one as the reference's
 //      loop stops, and the lane's best with a strict > in triangulation
@@ -2656,17 +2658,17 @@ __device__ inline void swap_choose(SwapLds<MT>& L, u32 g, u32 lane, bool active,
     u32 ntri = k_sw_ntri[rs];
     unsigned char const(*tris)[3] = k_sw_tris + k_sw_tri_off[rs];
     u32 const E0 = rs, E1 = rs + 1;  // edge vertices follow the ring in LDS
-    for (u32 t = lane; t < ntri; t += SW_G) {
-      u32 a0 = tris[t][0], a1 = tris[t][1], a2 = tris[t][2];
-      double tmin = 1, q;
+    for (u32 k = lane; k < 2 * ntri; k += SW_G) {
       // the triangle with edge end 1, then with the first two corners
-      // exchanged and edge end 0 (choose_edge_swap's two tets)
-      q = swap_tet_q<MT, F32>(L, g, a0, a1, a2, E1);
-      if (q < tmin) tmin = q;
-      q = swap_tet_q<MT, F32>(L, g, a1, a0, a2, E0);
-      if (q < tmin) tmin = q;
+      // exchanged and edge end 0 (choose_edge_swap's two tets), on two
+      // neighbouring lanes
+      u32 const t = k / 2, end = k & 1u;
+      double const q = swap_tet_q<MT, F32>(L, g, tris[t][end], tris[t][1 - end], tris[t][2], end ? E0 : E1);
+      double tmin = q < 1 ? q : 1;
+      double const other = __shfl_xor(tmin, 1, SW_G);
+      if (other < tmin) tmin = other;
       if (F32 && !(tmin > (double) SCREEN_MARGIN || tmin < -(double) SCREEN_MARGIN)) nz = true;
-      L.tq[g][t] = tmin;
+      if (!end) L.tq[g][t] = tmin;
     }
   }
   __syncthreads();
@@ -3639,7 +3641,10 @@ u32 swap_slivers(Mesh& m, double good_qual, u32 nlayers, double const* eq, doubl
 // of its pairs was removed in a pass after the one that made the face.
 
 // Words of a swap run (SwapRunView::words)
-enum { RW_ACC = 0, RW_EVAL = 1, RW_AFF = 2, RW_POOL = 3, RW_FIRST = 4, RW_NEED = 5, RW_FLAGS = 8, RW_WORDS = 16 };
+enum { RW_ACC = 0, RW_AFF = 2, RW_POOL = 3, RW_FIRST = 4, RW_NEED = 5, RW_FLAGS = 8, RW_EVAL = 16, RW_WORDS = 24 };
+// ring sizes 3 to MAX_EDGE_SWAP: the candidates to evaluate are listed by
+// ring size
+constexpr u32 RUN_RINGS = MAX_EDGE_SWAP - 2;
 // an edge's word in a run: its choice is known, it is accepted, then ring
 // size and triangulation code as in the swap cache; a dead or boundary edge
 // is known and rejected for good
@@ -3672,8 +3677,9 @@ struct SwapRunView {
   u32* fcd;
   u32* fci;
   u32* fbirth;
-  u32* acc;  // accepted candidates and candidates to evaluate (any order)
-  u32* eval;
+  u32* acc;  // accepted candidates (any order)
+  u32* eval; // candidates to evaluate (any order), a list of ecap places per ring size
+  u32 ecap;
   u32* sw;   // swapped edges in order, their first products of each dimension
   u32* o1;
   u32* o2;
@@ -3771,56 +3777,98 @@ __global__ __launch_bounds__(BLOCK) void run_layer_k(u32 n, uint4 const* __restr
 }
 
 // the candidates: live interior edges of marked tets whose swap is accepted
-// (they enter the independent set) or not yet known (to be evaluated)
+// (they enter the independent set) or not yet known (to be evaluated, listed
+// by ring size: a ring of 7 has 35 triangles and one of 4 has 4, and a wave
+// takes as long as its longest); a ring too large is rejected here
 __global__ __launch_bounds__(RUN_AB) void run_candidates_k(SwapRunView R, unsigned char const* __restrict__ marks) {
   __shared__ u32 lds[RUN_AB / 64];
+  constexpr u32 LISTS = 1 + RUN_RINGS;  // the accepted, then the rings
   u32 const e0 = blockIdx.x * RUN_AT + threadIdx.x;
-  u32 acc = 0, ask = 0;  // bits: this thread's edges e0 + k RUN_AB
+  u32 list[RUN_AI];  // each edge's list, LISTS: none
+  u32 count[(LISTS + 1) / 2] = {};  // two lists' counts a word: a block has at most 4096 of each
+#pragma unroll
   for (u32 k = 0; k < RUN_AI; ++k) {
+    list[k] = LISTS;
     u32 const e = e0 + k * RUN_AB;
-    if (e >= R.nE) break;
+    if (e >= R.nE) continue;
     u32 const w = R.info[e];
     if ((w & RI_KNOWN) && !(w & RI_ACCEPT)) continue;
     bool in = false;
     u32 const f = R.lb[e], n = R.ln[e];
     for (u32 j = 0; j < n && !in; ++j) in = marks[R.ua[f + j]] != 0;
-    if (in) (w & RI_KNOWN ? acc : ask) |= 1u << k;
+    if (!in) continue;
+    if (w & RI_KNOWN)
+      list[k] = 0;
+    else if (n > MAX_EDGE_SWAP)
+      R.info[e] = RI_KNOWN;
+    else
+      list[k] = n < 3 ? 1 : n - 2;  // (below 3: the evaluation reports it)
   }
-  // both lists' places in one prefix (a block has at most 4096 of each)
-  u32 total;
-  u32 const p = run_block_prefix((u32) __popc(acc) | ((u32) __popc(ask) << 16), lds, &total);
-  if (threadIdx.x == 0) {
-    lds[0] = (total & 0xffffu) ? atomicAdd(R.words + RW_ACC, total & 0xffffu) : 0u;
-    lds[1] = (total >> 16) ? atomicAdd(R.words + RW_EVAL, total >> 16) : 0u;
-  }
-  __syncthreads();
-  u32 a = lds[0] + (p & 0xffffu), b = lds[1] + (p >> 16);
-  for (u32 k = 0; k < RUN_AI; ++k) {
-    u32 const e = e0 + k * RUN_AB;
-    if ((acc >> k) & 1u) {
-      R.acc[a++] = e;
-      R.sa[e] = UNKNOWN;
+#pragma unroll
+  for (u32 k = 0; k < RUN_AI; ++k)
+#pragma unroll
+    for (u32 l = 0; l < LISTS; ++l)
+      if (list[k] == l) count[l / 2] += 1u << (16 * (l % 2));
+#pragma unroll
+  for (u32 p = 0; p < (LISTS + 1) / 2; ++p) {
+    u32 total;
+    u32 const mine = run_block_prefix(count[p], lds, &total);
+    if (threadIdx.x < 2) {
+      u32 const l = 2 * p + threadIdx.x, n = (total >> (16 * threadIdx.x)) & 0xffffu;
+      lds[threadIdx.x] = n ? atomicAdd(R.words + (l == 0 ? (u32) RW_ACC : RW_EVAL + l - 1), n) : 0u;
     }
-    if ((ask >> k) & 1u) R.eval[b++] = e;
+    __syncthreads();
+    u32 at[2] = {lds[0] + (mine & 0xffffu), lds[1] + (mine >> 16)};
+    __syncthreads();
+#pragma unroll
+    for (u32 k = 0; k < RUN_AI; ++k) {
+      if (list[k] / 2 != p || list[k] == LISTS) continue;
+      u32 const e = e0 + k * RUN_AB;
+      if (list[k] == 0) {
+        R.acc[at[0]++] = e;
+        R.sa[e] = UNKNOWN;
+      } else if (list[k] % 2 == 0) {
+        R.eval[(size_t) (list[k] - 1) * R.ecap + at[0]++] = e;
+      } else {
+        R.eval[(size_t) (list[k] - 1) * R.ecap + at[1]++] = e;
+      }
+    }
   }
 }
 
 // swap qualities of the candidates to evaluate: the choice goes into the
-// edge's word
+// edge's word.  Bound by FP64 arithmetic with a wave's groups in step, so a
+// batch holds one ring size: with the rings mixed as they came and both tets
+// of a triangle on one lane, a call took 420 us where it now takes 247 us
+// (mean of the 302 calls of an adaptation to 511 thousand tets), 101 us where
+// it now takes 62 us at 55 thousand.
 template <bool MT, bool MIXED>
 __global__ __launch_bounds__(BLOCK, 4) void run_quality_k(SwapRunView R, double const* __restrict__ x,
                                                           double const* __restrict__ mt,
                                                           double const* __restrict__ tq, u32* __restrict__ err,
                                                           ScreenStats st) {
   __shared__ SwapLds<MT> L;
-  u32 const n = R.words[RW_EVAL];
   u32 const group = threadIdx.x / SW_G;
   bool const lead = threadIdx.x % SW_G == 0;
-  for (u32 base = blockIdx.x * SW_EDGES; base < n; base += gridDim.x * SW_EDGES) {
+  // batches of one ring size, the largest rings first
+  u32 before[RUN_RINGS + 1];
+  before[0] = 0;
+#pragma unroll
+  for (u32 c = 0; c < RUN_RINGS; ++c)
+    before[c + 1] = before[c] + (R.words[RW_EVAL + RUN_RINGS - 1 - c] + SW_EDGES - 1) / SW_EDGES;
+  for (u32 batch = blockIdx.x; batch < before[RUN_RINGS]; batch += gridDim.x) {
+    u32 c = 0, first = 0;
+#pragma unroll
+    for (u32 k = 1; k < RUN_RINGS; ++k)
+      if (batch >= before[k]) {
+        c = k;
+        first = before[k];
+      }
+    u32 const ring = RUN_RINGS - 1 - c, n = R.words[RW_EVAL + ring], base = (batch - first) * SW_EDGES;
     u32 e, rs, code;
     bool settled;
     double best;
-    bool const accept = swap_quality_batch<MT, MIXED>(L, n, base + group, R.eval, R.lb, R.ln, R.ua, R.ud, R.ev, R.vt,
+    bool const accept = swap_quality_batch<MT, MIXED>(L, n, base + group, R.eval + (size_t) ring * R.ecap, R.lb, R.ln, R.ua, R.ud, R.ev, R.vt,
                                                       x, mt, tq, err, st, &e, &settled, &best, &rs, &code);
     if (settled && lead) {
       R.info[e] = accept ? RI_KNOWN | RI_ACCEPT | (rs << 16) | code : RI_KNOWN;
@@ -3833,13 +3881,14 @@ __global__ __launch_bounds__(BLOCK, 4) void run_quality_k(SwapRunView R, double 
 // the evaluated candidates that are accepted join the accepted ones
 __global__ __launch_bounds__(RUN_AB) void run_accept_k(SwapRunView R) {
   __shared__ u32 lds[RUN_AB / 64];
-  u32 const n = R.words[RW_EVAL];
+  u32 const ring = blockIdx.y;
+  u32 const n = R.words[RW_EVAL + ring];
   for (u32 base = blockIdx.x * RUN_AT; base < n; base += gridDim.x * RUN_AT) {
     u32 e[RUN_AI], in = 0;
 #pragma unroll
     for (u32 k = 0; k < RUN_AI; ++k) {
       u32 const i = base + k * RUN_AB + threadIdx.x;
-      e[k] = i < n ? R.eval[i] : INVALID;
+      e[k] = i < n ? R.eval[(size_t) ring * R.ecap + i] : INVALID;
     }
 #pragma unroll
     for (u32 k = 0; k < RUN_AI; ++k)
@@ -4484,7 +4533,7 @@ struct SwapRun {
     need(ln, nE, want);
     need(cnt, nE, want);
     need(acc, nE, want);  // still read: its edges' states are cleared at the pass's end
-    eval = Buf<u32>(info.size());
+    eval = Buf<u32>(RUN_RINGS * info.size());
     size_t const states = (info.size() + RUN_PER) / RUN_PER * RUN_PER;
     Buf<unsigned char> a2(states), b2(states);
     if (old) {
@@ -4541,6 +4590,7 @@ struct SwapRun {
     R.fbirth = fbirth.get();
     R.acc = acc.get();
     R.eval = eval.get();
+    R.ecap = (u32) info.size();
     R.words = words.get();
     return R;
   }
@@ -4586,7 +4636,7 @@ struct SwapRun {
     ln = Buf<u32>(cE);
     cnt = Buf<u32>(cE);
     acc = Buf<u32>(cE);
-    eval = Buf<u32>(cE);
+    eval = Buf<u32>(RUN_RINGS * cE);
     size_t const states = (cE + RUN_PER) / RUN_PER * RUN_PER;
     sa = Buf<unsigned char>(states);
     sb = Buf<unsigned char>(states);
@@ -4692,7 +4742,7 @@ struct SwapRun {
     else
       mt ? go(run_quality_k<true, false>, "swap_quality_f64") : go(run_quality_k<false, false>, "swap_quality_f64");
     u32 const ab = nblocks(aE, RUN_AT);
-    hipLaunchKernelGGL(run_accept_k, dim3(ab < 256 ? ab : 256), dim3(RUN_AB), 0, stream(), R);
+    hipLaunchKernelGGL(run_accept_k, dim3(ab < 64 ? ab : 64, RUN_RINGS), dim3(RUN_AB), 0, stream(), R);
     check_launch("run_accept");
   }
 

@@ -70,6 +70,20 @@ def test_swap_run_equals_whole_mesh_passes(libs, n, ops):
         assert np.array_equal(got, want)
 
 
+@pytest.mark.parametrize("n,before", [(4, 12), (5, 14), (6, 16)])
+def test_swap_run_over_every_ring_size(libs, n, before):
+    """The candidates are evaluated by ring size: between the meshes before
+    and after the passes, rings of every size from 3 to the largest a swap
+    takes (7) and larger ones are met."""
+    a, b = (front(lib, n, 0.3) for lib in libs)
+    rings = set()
+    for ops in (before, before + 3, 40):
+        assert a.adapt(max_ops=ops) == b.adapt(max_ops=ops)
+        rings |= set(np.diff(a.up(1, 3)[0])[a.tag(1, "class_dim") == 3].tolist())
+    assert set(range(3, 9)) <= rings
+    assert same(a, b) is None
+
+
 def test_round_limit_inside_a_swap_run(libs):
     """A run whose independent set reaches the round limit fails as a pass
     over a whole mesh does, and leaves the mesh of the passes before."""
