@@ -1186,6 +1186,7 @@ __device__ inline double collapse_elem_q(u32 e, u32 dir, u32 gen, V3 const& pg, 
 
 struct CqArgs {
   u32 ncand;
+  u32 chunk;        // directions per block, at most CQ_CHUNK
   u32 const* list;  // candidate directions 2 e + j, grouped by collapsing vertex
   u32 const* ev;
   u32 const* uo;    // up(0, dim)
@@ -1203,103 +1204,186 @@ struct CqArgs {
   ScreenStats st;
 };
 
-// One collapse direction per group of G lanes.  The directions come
+// Collapse directions, a group of G lanes each.  The directions come
 // grouped by collapsing vertex (the list is built from each vertex's edges
 // in turn), so the groups of one block share the vertex's element star and
 // its vertices in the caches: measured on C3, the edge-ordered form fetched
 // about seven times the arrays' size from beyond L2 per launch.  Both
 // directions of an edge may be in flight at once, so the code bits are
 // cleared (or the inexact bit set) with atomics on the edge's word.
+//
+// FP64 arithmetic bounds it, and how many of a wave's lanes take part: a
+// direction ends at its first element below the floor or after a whole star
+// of about 20, so with one direction per group a wave ran at 20 of its 64
+// lanes.  A block takes a.chunk directions instead, and a group whose
+// direction has ended takes the block's next one (once a quarter of the
+// wave's groups wait, as taking one is a chain of loads).
+// The directions that FP32 leaves open are listed and follow in FP64 in the
+// same way.
+constexpr u32 CQ_CHUNK = 1024, CQ_BLOCKS = 1024;
+
+// a group's direction
+struct CqDir {
+  u32 i, j, gen, k, end;
+  double floor_;
+  V3 pg;
+  Sym mg;
+};
+
+// Evaluates directions get(0) ... get(n - 1), shared by the block's groups
+// through the LDS counter *next (zero).  A direction ends early once its
+// minimum is below d.floor_ - margin, where STOP allows it; done(d, minimum,
+// minimum of the elements' present quality, NaN seen) is called by the
+// group's first lane.
+template <u32 DIM, u32 G, bool F32, bool STOP, class Get, class Done>
+__device__ inline void cq_directions(CqArgs const& A, u32 n, u32* next, double margin, Get get, Done done) {
+  constexpr u32 ENOUGH = G < 16 ? 16 / G : 1;
+  u32 const lane = threadIdx.x & 63u, gl = lane % G, lead = lane - gl;
+  u64 const group = (G == 64 ? ~0ull : ((1ull << G) - 1)) << lead;
+  double const* __restrict__ eq = F32 ? nullptr : A.eq;
+  CqDir d{};
+  bool has = false, more = true;
+  double minq = 1, old_minq = 1;
+  bool nan = false;
+  for (;;) {
+    u64 const waiting = __ballot(!has && gl == 0);
+    u32 const nwait = (u32) __popcll(waiting);
+    if (more && nwait >= ENOUGH) {
+      u32 at = 0;
+      if (lane == 0) at = atomicAdd(next, nwait);
+      at = (u32) __builtin_amdgcn_readfirstlane((int) at);
+      more = at + nwait < n;
+      if (!has) {
+        at += (u32) __popcll(waiting & ((1ull << lead) - 1));
+        u32 dir;
+        if (at < n && get(at, &dir)) {
+          d.i = dir >> 1;
+          d.j = dir & 1u;
+          u32 const col = A.ev[2 * (size_t) d.i + d.j];
+          d.gen = A.ev[2 * (size_t) d.i + (1 - d.j)];
+          // one floor for the mesh, or its component's in a batch
+          d.floor_ = A.qfe ? A.qfe[d.i] : A.qual_floor;
+          d.pg = ld3(A.x + 3 * (size_t) d.gen);
+          if (A.mt) d.mg = ld6(A.mt + 6 * (size_t) d.gen);
+          d.k = A.uo[col] + gl;
+          d.end = A.uo[col + 1];
+          minq = old_minq = 1;
+          nan = false;
+          has = true;
+        }
+      }
+    }
+    if (!__ballot(has)) {
+      if (more) continue;
+      break;
+    }
+    bool ended = true, low = false;
+    if (has) {
+      if (d.k < d.end) {
+        u32 const e = A.ua[d.k];
+        if (eq && eq[e] < old_minq) old_minq = eq[e];
+        bool adj;
+        double const q = collapse_elem_q<DIM, F32>(e, A.ud[d.k], d.gen, d.pg, d.mg, A.vel, A.x, A.mt, &adj);
+        if (!adj) {
+          if (F32 && !(q == q)) nan = true;
+          if (q < minq) minq = q;
+        }
+        d.k += G;
+      }
+      ended = d.k >= d.end;
+      // below the floor the direction is rejected whatever the remaining
+      // elements give (the minimum only falls)
+      low = STOP && minq < d.floor_ - margin;
+    }
+    if (G == 1) {
+      if (has && (ended || low)) {
+        done(d, minq, old_minq, nan);
+        has = false;
+      }
+    } else {
+      bool const fin = has && ((__ballot(ended) & group) == group || (__ballot(low) & group) != 0);
+      if (__ballot(fin)) {
+        double const gm = group_min<G>(minq), go = eq ? group_min<G>(old_minq) : 1;
+        bool const gn = F32 && (__ballot(nan) & group) != 0;
+        if (fin && gl == 0) done(d, gm, go, gn);
+        if (fin) has = false;
+      }
+    }
+  }
+}
+
 template <u32 DIM, u32 G, u32 MODE>
 __global__ __launch_bounds__(BLOCK) void coarsen_quality_f64(CqArgs A) {
-  u32 const ncand = A.ncand;
-  u32 const* __restrict__ ev = A.ev;
-  u32 const* __restrict__ uo = A.uo;
-  u32 const* __restrict__ ua = A.ua;
-  u32 const* __restrict__ ud = A.ud;
-  u32 const* __restrict__ vel = A.vel;
-  double const* __restrict__ x = A.x;
-  double const* __restrict__ mt = A.mt;
-  double const* __restrict__ eq = A.eq;
+  constexpr bool SCREENED = MODE == CQ_SCREEN || MODE == CQ_CERTIFIED;
+  __shared__ u32 next[2], nopen;
+  __shared__ u32 open[SCREENED ? CQ_CHUNK : 1];
+  u32 const first = xcd_block() * A.chunk;
+  if (first >= A.ncand) return;  // the whole block
+  u32 n = A.ncand - first < A.chunk ? A.ncand - first : A.chunk;
+  if (threadIdx.x < 2) next[threadIdx.x] = 0;
+  if (threadIdx.x == 2) nopen = 0;
+  __syncthreads();
   u32* __restrict__ codes = A.codes;
   double* __restrict__ out = A.out;
   ScreenStats const st = A.st;
-  size_t gid = (size_t) xcd_block() * BLOCK + threadIdx.x;
-  size_t slot = gid / G;
-  u32 lane = (u32) (gid % G);
-  if (slot >= ncand) return;  // whole groups leave together
-  u32 const ed = A.list[slot];
-  u32 const i = ed >> 1, j = ed & 1u;
-  u32 const col = ev[2 * (size_t) i + j], gen = ev[2 * (size_t) i + (1 - j)];
-  if (MODE == CQ_FORCE && !((codes[i] & inexact_bit(j)) && A.vmark[col])) return;
-  // one floor for the mesh, or its component's in a batch
-  double const qual_floor = A.qfe ? A.qfe[i] : A.qual_floor;
-  bool const f32 = (MODE == CQ_SCREEN || MODE == CQ_CERTIFIED) && !eq;
-  V3 const pg = ld3(x + 3 * (size_t) gen);
-  Sym mg;
-  if (mt) mg = ld6(mt + 6 * (size_t) gen);
-  double minq32 = 1;
+  u32 const* list = A.list + first;
+  bool const f32 = SCREENED && !A.eq;
   if (f32) {
     // FP32: a direction certainly below the floor is rejected at its first
     // element below it; CQ_CERTIFIED also accepts one certainly above
-    bool nan = false;
-    double const lo = qual_floor - (double) SCREEN_MARGIN;
-    for (u32 k = uo[col] + lane; k < uo[col + 1]; k += G) {
-      bool adj;
-      double q = collapse_elem_q<DIM, true>(ua[k], ud[k], gen, pg, mg, vel, x, mt, &adj);
-      if (adj) continue;
-      if (!(q == q)) nan = true;
-      if (q < minq32) minq32 = q;
-      if (minq32 < lo) break;
-    }
-    minq32 = group_min<G>(minq32);
-#pragma unroll
-    for (u32 d = G / 2; d >= 1; d >>= 1) nan = nan || __shfl_xor((int) nan, d, G);
-    bool reject = !nan && minq32 < lo;
-    bool accept = MODE == CQ_CERTIFIED && !nan && minq32 > qual_floor + (double) SCREEN_MARGIN;
-    if (lane == 0) wave_count(st.screened, reject || accept);
-    if (reject) {
-      if (lane == 0) atomicXor(&codes[i], (1u << j) | rejected_bit(j));
-      return;
-    }
-    if (accept) {
-      if (lane == 0) {
-        out[2 * (size_t) i + j] = minq32;
-        atomicOr(&codes[i], inexact_bit(j));
-      }
-      return;
-    }
-    if (lane == 0) wave_count(st.reeval, true);
+    double const m = (double) SCREEN_MARGIN;
+    cq_directions<DIM, G, true, true>(
+        A, n, next, m,
+        [&](u32 at, u32* dir) {
+          *dir = list[at];
+          return true;
+        },
+        [&](CqDir const& d, double minq, double, bool nan) {
+          bool const reject = !nan && minq < d.floor_ - m;
+          bool const accept = MODE == CQ_CERTIFIED && !nan && minq > d.floor_ + m;
+          wave_count(st.screened, reject || accept);
+          if (reject) {
+            atomicXor(&codes[d.i], (1u << d.j) | rejected_bit(d.j));
+            return;
+          }
+          out[2 * (size_t) d.i + d.j] = minq;
+          if (accept) {
+            atomicOr(&codes[d.i], inexact_bit(d.j));
+            return;
+          }
+          wave_count(st.reeval, true);
+          open[atomicAdd(&nopen, 1u)] = 2 * d.i + d.j;
+        });
+    __syncthreads();
+    n = nopen;
+    list = open;
   }
-  if (MODE == CQ_FORCE && lane == 0) wave_count(st.reeval, true);
-  double minq = 1, old_minq = 1;
-  for (u32 k = uo[col] + lane; k < uo[col + 1]; k += G) {
-    u32 e = ua[k];
-    if (eq && eq[e] < old_minq) old_minq = eq[e];
-    bool adj;
-    double q = collapse_elem_q<DIM, false>(e, ud[k], gen, pg, mg, vel, x, mt, &adj);
-    if (adj) continue;
-    if (q < minq) minq = q;
-    // below the floor the direction is rejected whatever the remaining
-    // elements give (the minimum only falls), so the lane stops; the
-    // screened kernels keep the full minimum for their error statistic
-    if (MODE == CQ_F64 && minq < qual_floor) break;
-  }
-  minq = group_min<G>(minq);
-  if (eq) old_minq = group_min<G>(old_minq);
-  if (lane != 0) return;
-  if ((f32 || MODE == CQ_FORCE) && minq == minq) {
-    double d = MODE == CQ_FORCE ? minq - out[2 * (size_t) i + j] : minq - minq32;
-    note_max_err(st.max_err, (float) (d < 0 ? -d : d));
-  }
-  if ((minq < qual_floor) || (eq && (minq <= old_minq))) {
-    // the direction's bit is set and its rejected bit is not, and the
-    // inexact bit is set exactly where an FP32 value is measured again
-    atomicXor(&codes[i], (1u << j) | rejected_bit(j) | (MODE == CQ_FORCE ? inexact_bit(j) : 0u));
-  } else {
-    out[2 * (size_t) i + j] = minq;
-    if (MODE == CQ_FORCE) atomicAnd(&codes[i], ~inexact_bit(j));
-  }
+  // the screened kernels keep the full minimum for their error statistic
+  cq_directions<DIM, G, false, MODE == CQ_F64>(
+      A, n, next + 1, 0.0,
+      [&](u32 at, u32* dir) {
+        u32 const ed = list[at];
+        *dir = ed;
+        if (MODE != CQ_FORCE) return true;
+        bool const wanted =
+            (codes[ed >> 1] & inexact_bit(ed & 1u)) && A.vmark[A.ev[2 * (size_t) (ed >> 1) + (ed & 1u)]];
+        return wanted;
+      },
+      [&](CqDir const& d, double minq, double old_minq, bool) {
+        if (MODE == CQ_FORCE) wave_count(st.reeval, true);
+        if ((f32 || MODE == CQ_FORCE) && minq == minq) {
+          double const e = minq - out[2 * (size_t) d.i + d.j];
+          note_max_err(st.max_err, (float) (e < 0 ? -e : e));
+        }
+        if ((minq < d.floor_) || (A.eq && (minq <= old_minq))) {
+          // the direction's bit is set and its rejected bit is not, and the
+          // inexact bit is set exactly where an FP32 value is measured again
+          atomicXor(&codes[d.i], (1u << d.j) | rejected_bit(d.j) | (MODE == CQ_FORCE ? inexact_bit(d.j) : 0u));
+        } else {
+          out[2 * (size_t) d.i + d.j] = minq;
+          if (MODE == CQ_FORCE) atomicAnd(&codes[d.i], ~inexact_bit(d.j));
+        }
+      });
 }
 
 // collapse_to_vert (collapses_to_verts.cpp:13-42): whether each vertex
@@ -1685,8 +1769,12 @@ static char const* cq_name(u32 mode) {
 }
 
 template <u32 DIM, u32 MODE>
-static void cq_launch(u32 g, CqArgs const& a, double bytes, hipEvent_t ea, hipEvent_t eb) {
-  dim3 grid(nblocks((size_t) a.ncand * g));
+static void cq_launch(u32 g, CqArgs a, double bytes, hipEvent_t ea, hipEvent_t eb) {
+  // a block's share: at least a direction per group, and more as soon as
+  // that fills the chip (four blocks per CU)
+  u32 const share = (a.ncand + CQ_BLOCKS - 1) / CQ_BLOCKS, least = BLOCK / g;
+  a.chunk = share < least ? least : share < CQ_CHUNK ? share : CQ_CHUNK;
+  dim3 grid((a.ncand + a.chunk - 1) / a.chunk);
   char const* kn = cq_name(MODE);
   auto one = [&](auto kernel) {
     if (ea) {
