@@ -352,116 +352,144 @@ static std::unique_ptr<Up> up_patch(u32 deg, Up const& old, u32 nl_old, u32 cons
 // pass write them next to the connectivity.
 
 // --------------------------------------------------------------- refine
+// the minimum over a group of G lanes (it does not depend on the order, so
+// the result is the serial loop's)
+template <u32 G>
+__device__ inline double group_min(double v) {
+#pragma unroll
+  for (u32 d = G / 2; d >= 1; d >>= 1) {
+    double o = __shfl_xor(v, d, G);
+    if (o < v) v = o;
+  }
+  return v;
+}
+
 // Worst child quality of every candidate edge split
 // (refine_qualities.cpp:16-82); rejected candidates are cleared, the others
 // become UNKNOWN: cand is then the independent set's first state, and the
 // flags of its rounds are cleared on the way.
+//
+// FP64 arithmetic bounds it, and the lanes that take part in it: with a
+// thread per edge, of which a few are candidates with rings of 3 to 12, a
+// wave ran at 8 to 12 of its 64 lanes and a small mesh's call was as long as
+// ten child qualities in a row.  A block lists the candidates of `per` edges
+// and a group of G lanes takes each, a child per lane (a ring of five tets
+// has ten).
+constexpr u32 RQ_EDGES = 1024, RQ_BLOCKS = 2048;
+
+template <u32 DIM>
+struct SplitRing {
+  V3 split;
+  Sym msplit;
+};
+
+// the child t of a split: 2 to an element of the edge's ring
+template <u32 DIM, bool F32>
+__device__ inline double split_child_q(SplitRing<DIM> const& r, u32 e, u32 dir, u32 k, u32 const* __restrict__ ve,
+                                       double const* __restrict__ x, double const* __restrict__ mt) {
+  constexpr u32 VPE = DIM + 1;
+  u32 const* bv = canon(DIM, DIM - 1, 0, opp(DIM, 0)[canon(DIM, 1, 0, dir)[k]]);
+  V3 p[VPE];
+#pragma unroll
+  for (u32 l = 0; l + 1 < VPE; ++l) p[l] = ld3(x + 3 * (size_t) ve[(size_t) e * VPE + bv[l]]);
+  p[VPE - 1] = r.split;
+  if (mt) {
+    Sym pm[VPE];
+#pragma unroll
+    for (u32 l = 0; l + 1 < VPE; ++l) pm[l] = ld6(mt + 6 * (size_t) ve[(size_t) e * VPE + bv[l]]);
+    pm[VPE - 1] = r.msplit;
+    return F32 ? (double) quality32<DIM>(p, pm, false) : metric_quality<DIM>(p, pm, false);
+  }
+  return F32 ? (double) quality32<DIM>(p, nullptr, false) : entity_quality(DIM, p);
+}
+
 template <u32 DIM, bool MIXED>
 __global__ __launch_bounds__(BLOCK) void refine_quality_f64(
-    u32 ns, u32 const* __restrict__ vs, u32 const* __restrict__ uo, u32 const* __restrict__ ua,
+    u32 ns, u32 per, u32 const* __restrict__ vs, u32 const* __restrict__ uo, u32 const* __restrict__ ua,
     u32 const* __restrict__ ud, u32 const* __restrict__ ve, double const* __restrict__ x,
     double const* __restrict__ mt, double const* __restrict__ eq, double qual_floor_all,
     double const* __restrict__ qfe, u32* __restrict__ cand, double* __restrict__ out, u32* __restrict__ words, u32 tag,
     u32* __restrict__ err, ScreenStats st) {
-  u32 i = xcd_block() * BLOCK + threadIdx.x;
-  if (i < INDSET_FLAGS) words[W_FLAGS + i] = 0;
-  if (i >= ns || !cand[i]) return;
-  // one floor for the mesh, or its component's in a batch
-  double const qual_floor = qfe ? qfe[i] : qual_floor_all;
-  constexpr u32 VPE = DIM + 1;
-  V3 a = ld3(x + 3 * (size_t) vs[2 * i]), b = ld3(x + 3 * (size_t) vs[2 * i + 1]);
-  // average_element_field (element_field.hpp:8-25): ((0 + a) + b) / 2
-  V3 split;
-  {
-    double s;
-    s = 0; s += a.x; s += b.x; s /= 2; split.x = s;
-    s = 0; s += a.y; s += b.y; s /= 2; split.y = s;
-    s = 0; s += a.z; s += b.z; s /= 2; split.z = s;
-  }
-  // the new vertex's metric is the average its field would get on refinement
-  Sym msplit;
-  if (mt) {
-    Sym ma = ld6(mt + 6 * (size_t) vs[2 * i]), mb = ld6(mt + 6 * (size_t) vs[2 * i + 1]);
-    for (int k = 0; k < 6; ++k) {
-      double s = 0;
-      s += ma.m[k];
-      s += mb.m[k];
-      s /= 2;
-      msplit.m[k] = s;
+  constexpr u32 G = 4;
+  __shared__ u32 list[RQ_EDGES], nlist;
+  if (blockIdx.x == 0 && threadIdx.x < INDSET_FLAGS) words[W_FLAGS + threadIdx.x] = 0;
+  if (threadIdx.x == 0) nlist = 0;
+  __syncthreads();
+  u32 const first = xcd_block() * per;
+  for (u32 k = threadIdx.x; k < per && first + k < ns; k += BLOCK)
+    if (cand[first + k]) list[atomicAdd(&nlist, 1u)] = first + k;
+  __syncthreads();
+  u32 const lane = threadIdx.x % G, n = nlist;
+  for (u32 c = threadIdx.x / G; c < n; c += BLOCK / G) {
+    u32 const i = list[c];
+    // one floor for the mesh, or its component's in a batch
+    double const qual_floor = qfe ? qfe[i] : qual_floor_all;
+    u32 const v0 = vs[2 * (size_t) i], v1 = vs[2 * (size_t) i + 1];
+    V3 a = ld3(x + 3 * (size_t) v0), b = ld3(x + 3 * (size_t) v1);
+    // average_element_field (element_field.hpp:8-25): ((0 + a) + b) / 2
+    SplitRing<DIM> r;
+    {
+      double s;
+      s = 0; s += a.x; s += b.x; s /= 2; r.split.x = s;
+      s = 0; s += a.y; s += b.y; s /= 2; r.split.y = s;
+      s = 0; s += a.z; s += b.z; s /= 2; r.split.z = s;
     }
-  }
-  u32 const* bo = opp(DIM, 0);
-  float minq32 = 1.f;
-  if (MIXED && !eq) {
-    // FP32 screen: a split certainly below the floor is rejected here; one
-    // with a child near zero goes to FP64, which also checks q > 0
-    bool sure = true;
-    for (u32 j = uo[i]; j < uo[i + 1]; ++j) {
-      u32 dir = ud[j], e = ua[j];
-      u32 const* evs = canon(DIM, 1, 0, dir);
-      for (u32 k = 0; k < 2; ++k) {
-        u32 const* bv = canon(DIM, DIM - 1, 0, bo[evs[k]]);
-        V3 p[VPE];
-#pragma unroll
-        for (u32 l = 0; l + 1 < VPE; ++l) p[l] = ld3(x + 3 * (size_t) ve[(size_t) e * VPE + bv[l]]);
-        p[VPE - 1] = split;
-        float q;
-        if (mt) {
-          Sym pm[VPE];
-#pragma unroll
-          for (u32 l = 0; l + 1 < VPE; ++l) pm[l] = ld6(mt + 6 * (size_t) ve[(size_t) e * VPE + bv[l]]);
-          pm[VPE - 1] = msplit;
-          q = quality32<DIM>(p, pm, false);
-        } else {
-          q = quality32<DIM>(p, nullptr, false);
-        }
-        if (!(q > SCREEN_MARGIN)) sure = false;
-        minq32 = q < minq32 ? q : minq32;
+    // the new vertex's metric is the average its field would get on refinement
+    if (mt) {
+      Sym ma = ld6(mt + 6 * (size_t) v0), mb = ld6(mt + 6 * (size_t) v1);
+      for (int k = 0; k < 6; ++k) {
+        double s = 0;
+        s += ma.m[k];
+        s += mb.m[k];
+        s /= 2;
+        r.msplit.m[k] = s;
       }
     }
-    bool reject = sure && (minq32 < (float) qual_floor - SCREEN_MARGIN);
-    wave_count(st.screened, reject);
-    if (reject) {
-      cand[i] = 0;
-      return;
-    }
-    wave_count(st.reeval, true);
-  }
-  double minq = 1, old_minq = 1;
-  for (u32 j = uo[i]; j < uo[i + 1]; ++j) {
-    u32 dir = ud[j], e = ua[j];
-    if (eq && eq[e] < old_minq) old_minq = eq[e];
-    u32 const* evs = canon(DIM, 1, 0, dir);
-    for (u32 k = 0; k < 2; ++k) {
-      u32 const* bv = canon(DIM, DIM - 1, 0, bo[evs[k]]);
-      V3 p[VPE];
-#pragma unroll
-      for (u32 l = 0; l + 1 < VPE; ++l) p[l] = ld3(x + 3 * (size_t) ve[(size_t) e * VPE + bv[l]]);
-      p[VPE - 1] = split;
-      double q;
-      if (mt) {
-        Sym pm[VPE];
-#pragma unroll
-        for (u32 l = 0; l + 1 < VPE; ++l) pm[l] = ld6(mt + 6 * (size_t) ve[(size_t) e * VPE + bv[l]]);
-        pm[VPE - 1] = msplit;
-        q = metric_quality<DIM>(p, pm, false);
-      } else {
-        q = entity_quality(DIM, p);
+    u32 const begin = uo[i], nchild = 2 * (uo[i + 1] - begin);
+    double minq32 = 1;
+    if (MIXED && !eq) {
+      // FP32 screen: a split certainly below the floor is rejected here; one
+      // with a child near zero goes to FP64, which also checks q > 0
+      bool sure = true;
+      for (u32 t = lane; t < nchild; t += G) {
+        u32 const j = begin + t / 2;
+        double const q = split_child_q<DIM, true>(r, ua[j], ud[j], t & 1u, ve, x, mt);
+        if (!(q > (double) SCREEN_MARGIN)) sure = false;
+        if (q < minq32) minq32 = q;
       }
+      minq32 = group_min<G>(minq32);
+#pragma unroll
+      for (u32 d = G / 2; d >= 1; d >>= 1) sure = __shfl_xor((int) sure, d, G) && sure;
+      bool const reject = sure && ((float) minq32 < (float) qual_floor - SCREEN_MARGIN);
+      if (lane == 0) wave_count(st.screened, reject);
+      if (reject) {
+        if (lane == 0) cand[i] = 0;
+        continue;
+      }
+      if (lane == 0) wave_count(st.reeval, true);
+    }
+    double minq = 1, old_minq = 1;
+    for (u32 t = lane; t < nchild; t += G) {
+      u32 const j = begin + t / 2, e = ua[j];
+      if (eq && eq[e] < old_minq) old_minq = eq[e];
+      double const q = split_child_q<DIM, false>(r, e, ud[j], t & 1u, ve, x, mt);
       if (!(q > 0)) *err = ERR_REFINE_QUALITY;
       if (q < minq) minq = q;
     }
-  }
-  if (MIXED && !eq && minq == minq) {
-    float d = (float) minq - minq32;
-    note_max_err(st.max_err, d < 0 ? -d : d);
-  }
-  if ((minq < qual_floor) || (eq && (minq <= old_minq)))
-    cand[i] = 0;
-  else {
-    out[i] = minq;
-    cand[i] = UNKNOWN;
-    wave_flag_value(words + W_ANY, true, tag);
+    minq = group_min<G>(minq);
+    if (eq) old_minq = group_min<G>(old_minq);
+    if (lane != 0) continue;
+    if (MIXED && !eq && minq == minq) {
+      float const d = (float) minq - (float) minq32;
+      note_max_err(st.max_err, d < 0 ? -d : d);
+    }
+    if ((minq < qual_floor) || (eq && (minq <= old_minq))) {
+      cand[i] = 0;
+    } else {
+      out[i] = minq;
+      cand[i] = UNKNOWN;
+      wave_flag_value(words + W_ANY, true, tag);
+    }
   }
 }
 
@@ -495,14 +523,18 @@ static Buf<double> refine_qualities(Mesh& m, u32* cand, double qual_floor, bool 
   // in the mixed mode the FP32 screen is a variant chosen online (it pays
   // only where it rejects enough splits); both give identical results
   static thread_local Tuner tuners[2] = {Tuner("refine_quality_2d_mixed", {0, 1}), Tuner("refine_quality_3d_mixed", {0, 1})};
+  // a block's edges: as few as fill the chip (four blocks per CU)
+  u32 per = 32;
+  while (per < RQ_EDGES && (u64) per * RQ_BLOCKS < ns) per *= 2;
+  dim3 const grid((ns + per - 1) / per);
   auto go = [&](auto kernel, char const* kn, hipEvent_t ea, hipEvent_t eb) {
     if (ea) {
-      hipExtLaunchKernelGGL(kernel, dim3(nblocks(ns)), dim3(BLOCK), 0, stream(), ea, eb, 0, ns, vs, u.offsets.get(),
+      hipExtLaunchKernelGGL(kernel, grid, dim3(BLOCK), 0, stream(), ea, eb, 0, ns, per, vs, u.offsets.get(),
                             u.adj.get(), u.dirs.get(), ve, coords(m), metric_of(m), eq.get(), qual_floor, qfe,
                             cand, out.get(), scratch_words(), tag, dev_error_word(), sst);
       check_launch(kn);
     } else {
-      launch_timed(kn, prof_bytes, kernel, dim3(nblocks(ns)), dim3(BLOCK), ns, vs, u.offsets.get(), u.adj.get(),
+      launch_timed(kn, prof_bytes, kernel, grid, dim3(BLOCK), ns, per, vs, u.offsets.get(), u.adj.get(),
                    u.dirs.get(), ve, coords(m), metric_of(m), eq.get(), qual_floor, qfe, cand, out.get(),
                    scratch_words(), tag, dev_error_word(), sst);
     }
@@ -1125,18 +1157,7 @@ static void check_exposed_sides(Mesh& m, u32 ed, u32* codes) {
 
 // coarsen_quality (coarsen_qualities.cpp:12-79)
 // G lanes per edge: the elements around the collapsing vertex are split
-// over the group and the minima combined with shuffles (a minimum does not
-// depend on the order, so the result is the serial loop's).
-template <u32 G>
-__device__ inline double group_min(double v) {
-#pragma unroll
-  for (u32 d = G / 2; d >= 1; d >>= 1) {
-    double o = __shfl_xor(v, d, G);
-    if (o < v) v = o;
-  }
-  return v;
-}
-
+// over the group
 // Modes of the collapse-quality kernel.  CQ_F64: the reference's
 // arithmetic.  CQ_SCREEN: an FP32 pass rejects the directions certainly
 // below the floor, every other direction is measured again in FP64.
