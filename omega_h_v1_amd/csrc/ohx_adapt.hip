@@ -373,9 +373,11 @@ __device__ inline double group_min(double v) {
 // thread per edge, of which a few are candidates with rings of 3 to 12, a
 // wave ran at 8 to 12 of its 64 lanes and a small mesh's call was as long as
 // ten child qualities in a row.  A block lists the candidates of `per` edges
-// and a group of G lanes takes each, a child per lane (a ring of five tets
-// has ten).
-constexpr u32 RQ_EDGES = 1024, RQ_BLOCKS = 2048;
+// and a group of four lanes takes each, a child per lane (a ring of five tets
+// has ten): a call at 55 thousand tets 187 -> 111 us, in a box of 384 thousand
+// 60 -> 35 us, at 3 thousand 23 -> 14 us (groups of 8: 218, 47 and 17 us, of
+// 2: 208, 43 and 18 us, both with a quarter of the blocks).
+constexpr u32 RQ_EDGES = 1024, RQ_BLOCKS = 4096;
 
 template <u32 DIM>
 struct SplitRing {
@@ -403,6 +405,7 @@ __device__ inline double split_child_q(SplitRing<DIM> const& r, u32 e, u32 dir, 
   return F32 ? (double) quality32<DIM>(p, nullptr, false) : entity_quality(DIM, p);
 }
 
+// per: edges per block, at most RQ_EDGES
 template <u32 DIM, bool MIXED>
 __global__ __launch_bounds__(BLOCK) void refine_quality_f64(
     u32 ns, u32 per, u32 const* __restrict__ vs, u32 const* __restrict__ uo, u32 const* __restrict__ ua,
@@ -523,7 +526,8 @@ static Buf<double> refine_qualities(Mesh& m, u32* cand, double qual_floor, bool 
   // in the mixed mode the FP32 screen is a variant chosen online (it pays
   // only where it rejects enough splits); both give identical results
   static thread_local Tuner tuners[2] = {Tuner("refine_quality_2d_mixed", {0, 1}), Tuner("refine_quality_3d_mixed", {0, 1})};
-  // a block's edges: as few as fill the chip (four blocks per CU)
+  // a block's edges: as few as fill the chip (16 blocks per CU: the
+  // candidates lie close together, and many small blocks even that out)
   u32 per = 32;
   while (per < RQ_EDGES && (u64) per * RQ_BLOCKS < ns) per *= 2;
   dim3 const grid((ns + per - 1) / per);

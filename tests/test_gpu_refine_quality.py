@@ -1,7 +1,7 @@
 """The qualities of candidate splits, listed per block of edges and measured
 by groups of lanes: one split pass with scattered candidates equals the
-oracle's, from a single element to meshes whose blocks take 32, 64 and 128
-edges, none of them a multiple of it."""
+oracle's, from a single element to meshes whose blocks take 32 and 64 edges,
+none of them a multiple of it."""
 import numpy as np
 import pytest
 
