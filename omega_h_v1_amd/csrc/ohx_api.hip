@@ -187,6 +187,7 @@ unsigned ohx_element_qualities_f64(unsigned dim, unsigned n, unsigned const* ev,
     Buf<double> q = element_qualities(dim, n, ev, x);
     d2d(out, q.get(), n);
     sync();
+    sc.drained = true;
     return 0u;
   });
 }
@@ -195,7 +196,9 @@ double ohx_min_quality_f64(unsigned dim, unsigned n, unsigned const* ev, double 
   return guard(std::numeric_limits<double>::quiet_NaN(), [&]() -> double {
     OHX_REQUIRE(dim == 2 || dim == 3, "dim must be 2 or 3");
     StreamScope sc((hipStream_t) s);
-    return min_element_quality(dim, n, ev, x);
+    double const least = min_element_quality(dim, n, ev, x);
+    sc.drained = n > 1;  // (it has read its result)
+    return least;
   });
 }
 
@@ -210,6 +213,7 @@ unsigned ohx_measure_edges_f64(unsigned ne, unsigned const* ev, double const* x,
       out[i] = len / want;
     });
     sync();
+    sc.drained = true;
     return 0u;
   });
 }
@@ -219,6 +223,7 @@ unsigned ohx_exscan_u32(unsigned const* a, unsigned n, unsigned* out, void* s) {
     StreamScope sc((hipStream_t) s);
     exscan(a, n, out);
     sync();
+    sc.drained = true;
     return 0u;
   });
 }
@@ -228,6 +233,17 @@ unsigned ohx_up_from_down(unsigned hd, unsigned ld, unsigned nh, unsigned nl, un
   return guard(OHX_ERROR, [&]() -> unsigned {
     OHX_REQUIRE(hd <= 3 && ld < hd, "bad dimensions");
     StreamScope sc((hipStream_t) s);
+    size_t const uses = (size_t) nh * h_down_deg[hd][ld];
+    // straight into the caller's arrays (240 -> 215 us for 3.6 million uses,
+    // against arrays of its own copied at the end), unless one overlaps the
+    // down map, which is read until the uses are in their buckets
+    auto apart = [&](u32 const* p, size_t n) { return p + n <= lh || lh + uses <= p; };
+    if (apart(offs, (size_t) nl + 1) && apart(adj, uses) && apart(dirs, uses)) {
+      up_from_down_into(hd, ld, nh, nl, lh, offs, adj, dirs);
+      sync();
+      sc.drained = true;
+      return 0u;
+    }
     Up u;
     up_from_down(hd, ld, nh, nl, lh, u);
     u32 nuses = nh * h_down_deg[hd][ld];
@@ -235,6 +251,7 @@ unsigned ohx_up_from_down(unsigned hd, unsigned ld, unsigned nh, unsigned nl, un
     d2d(adj, u.adj.get(), nuses);
     d2d(dirs, u.dirs.get(), nuses);
     sync();
+    sc.drained = true;
     return 0u;
   });
 }

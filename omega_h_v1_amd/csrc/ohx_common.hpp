@@ -65,11 +65,13 @@ struct StreamScope {
   // the caller's stream, which is drained at the end because the call's
   // temporaries go back to the arena, which reuses blocks in library-stream
   // order
+  // drained: the call has just synchronised the stream and launches nothing more
+  bool drained = false;
   explicit StreamScope(hipStream_t s) : prev(g_stream_override), own(s == nullptr) {
     if (s) g_stream_override = s;
   }
   ~StreamScope() {
-    (void) hipStreamSynchronize(stream());
+    if (!drained) (void) hipStreamSynchronize(stream());
     g_stream_override = prev;
   }
 };

@@ -397,7 +397,10 @@ u32* take_zeroed_counters(u32 n) {
 }
 }  // namespace
 
-void up_from_down(u32 hd, u32 ld, u32 nhighs, u32 nlows, u32 const* lows_of_highs, Up& u) {
+// own: gets arrays of its own (each made when it is written, the slots gone
+// before the last two); else offs, adj and dirs are written
+static void up_from_down_to(u32 hd, u32 ld, u32 nhighs, u32 nlows, u32 const* lows_of_highs, Up* own, u32* offs,
+                            u32* adj, u32* dirs) {
   u32 deg = h_down_deg[hd][ld];
   if ((size_t) nhighs * deg >= ((size_t) 1 << 32)) fail("up_from_down: more than 2^32 uses", __FILE__, __LINE__);
   u32 nuses = nhighs * deg;
@@ -405,7 +408,6 @@ void up_from_down(u32 hd, u32 ld, u32 nhighs, u32 nlows, u32 const* lows_of_high
   Buf<u32> slot(nuses);
   if (nuses) {
     zero_counters().dirty = true;
-    // compulsory bytes: the down map in, each counter read and written
     // compulsory bytes: the down map in, slots out, each counter read and
     // written; plain or wave-combined adds, chosen online per (high, low)
     // dimension pair and size class
@@ -431,17 +433,25 @@ void up_from_down(u32 hd, u32 ld, u32 nhighs, u32 nlows, u32 const* lows_of_high
       else go(upfd_count<false>, ea, eb);
     });
   }
-  u.offsets = exscan(counts, nlows);
+  if (own) {
+    own->offsets = Buf<u32>((size_t) nlows + 1);
+    offs = own->offsets.get();
+  }
+  exscan(counts, nlows, offs);
   Buf<u32> tmp(nuses);
   if (nuses) {
     // down map and slots in, uses out, offsets read and counters cleared
     launch_timed("upfd_fill", (double) nuses * 12 + (double) nlows * 8, upfd_fill, dim3(nblocks(nuses)),
-                 dim3(BLOCK), nuses, lows_of_highs, slot.get(), u.offsets.get(), counts, tmp.get());
+                 dim3(BLOCK), nuses, lows_of_highs, slot.get(), offs, counts, tmp.get());
     zero_counters().dirty = false;
   }
   slot.release();
-  u.adj = Buf<u32>(nuses);
-  u.dirs = Buf<u32>(nuses);
+  if (own) {
+    own->adj = Buf<u32>(nuses);
+    own->dirs = Buf<u32>(nuses);
+    adj = own->adj.get();
+    dirs = own->dirs.get();
+  }
   if (nlows && nuses) {
     // offsets, uses in, (high, direction) out; lanes per bucket (4 to 32)
     // chosen online per (high, low) dimension pair and size class
@@ -455,16 +465,15 @@ void up_from_down(u32 hd, u32 ld, u32 nhighs, u32 nlows, u32 const* lows_of_high
         {Tuner("upfd_rank_split_3_0", V), Tuner("upfd_rank_split_3_1", V), Tuner("upfd_rank_split_3_2", V),
          Tuner("-", {4})}};
     double bytes = (double) (nlows + 1) * 4 + (double) nuses * 12;
-    u32 const* o = u.offsets.get();
     auto go = [&](auto kernel, u32 g, hipEvent_t ea, hipEvent_t eb) {
       dim3 grid(nblocks((size_t) nlows * g));
       if (ea) {
-        hipExtLaunchKernelGGL(kernel, grid, dim3(BLOCK), 0, stream(), ea, eb, 0, nlows, deg, o, tmp.get(),
-                              u.adj.get(), u.dirs.get());
+        hipExtLaunchKernelGGL(kernel, grid, dim3(BLOCK), 0, stream(), ea, eb, 0, nlows, deg, offs, tmp.get(),
+                              adj, dirs);
         check_launch("upfd_rank_split");
       } else {
-        launch_timed("upfd_rank_split", bytes, kernel, grid, dim3(BLOCK), nlows, deg, o, tmp.get(), u.adj.get(),
-                     u.dirs.get());
+        launch_timed("upfd_rank_split", bytes, kernel, grid, dim3(BLOCK), nlows, deg, offs, tmp.get(), adj,
+                     dirs);
       }
     };
     tuned(tuners[hd][ld], nlows, [&](u32 g, hipEvent_t ea, hipEvent_t eb) {
@@ -478,6 +487,15 @@ void up_from_down(u32 hd, u32 ld, u32 nhighs, u32 nlows, u32 const* lows_of_high
       else go(upfd_rank_seg<64>, 64, ea, eb);
     });
   }
+}
+
+void up_from_down(u32 hd, u32 ld, u32 nhighs, u32 nlows, u32 const* lows_of_highs, Up& u) {
+  up_from_down_to(hd, ld, nhighs, nlows, lows_of_highs, &u, nullptr, nullptr, nullptr);
+}
+
+void up_from_down_into(u32 hd, u32 ld, u32 nhighs, u32 nlows, u32 const* lows_of_highs, u32* offs, u32* adj,
+                       u32* dirs) {
+  up_from_down_to(hd, ld, nhighs, nlows, lows_of_highs, nullptr, offs, adj, dirs);
 }
 
 // ---------------------------------------------------------- reflect_down

