@@ -1891,12 +1891,16 @@ __device__ inline u32 up_patch_low(UpPatch const& a, u32 u) {
   return e < a.nsame_l + a.ngen_l ? e : INVALID;
 }
 
-// each product use takes a place after its low's surviving uses
+// each product use takes a place after its low's surviving uses.  Bound by the
+// atomics' rate; the products of a cavity share their lows (the 60 edge uses of
+// ten tets around a new vertex have 22), so a wave combines its adds: a split
+// adaptation of 384 thousand tets 5.33 -> 5.18 ms, of 3 thousand 2.40 -> 2.31.
 __global__ __launch_bounds__(BLOCK) void up_patch_slot_k(UpPatch a) {
-  u32 u = xcd_block() * BLOCK + threadIdx.x;
-  if (u >= a.ngen_h * a.deg) return;
-  u32 e = up_patch_low(a, u);
-  if (e != INVALID) a.slot[u] = atomicAdd(&a.cnt[e], 1u);
+  u32 const u = xcd_block() * BLOCK + threadIdx.x;
+  bool const in = u < a.ngen_h * a.deg;
+  u32 const e = in ? up_patch_low(a, u) : INVALID;
+  u32 const s = wave_slot_add(a.cnt, e == INVALID ? 0u : e, e != INVALID);
+  if (e != INVALID) a.slot[u] = s;
 }
 
 // after the scan of the counts: groups of G lanes over the old lows write
