@@ -3760,7 +3760,7 @@ u32 swap_slivers(Mesh& m, double good_qual, u32 nlayers, double const* eq, doubl
 // of its pairs was removed in a pass after the one that made the face.
 
 // Words of a swap run (SwapRunView::words)
-enum { RW_ACC = 0, RW_AFF = 2, RW_POOL = 3, RW_FIRST = 4, RW_NEED = 5, RW_FLAGS = 8, RW_EVAL = 16, RW_WORDS = 24 };
+enum { RW_ACC = 0, RW_AFF = 2, RW_POOL = 3, RW_FIRST = 4, RW_FLAGS = 8, RW_EVAL = 16, RW_WORDS = 24 };
 // ring sizes 3 to MAX_EDGE_SWAP: the candidates to evaluate are listed by
 // ring size
 constexpr u32 RUN_RINGS = MAX_EDGE_SWAP - 2;
@@ -4358,20 +4358,6 @@ __global__ __launch_bounds__(BLOCK) void run_products_k(SwapRunView R, u32 ns, u
   R.dual[4 * (size_t) self] = first + 2 * p + x;  // the twin: the same triangle, the other end
 }
 
-// at most how many list places the surviving uses of the changed edges take
-__global__ __launch_bounds__(BLOCK) void run_need_k(SwapRunView R, u32 ns, u32* __restrict__ out) {
-  u32 const s = blockIdx.x * BLOCK + threadIdx.x;
-  u32 n = 0;
-  if (s < ns) {
-    u32 const e = R.sw[s], f = R.lb[e], l = R.ln[e];
-    for (u32 j = f; j < f + l; ++j)
-      for (u32 k = 0; k < 6; ++k) n += R.ln[R.te[6 * (size_t) R.ua[j] + k]];
-  }
-#pragma unroll
-  for (u32 d = 32; d >= 1; d >>= 1) n += (u32) __shfl_down((int) n, d, 64);
-  if ((threadIdx.x & 63u) == 0 && n) atomicAdd(out, n);
-}
-
 // every use of an edge by a product tet takes a place among its edge's
 // product uses; the edge's first one puts the edge on the list of changed
 // edges
@@ -4607,7 +4593,9 @@ struct SwapRun {
   Buf<double> q, tq, qpart;
   Buf<unsigned char> sa, sb, dead, marks, marks2;
   Buf<RunCount> part;
-  u32 nE = 0, nF = 0, nT = 0, nF0 = 0, aE = 0, aF = 0, aT = 0, pass = 0, pool = 0;
+  u32 nE = 0, nF = 0, nT = 0, nF0 = 0, aE = 0, aF = 0, aT = 0, pass = 0;
+  size_t pool = 0;  // at most so many list places are in use
+  static constexpr size_t MAX_USES = (size_t) 1 << 32;
   bool has_id = false;
   bool limit_hit = false;  // the independent set reached its round limit
   u32 got[6];
@@ -4677,6 +4665,23 @@ struct SwapRun {
     marks2 = Buf<unsigned char>(dead.size());
   }
 
+  // room for the lists of a pass that leaves so many tets: the changed edges'
+  // new lists are some of the lists of the mesh it leaves, which have 6 uses a
+  // tet (counting around the cavities instead took a wait and, as an edge was
+  // counted once for each tet that goes, found several times as many)
+  void list_room(u32 tets) {
+    size_t const want = got[4] + 6 * (size_t) tets;
+    if (want >= MAX_USES) fail("swap: more than 2^32 uses", __FILE__, __LINE__);
+    need(ua, got[4], want);
+    need(ud, got[4], want);
+  }
+  // whether the next pass could run out of places that 32 bits can number: a
+  // pass replaces a ring of 7 tets with 10 at most, so its lists take fewer
+  // than 9 places for each tet before it.  Lists in use take 6 a tet, and
+  // check_index_space keeps a mesh below 2^32 / 36 tets: with the gaps closed
+  // there is always room.
+  bool lists_full() const { return pool + 9 * (size_t) aT >= MAX_USES; }
+
   SwapRunView view() const {
     SwapRunView R{};
     R.nE = nE;
@@ -4726,7 +4731,7 @@ struct SwapRun {
     nT = aT = count(m, 3);
     pass = 0;
     pool = u.adj.size();
-    size_t const cE = room(nE), cF = room(nF), cT = room(nT), cL = 2 * (size_t) pool + pool / 4 + 4096;
+    size_t const cE = room(nE), cF = room(nF), cT = room(nT), cL = 2 * pool + pool / 4 + 4096;
     ev = taken(ask_down(m, 1, 0), 2 * (size_t) nE, 2 * cE);
     ecd = taken(u32_tag(m, 1, "class_dim"), nE, cE);
     vt = taken(ask_down(m, 3, 0), 4 * (size_t) nT, 4 * cT);
@@ -4765,7 +4770,7 @@ struct SwapRun {
     // their room) and the tets
     SwapRunView R = view();
     u32 const* off = u.offsets.get();
-    u32 const p0 = pool, ns = (u32) states;
+    u32 const p0 = (u32) pool, ns = (u32) states;
     parallel_for(ns > nT ? ns : nT, OHX_LAMBDA(u32 i) {
       if (i < ns) {
         R.sa[i] = 0;
@@ -4988,13 +4993,16 @@ struct SwapRun {
 
   void swap(SwapRunView R, unsigned char const* state, u32 nb) {
     u32 const ns = got[0], n1 = got[1], n2 = got[2], n3 = got[3];
-    if (6 * ((size_t) nT + n3) >= ((size_t) 1 << 32)) fail("swap: more than 2^32 uses", __FILE__, __LINE__);
+    if (6 * ((size_t) nT + n3) >= MAX_USES) fail("swap: more than 2^32 uses", __FILE__, __LINE__);
     edge_room(nE + n1);
     tet_room(nT + n3);
     need(fv, 3 * (size_t) nF, 3 * ((size_t) nF + n2));
     need(fcd, nF, (size_t) nF + n2);
     if (has_id) need(fci, nF, (size_t) nF + n2);
     need(fbirth, nF - nF0, (size_t) nF - nF0 + n2);
+    // a ring of rs tets and faces goes, 2 (rs - 2) tets come
+    u32 const ring = n3 / 2 + 2 * ns;
+    list_room(aT + n3 - ring);
     Buf<u32> lists((size_t) 4 * ns), uses((size_t) 12 * n3), deferred((size_t) 4 * n3);
     // the states may have moved: the round's result is in sa or sb as before
     bool const in_a = state == R.sa;
@@ -5008,24 +5016,6 @@ struct SwapRun {
     u32 *slot = uses.get(), *changed = slot + nuse;
     hipLaunchKernelGGL(run_list_k, dim3(nb), dim3(BLOCK), 0, stream(), R, state, part.get());
     check_launch("run_list");
-    // the changed edges' lists: their product uses, and no more surviving
-    // uses than all lists have; only where the pool has not that much room
-    // left are the lists around the cavities counted (one more wait)
-    u32 const used = got[4];
-    if (ua.size() < (size_t) used + 6 * (size_t) aT + nuse) {
-      u32* word = words.get() + RW_NEED;
-      hipLaunchKernelGGL(run_need_k, dim3(nblocks(ns)), dim3(BLOCK), 0, stream(), R, ns, word);
-      check_launch("run_need");
-      u32 const* wp = word;
-      u32 bound;
-      read_many(&wp, 1, &bound);
-      size_t const want = (size_t) used + bound + nuse;
-      if (want >= ((size_t) 1 << 32)) fail("swap: more than 2^32 uses", __FILE__, __LINE__);
-      need(ua, used, want);
-      need(ud, used, want);
-      R.ua = ua.get();
-      R.ud = ud.get();
-    }
     launch_timed("swap_cavity", (double) n1 * 8 + (double) n2 * 12 + (double) n3 * 16 + (double) ns * 12,
                  run_products_k, dim3(nblocks((size_t) ns * RUN_G)), dim3(BLOCK), R, ns, face_prod.get(),
                  deferred.get(), dev_error_word());
@@ -5040,11 +5030,10 @@ struct SwapRun {
     nE += n1;
     nF += n2;
     nT += n3;
-    // a ring of rs tets and faces goes, 2 (rs - 2) tets come
-    u32 const ring = n3 / 2 + 2 * ns;
     aE = aE + n1 - ns;
     aF = aF + n2 - ring;
     aT = aT + n3 - ring;
+    pool = got[4] + 6 * (size_t) aT;
   }
 };
 }  // namespace
@@ -5193,7 +5182,7 @@ bool swap_passes(Mesh& m, Ctx& c, double good_qual, u32 nlayers, Buf<double>& eq
     }
     // more gaps than tets: close them, so that what each pass reads of the
     // whole mesh stays below twice the mesh
-    if (run.nT - run.aT > run.aT) {
+    if (run.nT - run.aT > run.aT || run.lists_full()) {
       Buf<u32> known;
       Buf<double> values;
       run.finish(eq, &known, &values);

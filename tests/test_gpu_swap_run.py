@@ -84,6 +84,38 @@ def test_swap_run_over_every_ring_size(libs, n, before):
     assert same(a, b) is None
 
 
+@pytest.mark.parametrize("n", [2, 3, 4])
+@pytest.mark.parametrize("more", [0, 1])
+def test_a_run_waits_once_per_pass(libs, n, more):
+    """The room a pass's new lists need follows from the numbers the host has:
+    a run costs the host one wait for each pass and one at its end, also where
+    a pass's lists need new room (both passes here whose sets settle at once).
+    The size passes before the run are those of the same mesh with its own
+    least quality for the good one, which needs no swap."""
+    lib = libs[0]
+    dll = lib.dll
+    dll.ohx_profile_get.argtypes = [C.c_char_p] + 3 * [C.c_void_p]
+    m = front(lib, n, 0.16)
+    m.adapt(max_ops=1000)
+
+    def waits(good, ops):
+        c = m.clone()
+        ms, k = C.c_double(), C.c_ulonglong()
+        dll.ohx_profile_enable(1)
+        try:
+            dll.ohx_profile_reset()
+            _, stats = c.adapt_timed(good_qual=good, max_ops=ops)
+            dll.ohx_profile_get(b"host_sync", C.byref(ms), C.byref(k), None)
+        finally:
+            dll.ohx_profile_enable(0)
+        return k.value, int(stats[0])
+
+    none, before = waits(m.min_quality(), 1000)
+    run, passes = waits(0.9, before + more)
+    assert passes == before + 2 + more
+    assert run - none == passes - before + 1
+
+
 def test_round_limit_inside_a_swap_run(libs):
     """A run whose independent set reaches the round limit fails as a pass
     over a whole mesh does, and leaves the mesh of the passes before."""
