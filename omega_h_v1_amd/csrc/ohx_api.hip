@@ -228,17 +228,30 @@ unsigned ohx_exscan_u32(unsigned const* a, unsigned n, unsigned* out, void* s) {
   });
 }
 
+// whether kernels may write here: memory of this GPU.  Host memory, which the
+// runtime copies to, would be a fault for a kernel.
+static bool on_this_gpu(void const* p) {
+  hipPointerAttribute_t a{};
+  if (hipPointerGetAttributes(&a, p) != hipSuccess) {
+    (void) hipGetLastError();
+    return false;
+  }
+  return a.type == hipMemoryTypeDevice && a.device == rt().device;
+}
+
 unsigned ohx_up_from_down(unsigned hd, unsigned ld, unsigned nh, unsigned nl, unsigned const* lh,
                           unsigned* offs, unsigned* adj, unsigned* dirs, void* s) {
   return guard(OHX_ERROR, [&]() -> unsigned {
     OHX_REQUIRE(hd <= 3 && ld < hd, "bad dimensions");
     StreamScope sc((hipStream_t) s);
     size_t const uses = (size_t) nh * h_down_deg[hd][ld];
+    OHX_REQUIRE(offs && (!uses || (adj && dirs)), "an output array is missing");
     // straight into the caller's arrays (243 -> 222 us for 3.6 million uses,
     // against arrays of its own copied at the end), unless one overlaps the
-    // down map, which is read until the uses are in their buckets
-    auto apart = [&](u32 const* p, size_t n) { return p + n <= lh || lh + uses <= p; };
-    if (apart(offs, (size_t) nl + 1) && apart(adj, uses) && apart(dirs, uses)) {
+    // down map, which is read until the uses are in their buckets, or is not
+    // this GPU's memory, where the copy decides
+    auto direct = [&](u32* p, size_t n) { return !n || ((p + n <= lh || lh + uses <= p) && on_this_gpu(p)); };
+    if (direct(offs, (size_t) nl + 1) && direct(adj, uses) && direct(dirs, uses)) {
       up_from_down_into(hd, ld, nh, nl, lh, offs, adj, dirs);
       sync();
       sc.drained = true;

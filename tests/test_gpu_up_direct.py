@@ -1,6 +1,7 @@
 """Upward adjacency written straight into the caller's arrays, from down maps
-whose lows lie close together, far apart, and both in a wave; and where an output
-array is the down map itself."""
+whose lows lie close together, far apart, and both in a wave; where an output
+array is the down map itself, or is host memory, which the runtime copies to;
+and no output array at all, which is refused."""
 import numpy as np
 import pytest
 
@@ -41,3 +42,35 @@ def test_up_from_down_into(lib, dev, kind, hd, ld, nhighs, nlows, into):  # noqa
     assert np.array_equal(dev.get(po, nlows + 1, np.uint32), want)
     assert np.array_equal(dev.get(pa, len(lows), np.uint32), (order // deg).astype(np.uint32))
     assert np.array_equal(dev.get(pd, len(lows), np.uint32), (order % deg).astype(np.uint32))
+
+
+def small():
+    lows = np.array([[0, 1, 2, 3], [1, 2, 3, 4]], dtype=np.uint32)
+    order = np.argsort(lows.ravel(), kind="stable")
+    offs = np.concatenate([[0], np.cumsum(np.bincount(lows.ravel(), minlength=5))])
+    return lows, [a.astype(np.uint32) for a in (offs, order // 4, order % 4)]
+
+
+@pytest.mark.parametrize("on_host", [(0,), (1,), (2,), (0, 1, 2)])
+def test_up_from_down_into_host_memory(lib, dev, on_host):  # noqa: F811
+    lows, want = small()
+    p = dev.put(lows)
+    host = [np.zeros(len(w), np.uint32) for w in want]
+    out = [host[k].ctypes.data if k in on_host else dev.empty(len(want[k]), np.uint32) for k in range(3)]
+    assert lib.ohx_up_from_down(3, 0, 2, 5, p, *out, None) == 0
+    for k in range(3):
+        got = host[k] if k in on_host else dev.get(out[k], len(want[k]), np.uint32)
+        assert np.array_equal(got, want[k])
+
+
+@pytest.mark.parametrize("missing", [0, 1, 2])
+def test_up_from_down_without_an_output_array(lib, dev, missing):  # noqa: F811
+    lows, want = small()
+    p = dev.put(lows)
+    out = [None if k == missing else dev.empty(len(want[k]), np.uint32) for k in range(3)]
+    assert lib.ohx_up_from_down(3, 0, 2, 5, p, *out, None) == 0xFFFFFFFF
+    assert lib.ohx_last_error()
+    # no uses: only the offsets are written
+    if missing:
+        assert lib.ohx_up_from_down(3, 0, 0, 5, p, out[0], None, None, None) == 0
+        assert not dev.get(out[0], 6, np.uint32).any()
