@@ -289,6 +289,9 @@ int ohx_profile_get(char const* name, double* ms, unsigned long long* launches,
 unsigned ohx_profile_names(char* buf, unsigned cap) OSH_PUBLIC;
 unsigned long long ohx_device_bytes_high_water(void) OSH_PUBLIC;
 void ohx_device_reset_high_water(void) OSH_PUBLIC;
+/* refuse device memory beyond this many bytes in use, as where the device has
+ * no more (0, the default: no limit): the call that asks for it fails */
+void ohx_set_device_bytes_limit(unsigned long long bytes) OSH_PUBLIC;
 void ohx_synchronize(void) OSH_PUBLIC;
 /* interior-edge table of the swap triangulations (edge_swap_edges.cpp) */
 unsigned ohx_swap_nint_edges(unsigned ring_size) OSH_PUBLIC;

@@ -4931,7 +4931,6 @@ struct SwapRun {
     }, fr.get());
     Mesh mo(3, true);
     set_ents(mo, 0, m.counts[0], Buf<u32>());
-    mo.tags[0] = std::move(m.tags[0]);
     u32 const alive[4] = {0, aE, aF, aT};
     Buf<u32> lens(aE), nd31((size_t) 6 * aT), ndual((size_t) 4 * aT);
     Buf<double> neq(aT);
@@ -4987,6 +4986,8 @@ struct SwapRun {
     mo.up[1][3] = std::move(up);
     mo.down[3][1] = std::move(nd31);
     mo.dual = std::move(ndual);
+    // nothing below fails: until here m is the mesh the run began with
+    mo.tags[0] = std::move(m.tags[0]);
     overwrite(m, std::move(mo));
     eq = std::move(neq);
   }

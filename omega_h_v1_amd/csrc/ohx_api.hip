@@ -804,6 +804,7 @@ unsigned ohx_profile_names(char* buf, unsigned cap) {
 }
 unsigned long long ohx_device_bytes_high_water(void) { return dev_bytes_high_water(); }
 void ohx_device_reset_high_water(void) { dev_reset_high_water(); }
+void ohx_set_device_bytes_limit(unsigned long long bytes) { dev_limit(bytes); }
 void ohx_synchronize(void) {
   guard_void([&]() { sync(); });
 }

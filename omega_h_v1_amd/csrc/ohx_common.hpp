@@ -110,6 +110,9 @@ void dev_free(void* p);
 size_t dev_bytes_in_use();
 size_t dev_bytes_high_water();
 void dev_reset_high_water();
+// allocations that would bring the bytes in use above this fail, as where the
+// device has no more (0: no limit)
+void dev_limit(size_t bytes);
 void dev_trim();
 
 template <class T>

@@ -197,7 +197,7 @@ struct Arena {
   std::mutex mu;
   std::vector<std::unique_ptr<StreamFree>> free_by_stream;
   LiveTable live;
-  size_t in_use = 0, high = 0, cached = 0;
+  size_t in_use = 0, high = 0, cached = 0, limit = 0;
   StreamFree& of(hipStream_t s) {
     for (auto& f : free_by_stream)
       if (f->s == s) return *f;
@@ -226,6 +226,7 @@ void* dev_alloc(size_t bytes) {
   void* p = nullptr;
   {
     std::lock_guard<std::mutex> lock(a.mu);
+    if (a.limit && a.in_use + c > a.limit) fail("device memory limit reached", __FILE__, __LINE__);
     std::vector<void*>& fl = a.of(s).lists[k];
     if (!fl.empty()) {
       p = fl.back();
@@ -292,6 +293,10 @@ size_t dev_bytes_in_use() {
 size_t dev_bytes_high_water() {
   std::lock_guard<std::mutex> lock(arena().mu);
   return arena().high;
+}
+void dev_limit(size_t bytes) {
+  std::lock_guard<std::mutex> lock(arena().mu);
+  arena().limit = bytes;
 }
 void dev_reset_high_water() {
   std::lock_guard<std::mutex> lock(arena().mu);

@@ -43,6 +43,32 @@ def front(lib, n, jitter):
     return m
 
 
+def rough(lib, n, jitter):
+    """A box of badly shaped tets that are of the desired size: the shape
+    loop, which starts with a swap run, is all there is to do."""
+    x, c = ML.box(3, n)
+    inner = ((x > 0) & (x < 1)).all(1)
+    x = x + (np.random.default_rng(n).random(x.shape) - 0.5) * (jitter / n) * inner[:, None]
+    m = ML.Mesh(lib, 3, x, c)
+    m.derive_model_full()
+    m.add_field(0, "adapt_size", W.uniform_size(m.count(0), 10.0))
+    return m
+
+
+ROUGH = {"size_floor": 0.0, "good_qual": 0.6}
+
+
+def after_each_operation(m):
+    """The mesh, and what adapting leaves of it at every operation limit."""
+    got = [m]
+    for ops in range(1000):
+        c = m.clone()
+        end = c.adapt(max_ops=ops, **ROUGH) != -1
+        got.append(c)
+        if end:
+            return got
+
+
 def same(a, b):
     return P.diff_states(a, b)
 
@@ -136,3 +162,42 @@ def test_round_limit_inside_a_swap_run(libs):
         assert same(left[0], left[1]) is None
     finally:
         lib.dll.ohx_set_indset_max_rounds(ROUNDS)
+
+
+@pytest.fixture
+def memory(libs):
+    dll = libs[0].dll
+    dll.ohx_device_bytes_high_water.restype = C.c_ulonglong
+    dll.ohx_set_device_bytes_limit.argtypes = [C.c_ulonglong]
+    yield dll
+    dll.ohx_set_device_bytes_limit(0)
+
+
+@pytest.mark.parametrize("n,jitter", [(3, 0.8), (8, 0.5)])
+def test_a_run_out_of_memory_leaves_a_mesh(libs, memory, n, jitter):
+    """Wherever device memory runs out, the mesh is that of the passes before
+    or an earlier one, whole."""
+    m = rough(libs[0], n, jitter)
+    left = after_each_operation(m)
+    assert len(left) > 4
+
+    def adapt(limit):
+        c = m.clone()
+        memory.ohx_device_reset_high_water()
+        start = memory.ohx_device_bytes_high_water()
+        memory.ohx_set_device_bytes_limit(start + limit if limit else 0)
+        try:
+            c.adapt(**ROUGH)
+            return c, memory.ohx_device_bytes_high_water() - start, False
+        except RuntimeError as e:
+            assert "limit" in str(e)
+            return c, 0, True
+        finally:
+            memory.ohx_set_device_bytes_limit(0)
+
+    _, peak, failed = adapt(0)
+    assert not failed
+    for k in range(1, 64):
+        c, _, failed = adapt(peak * k // 64)
+        assert failed
+        assert any(c.counts() == p.counts() and same(c, p) is None for p in left)
