@@ -3759,8 +3759,10 @@ u32 swap_slivers(Mesh& m, double good_qual, u32 nlayers, double const* eq, doubl
 // hash table with the last pass that removed it, and a face is gone if one
 // of its pairs was removed in a pass after the one that made the face.
 
-// Words of a swap run (SwapRunView::words)
-enum { RW_ACC = 0, RW_AFF = 2, RW_POOL = 3, RW_FIRST = 4, RW_FLAGS = 8, RW_EVAL = 16, RW_WORDS = 24 };
+// Words of a swap run (SwapRunView::words).  RW_ERR: the error code of a
+// kernel that changes the run's mesh, which is then of no use; an error found
+// while a pass is only decided goes into the error word of every sync().
+enum { RW_ACC = 0, RW_AFF = 2, RW_POOL = 3, RW_FIRST = 4, RW_ERR = 5, RW_FLAGS = 8, RW_EVAL = 16, RW_WORDS = 24 };
 // ring sizes 3 to MAX_EDGE_SWAP: the candidates to evaluate are listed by
 // ring size
 constexpr u32 RUN_RINGS = MAX_EDGE_SWAP - 2;
@@ -3853,7 +3855,8 @@ __global__ __launch_bounds__(BLOCK) void run_slivers_k(SwapRunView R, double con
                                                        unsigned char* __restrict__ marks,
                                                        double* __restrict__ part) {
   __shared__ double lds[BLOCK / 64];
-  if (blockIdx.x == 0 && threadIdx.x < RW_WORDS && threadIdx.x != RW_POOL && threadIdx.x != RW_FIRST)
+  if (blockIdx.x == 0 && threadIdx.x < RW_WORDS && threadIdx.x != RW_POOL && threadIdx.x != RW_FIRST &&
+      threadIdx.x != RW_ERR)
     R.words[threadIdx.x] = 0;
   u32 const first = R.words[RW_FIRST];
   double v = 1.7976931348623157e308;
@@ -4122,7 +4125,8 @@ __global__ __launch_bounds__(BLOCK) void run_count_k(SwapRunView R, unsigned cha
 }
 
 // one block: the blocks' totals become their first products, and the totals,
-// the pool's top, the set's flag and the quality minimum go to the host
+// the pool's top, the set's flag, the run's error and the quality minimum go
+// to the host
 __global__ __launch_bounds__(1024) void run_offsets_k(u32 nb, RunCount* __restrict__ part, u32 npart,
                                                       double const* __restrict__ qpart, SwapRunView R,
                                                       u32 const* __restrict__ flag, u32* __restrict__ host,
@@ -4156,6 +4160,7 @@ __global__ __launch_bounds__(1024) void run_offsets_k(u32 nb, RunCount* __restri
   for (u32 k = 0; k < 4; ++k) host[k] = tot.v[k];
   host[4] = R.words[RW_POOL];
   host[5] = *flag;
+  host[6] = R.words[RW_ERR];
   *host_min = v;
 }
 
@@ -4597,8 +4602,8 @@ struct SwapRun {
   size_t pool = 0;  // at most so many list places are in use
   static constexpr size_t MAX_USES = (size_t) 1 << 32;
   bool has_id = false;
-  bool limit_hit = false;  // the independent set reached its round limit
-  u32 got[6];
+  bool intact = true;  // the mesh in the arrays is that of the passes so far
+  u32 got[7];
   double min_q = 0;
 
   explicit SwapRun(Mesh& mesh) : m(mesh) {}
@@ -4833,8 +4838,18 @@ struct SwapRun {
       hipLaunchKernelGGL(run_offsets_k, dim3(1), dim3(1024), 0, stream(), nb, part.get(), rb, qpart.get(), R, flag,
                          ds, dev_slot<double>(SLOT_RUN_MIN));
       check_launch("run_offsets");
-      sync();
-      for (u32 k = 0; k < 6; ++k) got[k] = hs[k];
+      hs[6] = 0;
+      try {
+        sync();
+      } catch (Error const&) {
+        intact = !hs[6];
+        throw;
+      }
+      for (u32 k = 0; k < 7; ++k) got[k] = hs[k];
+      if (got[6]) {
+        intact = false;
+        fail_device(got[6]);
+      }
     };
     totals();
     min_q = *host_slot<double>(SLOT_RUN_MIN);
@@ -4889,14 +4904,26 @@ struct SwapRun {
         return;
       }
     }
-    limit_hit = true;
     fail("independent set did not converge within the round limit (indset.cpp:107-116)", __FILE__, __LINE__);
   }
 
   // the run's mesh, gaps closed, becomes m; eq its element qualities, and
   // known and values (when wanted) its edges' words and values
   void finish(Buf<double>& eq, Buf<u32>* known, Buf<double>* values) {
-    sync();  // an error of the last pass's kernels shows here, before its output is followed
+    // an error of the last pass's kernels shows here, before its output is followed
+    u32 const* err = words.get() + RW_ERR;
+    u32 code;
+    read_many(&err, 1, &code);
+    if (code) fail_device(code);
+    // what only the passes need goes first, and the maps of the mesh that
+    // goes: there is room then also where a pass found too little
+    for (auto* b : {&face_prod, &acc, &eval, &cnt}) b->release();
+    for (auto* b : {&sa, &sb, &marks, &marks2}) b->release();
+    part.release();
+    qpart.release();
+    m.up[1][3].reset();
+    m.down[3][1].release();
+    m.dual.release();
     SwapRunView R = view();
     Buf<u32> er(nE + 1), tr(nT + 1), fr(nF + 1);
     exscan_fn(nE, OHX_LAMBDA(u32 i) { return R.death[i] ? 0u : 1u; }, er.get());
@@ -5015,19 +5042,21 @@ struct SwapRun {
     R.o3 = R.o2 + ns;
     u32 const nuse = 6 * n3;
     u32 *slot = uses.get(), *changed = slot + nuse;
+    intact = false;  // until the pass is whole
     hipLaunchKernelGGL(run_list_k, dim3(nb), dim3(BLOCK), 0, stream(), R, state, part.get());
     check_launch("run_list");
     launch_timed("swap_cavity", (double) n1 * 8 + (double) n2 * 12 + (double) n3 * 16 + (double) ns * 12,
                  run_products_k, dim3(nblocks((size_t) ns * RUN_G)), dim3(BLOCK), R, ns, face_prod.get(),
-                 deferred.get(), dev_error_word());
+                 deferred.get(), R.words + RW_ERR);
     element_qualities_into(3, n3, R.vt + 4 * (size_t) nT, coords(m), 0, metric_of(m), tq.get() + nT);
     hipLaunchKernelGGL(run_touch_k, dim3(nblocks(nuse, RUN_AT)), dim3(RUN_AB), 0, stream(), R, nuse, slot, changed);
     hipLaunchKernelGGL(run_lists_k, dim3(nblocks(nuse, RUN_AB)), dim3(RUN_AB), 0, stream(), R, changed);
     hipLaunchKernelGGL(run_place_k, dim3(nblocks(nuse)), dim3(BLOCK), 0, stream(), R, nuse, slot);
     hipLaunchKernelGGL(run_sort_k, dim3(nblocks(nuse)), dim3(BLOCK), 0, stream(), R, changed);
     hipLaunchKernelGGL(run_settle_k, dim3(nblocks(4 * (size_t) n3)), dim3(BLOCK), 0, stream(), R, n3,
-                       face_prod.get(), deferred.get(), dev_error_word());
+                       face_prod.get(), deferred.get(), R.words + RW_ERR);
     check_launch("run_settle");
+    intact = true;
     nE += n1;
     nF += n2;
     nT += n3;
@@ -5166,9 +5195,14 @@ bool swap_passes(Mesh& m, Ctx& c, double good_qual, u32 nlayers, Buf<double>& eq
     try {
       ok = run.step(good_qual, nlayers);
     } catch (Error const&) {
-      // the round limit leaves the mesh of the passes before, as the pass
-      // through a whole mesh does
-      if (run.limit_hit && changed) run.finish(eq, nullptr, nullptr);
+      // a pass that fails before it changes anything leaves the mesh of the
+      // passes before, as the pass through a whole mesh does
+      if (run.intact && changed) {
+        try {
+          run.finish(eq, nullptr, nullptr);
+        } catch (Error const&) {  // the pass's own error is the one to report
+        }
+      }
       throw;
     }
     c.stop(t, ok);

@@ -31,6 +31,8 @@ struct Error : std::runtime_error {
 };
 
 void fail(char const* what, char const* file, int line);
+// the failure a device error code stands for
+void fail_device(unsigned code);
 #define OHX_CHECK(x)                                                       \
   do {                                                                     \
     hipError_t e_ = (x);                                                   \

@@ -62,6 +62,8 @@ static char const* dev_error_text(unsigned e) {
   return "unknown device error";
 }
 
+void fail_device(unsigned code) { fail(dev_error_text(code), __FILE__, __LINE__); }
+
 #ifdef OHX_TRACE_SYNC
 }  // namespace ohx
 #include <execinfo.h>
@@ -90,7 +92,7 @@ void sync() {
   if (*e) {
     unsigned code = *e;
     *e = 0;
-    fail(dev_error_text(code), __FILE__, __LINE__);
+    fail_device(code);
   }
 }
 

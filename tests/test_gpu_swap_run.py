@@ -164,6 +164,27 @@ def test_round_limit_inside_a_swap_run(libs):
         lib.dll.ohx_set_indset_max_rounds(ROUNDS)
 
 
+def test_device_error_inside_a_swap_run(libs):
+    """Inverted tets, around which swaps leave an edge whose tets do not close
+    a ring: the pass that meets it fails, and the swap passes before it stay,
+    as with passes over a whole mesh."""
+    left = []
+    for whole in (False, True):
+        m = rough(libs[0], 8, 0.8)
+        assert m.min_quality() < 0
+        before = m.clone()
+        if whole:
+            m.add_field(3, "mass", np.ones(m.count(3)), transfer=P.CONSERVE)
+        with pytest.raises(RuntimeError, match="find_edge_ring"):
+            m.adapt(**ROUGH)
+        if whole:
+            m.free_field(3, "mass")
+        left.append(m)
+    assert same(left[0], left[1]) is None
+    # swaps only: the vertices are the same, the tets are not
+    assert left[0].count(0) == before.count(0) and left[0].count(3) != before.count(3)
+
+
 @pytest.fixture
 def memory(libs):
     dll = libs[0].dll
