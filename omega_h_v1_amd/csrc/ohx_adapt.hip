@@ -5081,7 +5081,7 @@ struct Ctx {
   // before it to the end of its own, host waits included)
   struct Timed {
     hipEvent_t a, b;
-    double tin;
+    double tin;  // input elements, or less than 0: part of the passes, but no pass
   };
   std::vector<Timed> timed;
   std::vector<hipEvent_t> pool;
@@ -5119,8 +5119,10 @@ struct Ctx {
     for (Timed& t : timed) {
       float ms = 0;
       OHX_CHECK(hipEventElapsedTime(&ms, t.a, t.b));
-      st.npass += 1;
-      st.nelems += t.tin;
+      if (t.tin >= 0) {
+        st.npass += 1;
+        st.nelems += t.tin;
+      }
       st.tpass += ms * 1e-3;
       pool.push_back(t.a);
       pool.push_back(t.b);
@@ -5186,11 +5188,12 @@ bool swap_run_fits(Mesh& m) {
 // Returns whether the operation limit was reached.
 bool swap_passes(Mesh& m, Ctx& c, double good_qual, u32 nlayers, Buf<double>& eq, bool* good_now) {
   SwapRun run(m);
-  run.begin(eq.get(), nullptr, nullptr);
   bool changed = false, limited = false;
   *good_now = false;
+  // copying the mesh is part of the first pass, closing the gaps of them all
+  Ctx::Timed t = c.start(count(m, 3));
+  run.begin(eq.get(), nullptr, nullptr);
   for (;;) {
-    Ctx::Timed const t = c.start(run.aT);
     bool ok;
     try {
       ok = run.step(good_qual, nlayers);
@@ -5218,14 +5221,21 @@ bool swap_passes(Mesh& m, Ctx& c, double good_qual, u32 nlayers, Buf<double>& eq
     // more gaps than tets: close them, so that what each pass reads of the
     // whole mesh stays below twice the mesh
     if (run.nT - run.aT > run.aT || run.lists_full()) {
+      Ctx::Timed const gaps = c.start(-1);
       Buf<u32> known;
       Buf<double> values;
       run.finish(eq, &known, &values);
       run.begin(eq.get(), known.get(), values.get());
+      c.stop(gaps, true);
       changed = false;
     }
+    t = c.start(run.aT);
   }
-  if (changed) run.finish(eq, nullptr, nullptr);
+  if (changed) {
+    Ctx::Timed const gaps = c.start(-1);
+    run.finish(eq, nullptr, nullptr);
+    c.stop(gaps, true);
+  }
   return limited;
 }
 }  // namespace
