@@ -948,45 +948,85 @@ static Buf<u32> dual_from_sides(Mesh& m) {
 // The same dual, unique in a conforming mesh (at most two elements per
 // side), by pairing the elements' sides in a hash table keyed by the sorted
 // side vertices: the first of a pair takes a slot, the second finds it and
-// writes both entries; sides without a partner stay INVALID, and a third
-// element on a side is the error that element_dual_from_verts (dual.cpp:40-98)
-// makes it.  It needs neither the sides' numbering (down(dim, dim - 1)) nor
-// their upward map, which a pass that only wants the dual would otherwise
-// build.  A mesh without sides takes it too: walking the vertices' element
-// lists together, as dual.cpp does, is a serial chain of about 70 dependent
-// reads per side (663,552 tets: 652 us, against 174 us).
+// writes both entries; sides without a partner stay INVALID.  A third element
+// on a side is told: without sides it is the error that
+// element_dual_from_verts (dual.cpp:40-98) makes it (crowd is the error
+// word), with sides the answer is that of element_dual_from_sides, an
+// element's lowest other one, from dual_crowded_k.  It needs neither the
+// sides' numbering (down(dim, dim - 1)) nor their upward map, which a pass
+// that only wants the dual would otherwise build.  A mesh without sides takes
+// it too: walking the vertices' element lists together, as dual.cpp does, is a
+// serial chain of about 70 dependent reads per side (663,552 tets: 652 us,
+// against 174 us).
+template <u32 DIM>
+__device__ inline void side_key(u32 const* __restrict__ ev, u32 t, u32 (&key)[DIM]) {
+  u32 const* sc = canon(DIM, DIM - 1, 0, t % (DIM + 1));
+#pragma unroll
+  for (u32 k = 0; k < DIM; ++k) key[k] = ev[(size_t) (t / (DIM + 1)) * (DIM + 1) + sc[k]];
+  sort_small(key);
+}
 template <u32 DIM>
 __global__ __launch_bounds__(BLOCK) void dual_pairs_k(u32 nsides, u32 const* __restrict__ ev, u32 mask,
                                                       u32* __restrict__ table, u32* __restrict__ dual,
-                                                      u32* __restrict__ err) {
+                                                      u32* __restrict__ crowd) {
   u32 t = xcd_block() * BLOCK + threadIdx.x;
   if (t >= nsides) return;
-  constexpr u32 VPE = DIM + 1, SPE = DIM + 1;
-  u32 const i = t / SPE, j = t % SPE;
-  u32 const* sc = canon(DIM, DIM - 1, 0, j);
+  constexpr u32 SPE = DIM + 1;
+  u32 const i = t / SPE;
   u32 key[DIM];
-#pragma unroll
-  for (u32 k = 0; k < DIM; ++k) key[k] = ev[(size_t) i * VPE + sc[k]];
-  sort_small(key);
+  side_key<DIM>(ev, t, key);
   u32 h = tuple_hash(key, mask);
   for (u32 probe = 0; probe <= mask; ++probe) {
     u32 prev = atomicCAS(&table[h], INVALID, t);
     if (prev == INVALID) return;  // first of its pair: the partner writes both
-    u32 pi = prev / SPE;
-    u32 const* pc = canon(DIM, DIM - 1, 0, prev % SPE);
     u32 pk[DIM];
-#pragma unroll
-    for (u32 k = 0; k < DIM; ++k) pk[k] = ev[(size_t) pi * VPE + pc[k]];
-    sort_small(pk);
+    side_key<DIM>(ev, prev, pk);
     bool same = true;
 #pragma unroll
     for (u32 k = 0; k < DIM; ++k) same = same && pk[k] == key[k];
     if (same) {
-      dual[t] = pi;
-      if (atomicExch(&dual[prev], i) != INVALID) *err = ERR_DUAL_NONMANIFOLD;  // a third element
+      dual[t] = prev / SPE;
+      if (atomicExch(&dual[prev], i) != INVALID) *crowd = ERR_DUAL_NONMANIFOLD;  // a third element
       return;
     }
     h = (h + 1) & mask;
+  }
+}
+
+// where a side has more than two elements (*crowd is set; else nothing to do,
+// which is the common case: one block looks): every element's side takes a slot
+// of its own, and each looks for the lowest other one of its side
+template <u32 DIM>
+__global__ __launch_bounds__(1024) void dual_crowded_k(u32 nsides, u32 const* __restrict__ ev, u32 mask, u32* table,
+                                                       u32* __restrict__ dual, u32 const* crowd) {
+  if (*crowd == INVALID) return;
+  constexpr u32 SPE = DIM + 1;
+  for (size_t h = threadIdx.x; h <= mask; h += 1024) table[h] = INVALID;
+  __threadfence();
+  __syncthreads();
+  for (u32 t = threadIdx.x; t < nsides; t += 1024) {
+    u32 key[DIM];
+    side_key<DIM>(ev, t, key);
+    u32 h = tuple_hash(key, mask);
+    for (u32 probe = 0; probe <= mask && atomicCAS(&table[h], INVALID, t) != INVALID; ++probe) h = (h + 1) & mask;
+  }
+  __threadfence();
+  __syncthreads();
+  for (u32 t = threadIdx.x; t < nsides; t += 1024) {
+    u32 key[DIM];
+    side_key<DIM>(ev, t, key);
+    u32 h = tuple_hash(key, mask), r = INVALID;
+    for (u32 probe = 0; probe <= mask; ++probe, h = (h + 1) & mask) {
+      u32 const o = __hip_atomic_load(&table[h], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if (o == INVALID) break;
+      u32 pk[DIM];
+      side_key<DIM>(ev, o, pk);
+      bool same = o / SPE != t / SPE;
+#pragma unroll
+      for (u32 k = 0; k < DIM; ++k) same = same && pk[k] == key[k];
+      if (same && o / SPE < r) r = o / SPE;
+    }
+    dual[t] = r;
   }
 }
 
@@ -1023,26 +1063,29 @@ __global__ __launch_bounds__(BLOCK) void dual_edges_k(u32 nt, u32 const* __restr
   dual[s] = r;
 }
 
-static Buf<u32> dual_by_pairs(Mesh& m) {
+static Buf<u32> dual_by_pairs(Mesh& m, bool sides) {
   u32 dim = m.dim;
   u32 ne = count(m, dim);
   u32 spe = h_down_deg[dim][dim - 1];
   size_t nsides = (size_t) ne * spe;
-  Buf<u32> out(nsides);
+  Buf<u32> out(nsides + 1);  // and a word behind: whether a side is crowded
   if (!nsides) return out;
   OHX_REQUIRE(nsides < ((size_t) 1 << 31), "dual: too many element sides");
   u32 cap = 1;
   while (cap < 2 * nsides) cap <<= 1;
   Buf<u32> table(cap);
   fill(table.get(), cap, INVALID);
-  fill(out.get(), (u32) nsides, INVALID);
+  fill(out.get(), (u32) nsides + 1, INVALID);
   u32 const* ev = ask_down(m, dim, 0);
-  if (dim == 3)
-    hipLaunchKernelGGL(dual_pairs_k<3>, dim3(nblocks(nsides)), dim3(BLOCK), 0, stream(), (u32) nsides, ev, cap - 1,
-                       table.get(), out.get(), dev_error_word());
-  else
-    hipLaunchKernelGGL(dual_pairs_k<2>, dim3(nblocks(nsides)), dim3(BLOCK), 0, stream(), (u32) nsides, ev, cap - 1,
-                       table.get(), out.get(), dev_error_word());
+  u32* crowd = sides ? out.get() + nsides : dev_error_word();
+  auto go = [&](auto pairs, auto crowded) {
+    hipLaunchKernelGGL(pairs, dim3(nblocks(nsides)), dim3(BLOCK), 0, stream(), (u32) nsides, ev, cap - 1, table.get(),
+                       out.get(), crowd);
+    if (sides)
+      hipLaunchKernelGGL(crowded, dim3(1), dim3(1024), 0, stream(), (u32) nsides, ev, cap - 1, table.get(), out.get(),
+                         crowd);
+  };
+  dim == 3 ? go(dual_pairs_k<3>, dual_crowded_k<3>) : go(dual_pairs_k<2>, dual_crowded_k<2>);
   check_launch("dual_pairs");
   return out;
 }
@@ -1174,9 +1217,10 @@ Graph const& ask_star(Mesh& m, u32 l, u32 h) {
 u32 const* ask_dual(Mesh& m) {
   if (!m.dual) {
     u32 d = m.dim;
-    if (m.down[d][d - 1] && m.up[d - 1][d])
+    bool const sides = has_dim(m, d - 1);
+    if (sides && m.down[d][d - 1] && m.up[d - 1][d])
       m.dual = dual_from_sides(m);  // the side maps are there already
-    else if (d == 3 && m.down[3][1] && m.up[1][3]) {
+    else if (sides && d == 3 && m.down[3][1] && m.up[1][3]) {
       u32 nt = m.counts[3];
       Buf<u32> out((size_t) 4 * nt);
       if (nt) {
@@ -1187,7 +1231,7 @@ u32 const* ask_dual(Mesh& m) {
       }
       m.dual = std::move(out);
     } else
-      m.dual = dual_by_pairs(m);
+      m.dual = dual_by_pairs(m, sides);
   }
   return m.dual.get();
 }

@@ -1,6 +1,10 @@
 """Deriving a model where its components matter: several bodies, holes, single
 elements and shuffled elements, against the oracle's search; and the element
-dual of a mesh without sides, whose third element on a side is an error."""
+dual where a side has three elements: an error in a mesh without sides, an
+element's lowest other one where the caller gave the sides."""
+import ctypes as C
+import itertools
+
 import numpy as np
 import pytest
 
@@ -58,3 +62,88 @@ def test_three_elements_on_a_side():
     m = ML.Mesh(ML.load("product"), 2, x, np.array([[0, 1, 2], [1, 0, 3], [0, 1, 4]], dtype=np.uint32))
     with pytest.raises(RuntimeError, match="non-manifold"):
         m.derive_model_full()
+
+
+def test_three_elements_on_a_side_beside_edge_maps():
+    """The same error in 3D also where the edges, but no faces, are there."""
+    x = np.vstack([np.eye(4, 3), [[1, 1, 1.0], [-1, -1, -1.0]]])
+    m = ML.Mesh(ML.load("product"), 3, x, np.array([[0, 1, 2, 3], [0, 1, 2, 4], [0, 1, 2, 5]], dtype=np.uint32))
+    m.down(1, 0), m.down(3, 1), m.up(1, 3)
+    with pytest.raises(RuntimeError, match="non-manifold"):
+        m.dual()
+
+
+SIDES = {2: [(0, 1), (1, 2), (2, 0)], 3: [(0, 2, 1), (0, 1, 3), (1, 2, 3), (2, 0, 3)]}
+
+
+class Given(ML.Mesh):
+    """A full mesh whose entities of every dimension the caller gives."""
+
+    def __init__(self, lib, x, elems):
+        dim = elems.shape[1] - 1
+        d = lib.dll
+        for f in ("osh_new", "osh_build_ents", "osh_new_field"):
+            getattr(d, f).restype = C.c_void_p
+        d.osh_build_ents.argtypes = [C.c_void_p, C.c_uint, C.c_uint]
+        d.osh_new_field.argtypes = [C.c_void_p, C.c_uint, C.c_char_p, C.c_uint, C.c_int]
+        hip = C.CDLL("libamdhip64.so")
+
+        def put(p, a):
+            a = np.ascontiguousarray(a)
+            assert hip.hipMemcpy(C.c_void_p(p), a.ctypes.data_as(C.c_void_p), C.c_size_t(a.nbytes), 1) == 0
+
+        self.lib, self.dim, self.h = lib, dim, d.osh_new(dim)
+        d.osh_build_ents(self.h, 0, len(x))
+        put(d.osh_new_field(self.h, 0, b"coordinates", 3, 1), x)
+        for k in range(1, dim):
+            ents = np.unique(np.sort(np.vstack([elems[:, c] for c in itertools.combinations(range(dim + 1), k + 1)]), 1),
+                             axis=0)
+            put(d.osh_build_ents(self.h, k, len(ents)), ents.astype(np.uint32))
+        put(d.osh_build_ents(self.h, dim, len(elems)), elems.astype(np.uint32))
+
+
+def books(dim, rng, spines, pages):
+    """Elements around common sides, 1 to `pages` on each, and plain boxes
+    between them, all in any order."""
+    xs, cs, at = [], [], 0
+    for k in range(spines):
+        n = 1 + k % pages
+        angle = 2 * np.pi * np.arange(n) / n
+        tips = np.stack([np.cos(angle), np.sin(angle), 0 * angle], 1)
+        spine = np.array([[0, 0, 0], [0, 0, 1], [0, 0, 2.0]])[:dim]
+        xs.append(np.vstack([spine, tips]) + [3.0 * k, 0, 0])
+        cs.append(np.array([list(range(dim)) + [dim + p] for p in range(n)]) + at)
+        at += dim + n
+    x, c = ML.box(dim, 3)
+    xs.append(x)
+    cs.append(c.astype(np.int64) + at)
+    c = np.vstack(cs)
+    return np.vstack(xs), c[rng.permutation(len(c))]
+
+
+def lowest_other(elems):
+    dim = elems.shape[1] - 1
+    of = {}
+    for i, e in enumerate(elems):
+        for j, s in enumerate(SIDES[dim]):
+            of.setdefault(tuple(sorted(e[list(s)])), []).append((i, j))
+    want = np.full((len(elems), dim + 1), 0xFFFFFFFF, np.uint32)
+    for uses in of.values():
+        for i, j in uses:
+            others = [o for o, _ in uses if o != i]
+            if others:
+                want[i, j] = min(others)
+    return want
+
+
+@pytest.mark.parametrize("dim,maps", [(2, ""), (2, "sides"), (3, ""), (3, "sides"), (3, "edges")])
+@pytest.mark.parametrize("spines,pages", [(1, 3), (9, 5), (4000, 4)])
+def test_dual_of_given_sides(dim, maps, spines, pages):
+    """One answer whichever maps the mesh has when the dual is asked for."""
+    x, c = books(dim, np.random.default_rng([dim, spines]), spines, pages)
+    m = Given(ML.load("product"), x, c)
+    if maps == "sides":
+        m.down(dim, dim - 1), m.up(dim - 1, dim)
+    elif maps == "edges":
+        m.down(3, 1), m.up(1, 3)
+    assert np.array_equal(m.dual().reshape(-1, dim + 1), lowest_other(c))
