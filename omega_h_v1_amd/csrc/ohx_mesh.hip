@@ -1070,19 +1070,27 @@ static Buf<u32> dual_by_pairs(Mesh& m, bool sides) {
   size_t nsides = (size_t) ne * spe;
   Buf<u32> out(nsides + 1);  // and a word behind: whether a side is crowded
   if (!nsides) return out;
-  OHX_REQUIRE(nsides < ((size_t) 1 << 31), "dual: too many element sides");
-  u32 cap = 1;
-  while (cap < 2 * nsides) cap <<= 1;
+  // sides are numbered in 32 bits; a mesh that has them is refused from 2^31 on
+  OHX_REQUIRE(nsides < ((size_t) 1 << (sides ? 31 : 32)) - BLOCK, "dual: too many element sides");
+  // two slots a side, up to the 2^32 that 32 bits can number (a side of two
+  // elements takes one slot)
+  size_t cap = 1;
+  while (cap < 2 * nsides && cap < ((size_t) 1 << 32)) cap <<= 1;
+  u32 const mask = (u32) (cap - 1);
   Buf<u32> table(cap);
-  fill(table.get(), cap, INVALID);
-  fill(out.get(), (u32) nsides + 1, INVALID);
+  auto clear = [](u32* p, size_t n) {
+    size_t const most = (size_t) 1 << 31;
+    for (size_t at = 0; at < n; at += most) fill(p + at, (u32) (n - at < most ? n - at : most), INVALID);
+  };
+  clear(table.get(), cap);
+  clear(out.get(), nsides + 1);
   u32 const* ev = ask_down(m, dim, 0);
   u32* crowd = sides ? out.get() + nsides : dev_error_word();
   auto go = [&](auto pairs, auto crowded) {
-    hipLaunchKernelGGL(pairs, dim3(nblocks(nsides)), dim3(BLOCK), 0, stream(), (u32) nsides, ev, cap - 1, table.get(),
+    hipLaunchKernelGGL(pairs, dim3(nblocks(nsides)), dim3(BLOCK), 0, stream(), (u32) nsides, ev, mask, table.get(),
                        out.get(), crowd);
     if (sides)
-      hipLaunchKernelGGL(crowded, dim3(1), dim3(1024), 0, stream(), (u32) nsides, ev, cap - 1, table.get(), out.get(),
+      hipLaunchKernelGGL(crowded, dim3(1), dim3(1024), 0, stream(), (u32) nsides, ev, mask, table.get(), out.get(),
                          crowd);
   };
   dim == 3 ? go(dual_pairs_k<3>, dual_crowded_k<3>) : go(dual_pairs_k<2>, dual_crowded_k<2>);

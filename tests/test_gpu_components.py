@@ -147,3 +147,15 @@ def test_dual_of_given_sides(dim, maps, spines, pages):
     elif maps == "edges":
         m.down(3, 1), m.up(1, 3)
     assert np.array_equal(m.dual().reshape(-1, dim + 1), lowest_other(c))
+
+
+def test_sides_of_a_mesh_of_more_than_a_billion():
+    """359 million triangles have 2^30 sides and more: twice as many table
+    slots are as many as 32 bits can number."""
+    lib = ML.load("product")
+    n = 13400
+    m = ML.Mesh.box_on_device(lib, 2, n)
+    assert 6 * n * n > 1 << 30
+    assert m.count(1) == 3 * n * n + 2 * n
+    del m
+    lib.dll.osh_fini()  # its memory goes back to the device
