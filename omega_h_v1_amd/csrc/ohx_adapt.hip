@@ -3321,9 +3321,8 @@ static Tuner& swap_tuner() {
   return tuner;
 }
 static bool swap_screen_pinned() {
-  if (!swap_tuner().forced()) return false;
-  hipEvent_t a = nullptr, b = nullptr;
-  return swap_tuner().pick(1, &a, &b) == 1;
+  u32 const* v = swap_tuner().forced_variant();
+  return v && *v == 1;
 }
 
 // swap_common + swap_interior + swap_ents (swap.cpp:27-136)

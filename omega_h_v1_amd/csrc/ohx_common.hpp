@@ -340,8 +340,10 @@ struct Tuner {
   u32 pick(u32 n, hipEvent_t* a, hipEvent_t* b);
   void harvest();
   int chosen(u32 n) const;
-  // pinned to a variant by tuning_force
+  // pinned by tuning_force (to any value), and the variant it is pinned to
+  // (null where the value is none of its variants, which pins nothing)
   bool forced() const;
+  u32 const* forced_variant() const;
 };
 // run launch(variant, start_event, stop_event) with the tuner's choice
 template <class L>

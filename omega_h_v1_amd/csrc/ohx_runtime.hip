@@ -561,13 +561,17 @@ void Tuner::harvest() {
 
 bool Tuner::forced() const { return forced_variants().count(name) != 0; }
 
+u32 const* Tuner::forced_variant() const {
+  auto f = forced_variants().find(name);
+  if (f != forced_variants().end())
+    for (u32 const& v : variants)
+      if (v == f->second) return &v;
+  return nullptr;
+}
+
 u32 Tuner::pick(u32 n, hipEvent_t* a, hipEvent_t* b) {
   if (std::find(tuners().begin(), tuners().end(), this) == tuners().end()) tuners().push_back(this);
-  auto f = forced_variants().find(name);
-  if (f != forced_variants().end()) {
-    for (u32 v : variants)
-      if (v == f->second) return v;
-  }
+  if (u32 const* v = forced_variant()) return *v;
   u32 cls = size_class(n);
   Cls& c = classes[cls];
   if (c.best.empty()) {

@@ -110,6 +110,25 @@ def test_swap_run_over_every_ring_size(libs, n, before):
     assert same(a, b) is None
 
 
+@pytest.mark.parametrize("value", [0, 1, 7])
+def test_screen_of_a_swap_run_pinned(libs, value):
+    """In the mixed mode, the FP32 screen of the swap qualities pinned off, on,
+    and to a value that is none of its variants, which pins nothing."""
+    lib = libs[0]
+    lib.dll.ohx_tuning_force.argtypes = [C.c_char_p, C.c_int]
+    a = front(lib, 4, 0.16)
+    b = a.clone()
+    a.adapt(max_ops=1000)
+    lib.dll.ohx_tuning_force(b"swap_quality_3d_mixed", value)
+    lib.dll.ohx_set_precision(1)
+    try:
+        b.adapt(max_ops=1000)
+    finally:
+        lib.dll.ohx_set_precision(0)
+        lib.dll.ohx_tuning_force(b"swap_quality_3d_mixed", -1)
+    assert same(a, b) is None
+
+
 @pytest.mark.parametrize("n", [2, 3, 4])
 @pytest.mark.parametrize("more", [0, 1])
 def test_a_run_waits_once_per_pass(libs, n, more):
