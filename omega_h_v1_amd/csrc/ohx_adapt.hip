@@ -2112,7 +2112,17 @@ static u32 coarsen_common(Mesh& m, Buf<u32>& codes, double qual_floor, bool requ
   Buf<u32> cand;
   Buf<double> vq;
   {
-    double prof_bytes = (double) ne * 32 + (double) ue.adj.size() * 8 + (double) count(m, dim) * (dim + 1) * 4 + (double) count(m, 0) * 28;
+    // compulsory bytes: of each direction measured its list entry, its edge's
+    // ends, code and value; and of the elements around the collapsing
+    // vertices, their vertices and coordinates at least the share of the
+    // mesh's that the directions are of all directions (a vertex's are mostly
+    // listed together).  The directions measured again in FP64 are chosen on
+    // the device among all: what is read to choose them.
+    double const share = (double) neval / (2.0 * ne);
+    double const prof_bytes =
+        (double) neval * 24 + share * ((double) ue.adj.size() * 8 + (double) count(m, dim) * (dim + 1) * 4 +
+                                       (double) count(m, 0) * (metric_of(m) ? 76 : 28));
+    double const force_bytes = (double) ncand * 16;
     // variants, chosen online per size class: lanes per edge (1, 2, 4 or
     // 8) and, in the mixed mode, the FP32 screen (+16) or the certified FP32
     // pass (+32); all give identical results.  The mixed mode takes the
@@ -2189,8 +2199,8 @@ static u32 coarsen_common(Mesh& m, Buf<u32>& codes, double qual_floor, bool requ
         f.ncand = ncand;
         f.list = clist.get();
         f.vmark = vmark.get();
-        dim == 3 ? cq_launch_mode<3>(CQ_FORCE, g, f, prof_bytes, nullptr, nullptr)
-                 : cq_launch_mode<2>(CQ_FORCE, g, f, prof_bytes, nullptr, nullptr);
+        dim == 3 ? cq_launch_mode<3>(CQ_FORCE, g, f, force_bytes, nullptr, nullptr)
+                 : cq_launch_mode<2>(CQ_FORCE, g, f, force_bytes, nullptr, nullptr);
         to_vert();
       }
       if (eb) OHX_CHECK(hipEventRecord(eb, stream()));
@@ -4124,14 +4134,23 @@ __global__ __launch_bounds__(BLOCK) void run_count_k(SwapRunView R, unsigned cha
 }
 
 // one block: the blocks' totals become their first products, and the totals,
-// the pool's top, the set's flag, the run's error and the quality minimum go
-// to the host
+// the pool's top, the set's flag, the run's error, the counts of candidates
+// and the quality minimum go to the host
 __global__ __launch_bounds__(1024) void run_offsets_k(u32 nb, RunCount* __restrict__ part, u32 npart,
                                                       double const* __restrict__ qpart, SwapRunView R,
                                                       u32 const* __restrict__ flag, u32* __restrict__ host,
                                                       double* __restrict__ host_min) {
   __shared__ u32 lds[16][4];
   __shared__ double mins[16];
+  // candidates in the set's rounds; evaluated ones, and the tets around them
+  u32 const accepted = R.words[RW_ACC];
+  u32 evals = 0, tets = 0;
+#pragma unroll
+  for (u32 r = 0; r < RUN_RINGS; ++r) {
+    u32 const n = R.words[RW_EVAL + r];
+    evals += n;
+    tets += (r + 3) * n;
+  }
   u32 const per = (nb + 1023) / 1024, b = threadIdx.x * per, e = b + per < nb ? b + per : nb;
   RunCount c{}, tot;
   for (u32 i = b; i < e; ++i)
@@ -4160,6 +4179,9 @@ __global__ __launch_bounds__(1024) void run_offsets_k(u32 nb, RunCount* __restri
   host[4] = R.words[RW_POOL];
   host[5] = *flag;
   host[6] = R.words[RW_ERR];
+  host[7] = accepted;
+  host[8] = evals;
+  host[9] = tets;
   *host_min = v;
 }
 
@@ -4602,7 +4624,7 @@ struct SwapRun {
   static constexpr size_t MAX_USES = (size_t) 1 << 32;
   bool has_id = false;
   bool intact = true;  // the mesh in the arrays is that of the passes so far
-  u32 got[7];
+  u32 got[10];
   double min_q = 0;
 
   explicit SwapRun(Mesh& mesh) : m(mesh) {}
@@ -4823,9 +4845,12 @@ struct SwapRun {
     unsigned char *a = sa.get(), *b = sb.get();
     u32* flags = words.get() + RW_FLAGS;
     auto round = [&](u32* fl) {
-      launch_timed("indset_round", (double) nE, run_round_k, dim3(gr), dim3(BLOCK), R, a, b, fl);
+      launch_timed("indset_round", 0, run_round_k, dim3(gr), dim3(BLOCK), R, a, b, fl);
       std::swap(a, b);
     };
+    // the first rounds' bytes at least: each candidate's list entry, state in
+    // and out, and in the first round its value
+    auto count_rounds = [&] { prof_add_bytes("indset_round", (6.0 * first + 8) * got[7]); };
     for (u32 r = 0; r < first; ++r) round(flags + r);
     u32 const nb = nblocks(nE, BLOCK * RUN_PER);
     if (!part || part.size() < nb) part = Buf<RunCount>(nb + nb / 2);
@@ -4844,13 +4869,17 @@ struct SwapRun {
         intact = !hs[6];
         throw;
       }
-      for (u32 k = 0; k < 7; ++k) got[k] = hs[k];
+      for (u32 k = 0; k < 10; ++k) got[k] = hs[k];
       if (got[6]) {
         intact = false;
         fail_device(got[6]);
       }
     };
     totals();
+    count_rounds();
+    // of each evaluated candidate its list entry, ends, list place and length,
+    // choice and value, and the tets around it and its places in them
+    prof_add_bytes(quality_name(), 36.0 * got[8] + 8.0 * got[9]);
     min_q = *host_slot<double>(SLOT_RUN_MIN);
     if (min_q >= good) return false;
     if (got[5]) {
@@ -4864,21 +4893,24 @@ struct SwapRun {
     return true;
   }
 
+  char const* quality_name() const {
+    return g_mixed && swap_screen_pinned() ? "swap_quality_mixed" : "swap_quality_f64";
+  }
   void evaluate(SwapRunView const& R) {
     double const* mt = metric_of(m);
     double const* x = coords(m);
     u32 const need = (aE + SW_EDGES - 1) / SW_EDGES;
     dim3 const grid(need < 2048 ? (need ? need : 1) : 2048);
     ScreenStats st = screen_stats();
-    auto go = [&](auto kernel, char const* kn) {
-      launch_timed(kn, (double) aE * 24, kernel, grid, dim3(BLOCK), R, x, mt, tq.get(), dev_error_word(), st);
+    auto go = [&](auto kernel) {
+      launch_timed(quality_name(), 0, kernel, grid, dim3(BLOCK), R, x, mt, tq.get(), dev_error_word(), st);
     };
     // the FP32 screen runs only where it is pinned on: timed on live
     // launches it lost to FP64 at every size class of the shipped table
     if (g_mixed && swap_screen_pinned())
-      mt ? go(run_quality_k<true, true>, "swap_quality_mixed") : go(run_quality_k<false, true>, "swap_quality_mixed");
+      mt ? go(run_quality_k<true, true>) : go(run_quality_k<false, true>);
     else
-      mt ? go(run_quality_k<true, false>, "swap_quality_f64") : go(run_quality_k<false, false>, "swap_quality_f64");
+      mt ? go(run_quality_k<true, false>) : go(run_quality_k<false, false>);
     u32 const ab = nblocks(aE, RUN_AT);
     hipLaunchKernelGGL(run_accept_k, dim3(ab < 64 ? ab : 64, RUN_RINGS), dim3(RUN_AB), 0, stream(), R);
     check_launch("run_accept");

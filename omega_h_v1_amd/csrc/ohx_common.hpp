@@ -297,6 +297,9 @@ void prof_only(char const* name);
 void prof_host(char const* name, double ms);
 ProfEvents prof_take();
 void prof_record(char const* name, double bytes, ProfEvents e);
+// bytes of launches of that name whose work only the device knew when they
+// were made
+void prof_add_bytes(char const* name, double bytes);
 
 template <class K, class... A>
 void launch_timed(char const* name, double bytes, K kernel, dim3 grid, dim3 block, A... args) {

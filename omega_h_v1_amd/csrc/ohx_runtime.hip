@@ -367,6 +367,10 @@ void prof_record(char const* name, double bytes, ProfEvents e) {
   prof().pending.push_back({name, e.a, e.b, bytes});
 }
 
+void prof_add_bytes(char const* name, double bytes) {
+  if (prof_on_for(name)) prof().totals[name].units += bytes;
+}
+
 void prof_enable(bool on) {
   Prof& p = prof();
   p.on = on;

@@ -11,6 +11,7 @@ import pytest
 import meshlib as ML
 import parity_cases as P
 from omega_h_v1_amd import workloads as W
+from test_gpu_swap_run import front
 
 pytestmark = pytest.mark.gpu
 
@@ -69,3 +70,53 @@ def test_collapse_loop(libs, mode, dim, n, h, jitter, metric):
     finally:
         d.ohx_set_precision(0)
         d.ohx_tuning_force(name, -1)
+
+
+PEAK = 8.0e9  # bytes per millisecond
+
+
+def test_bytes_of_what_is_measured(libs):
+    """The bytes counted for the collapse qualities are those of the directions
+    a pass measures: passes that know some of them count fewer than
+    passes on their own, which measure every one; and neither they nor the
+    swap run's kernels read more than the memory can give."""
+    d = libs[0].dll
+    d.ohx_profile_get.argtypes = [C.c_char_p] + 3 * [C.c_void_p]
+    start = front(libs[0], 9, 0.16)
+    floor = min(start.min_quality(), 0.3)
+    while start.refine_by_size(floor):
+        pass
+    floor = min(start.min_quality(), 0.3)
+
+    def counted(run, names):
+        d.ohx_profile_enable(1)
+        d.ohx_profile_reset()
+        got = {}
+        try:
+            run()
+            for name in names:
+                ms, k, b = C.c_double(), C.c_ulonglong(), C.c_double()
+                d.ohx_profile_get(name.encode(), C.byref(ms), C.byref(k), C.byref(b))
+                if k.value:
+                    got[name] = (k.value, b.value)
+                    assert 0 < b.value < PEAK * ms.value, (name, b.value, ms.value)
+        finally:
+            d.ohx_profile_enable(0)
+        return got
+
+    a, b = start.clone(), start.clone()
+    passes = 6
+    every = counted(lambda: [a.coarsen_by_size(floor, 1 / 3) for _ in range(passes)],
+                    ["coarsen_quality_f64"])["coarsen_quality_f64"]
+    names = ["coarsen_quality_f64", "swap_quality_f64", "indset_round"]
+    known = counted(lambda: b.adapt(max_ops=passes - 2), names)["coarsen_quality_f64"]
+    assert P.diff_states(a, b) is None
+    assert known[0] == every[0] and known[1] < every[1]
+    # the whole of an adaptation, in both modes
+    counted(lambda: start.clone().adapt(max_ops=1000), names)
+    d.ohx_set_precision(1)
+    try:
+        counted(lambda: start.clone().adapt(max_ops=1000),
+                names + ["coarsen_quality_mixed", "coarsen_quality_certified", "coarsen_quality_force"])
+    finally:
+        d.ohx_set_precision(0)
