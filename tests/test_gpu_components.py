@@ -159,3 +159,56 @@ def test_sides_of_a_mesh_of_more_than_a_billion():
     assert m.count(1) == 3 * n * n + 2 * n
     del m
     lib.dll.osh_fini()  # its memory goes back to the device
+
+
+def glued(dim, rng, balls, boxes):
+    """Balls glued three at a time along their whole surface (fans over the
+    facets of a simplex): every facet there has three elements and there is no
+    boundary; and plain boxes, all in any order."""
+    xs, cs, at = [], [], 0
+    facets = list(itertools.combinations(range(dim + 1), dim))
+    for k in range(balls):
+        x = rng.random((dim + 4, 3)) + [2.0 * k, 0, 0]
+        xs.append(x)
+        cs.append(np.array([list(f) + [dim + 1 + b] for b in range(3) for f in facets]) + at)
+        at += len(x)
+    for k in range(boxes):
+        x, c = ML.box(dim, 2)
+        xs.append(x - [2.0 * (k + 1), 0, 0])
+        cs.append(c.astype(np.int64) + at)
+        at += len(x)
+    c = np.vstack(cs)
+    return np.vstack(xs), c[rng.permutation(len(c))]
+
+
+def searched(elems):
+    """The reference's component search (bfs.cpp:18-103) over each side's first
+    other element in ascending order (derive_model.cpp:270-396)."""
+    to = lowest_other(elems)
+    comp = np.full(len(elems), -1)
+    n = 0
+    for i in range(len(elems)):
+        if comp[i] >= 0:
+            continue
+        queue = [i]
+        comp[i] = n
+        for u in queue:
+            for v in to[u]:
+                if v != 0xFFFFFFFF and comp[v] < 0:
+                    comp[v] = n
+                    queue.append(int(v))
+        n += 1
+    return comp
+
+
+@pytest.mark.parametrize("dim", [2, 3])
+@pytest.mark.parametrize("balls,boxes", [(1, 0), (2, 2), (40, 3)])
+def test_components_across_crowded_sides(dim, balls, boxes):
+    """Where a side joins more than two elements the search follows only the
+    first other one, so that components depend on the elements' order."""
+    for seed in range(4):
+        x, c = glued(dim, np.random.default_rng([dim, balls, seed]), balls, boxes)
+        m = Given(ML.load("product"), x, c)
+        m.derive_model_full()
+        assert (m.tag(dim, "class_dim") == dim).all()
+        assert np.array_equal(m.tag(dim, "class_id"), searched(c))
