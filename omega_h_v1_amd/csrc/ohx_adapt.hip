@@ -411,7 +411,7 @@ __global__ __launch_bounds__(BLOCK) void refine_quality_f64(
     u32 ns, u32 per, u32 const* __restrict__ vs, u32 const* __restrict__ uo, u32 const* __restrict__ ua,
     u32 const* __restrict__ ud, u32 const* __restrict__ ve, double const* __restrict__ x,
     double const* __restrict__ mt, double const* __restrict__ eq, double qual_floor_all,
-    double const* __restrict__ qfe, u32* __restrict__ cand, double* __restrict__ out, u32* __restrict__ words, u32 tag,
+    double const* __restrict__ qfe, u32* __restrict__ cand, double* __restrict__ out, u32* __restrict__ words,
     u32* __restrict__ err, ScreenStats st) {
   constexpr u32 G = 4;
   __shared__ u32 list[RQ_EDGES], nlist;
@@ -491,7 +491,6 @@ __global__ __launch_bounds__(BLOCK) void refine_quality_f64(
     } else {
       out[i] = minq;
       cand[i] = UNKNOWN;
-      wave_flag_value(words + W_ANY, true, tag);
     }
   }
 }
@@ -520,7 +519,6 @@ static Buf<double> refine_qualities(Mesh& m, u32* cand, double qual_floor, bool 
   Buf<double> eq;
   if (require_better) eq = mesh_qualities(m);
   Buf<double> out(ns);
-  u32 tag = next_any_tag();
   double prof_bytes = (double) ns * 20 + (double) u.adj.size() * 8 + (double) count(m, dim) * (dim + 1) * 4 + (double) count(m, 0) * 24;
   ScreenStats sst = screen_stats();
   // in the mixed mode the FP32 screen is a variant chosen online (it pays
@@ -535,12 +533,12 @@ static Buf<double> refine_qualities(Mesh& m, u32* cand, double qual_floor, bool 
     if (ea) {
       hipExtLaunchKernelGGL(kernel, grid, dim3(BLOCK), 0, stream(), ea, eb, 0, ns, per, vs, u.offsets.get(),
                             u.adj.get(), u.dirs.get(), ve, coords(m), metric_of(m), eq.get(), qual_floor, qfe,
-                            cand, out.get(), scratch_words(), tag, dev_error_word(), sst);
+                            cand, out.get(), scratch_words(), dev_error_word(), sst);
       check_launch(kn);
     } else {
       launch_timed(kn, prof_bytes, kernel, grid, dim3(BLOCK), ns, per, vs, u.offsets.get(), u.adj.get(),
                    u.dirs.get(), ve, coords(m), metric_of(m), eq.get(), qual_floor, qfe, cand, out.get(),
-                   scratch_words(), tag, dev_error_word(), sst);
+                   scratch_words(), dev_error_word(), sst);
     }
   };
   auto run = [&](u32 screen, hipEvent_t ea, hipEvent_t eb) {
@@ -1242,8 +1240,8 @@ struct CqArgs {
 // of about 20, so with one direction per group a wave ran at 20 of its 64
 // lanes.  A block takes a.chunk directions instead, and a group whose
 // direction has ended takes the block's next one (once a quarter of the
-// wave's groups wait, as taking one is a chain of loads): 541 -> 417 us for a
-// call at 55 thousand tets in FP64, at 32 lanes, and 3405 -> 3180 us for a
+// wave's groups wait, as taking one is a chain of loads): 541 -> 422 us for a
+// call at 55 thousand tets in FP64, at 32 lanes, and 3405 -> 3194 us for a
 // certified one at 511 thousand, at 48 (2048 blocks instead of 1024: 487 us).
 // The directions that FP32 leaves open are listed and follow in FP64 in the
 // same way.
@@ -2123,12 +2121,16 @@ static u32 coarsen_common(Mesh& m, Buf<u32>& codes, double qual_floor, bool requ
         (double) neval * 24 + share * ((double) ue.adj.size() * 8 + (double) count(m, dim) * (dim + 1) * 4 +
                                        (double) count(m, 0) * (metric_of(m) ? 76 : 28));
     double const force_bytes = (double) ncand * 16;
-    // variants, chosen online per size class: lanes per edge (1, 2, 4 or
-    // 8) and, in the mixed mode, the FP32 screen (+16) or the certified FP32
-    // pass (+32); all give identical results.  The mixed mode takes the
-    // certified pass from CQ_CERTIFIED_MIN candidates up (below that its
-    // three extra small launches cost more than the FP64 work it saves),
-    // lanes per edge tuned; the screen stays available to pin.
+    // variants, chosen online per size class of the directions measured: lanes
+    // per edge (1, 2, 4 or 8) and, in the mixed mode, the FP32 screen (+16) or
+    // the certified FP32 pass (+32); all give identical results.  The mixed
+    // mode takes an FP32 form from CQ_CERTIFIED_MIN directions up (below that
+    // the certified pass's three extra small launches cost more than the FP64
+    // work it saves).  Above it the FP32 forms no longer win: since a block's
+    // directions are handed on as they end, 8 cycles of the 64^3 x 6
+    // anisotropic box spend 134 ms on these kernels in FP64 and 180 ms in the
+    // mixed mode, which has no FP64 variant there (192 ms with every variant
+    // timed anew on live launches, the trials included).
     static thread_local Tuner tuners[2][3] = {
         {Tuner("coarsen_quality_2d_f64", {1, 2, 4, 8}),
          Tuner("coarsen_quality_2d_mixed", {33, 34, 36, 40, 17, 18, 20, 24}),
