@@ -380,13 +380,16 @@ ZeroCounters& zero_counters() {
 u32* take_zeroed_counters(u32 n) {
   ZeroCounters& z = zero_counters();
   if (n > z.cap) {
-    // stream-ordered release: the arena reuses the block only after the
-    // stream's earlier work
-    if (z.p) dev_free(z.p);
     size_t cap = z.cap * 2 > n ? z.cap * 2 : n;
     if (cap > 0xffffffffull) cap = 0xffffffffull;
-    z.cap = cap < ((size_t) 1 << 16) ? ((size_t) 1 << 16) : cap;
-    z.p = static_cast<u32*>(dev_alloc(z.cap * sizeof(u32)));
+    if (cap < ((size_t) 1 << 16)) cap = (size_t) 1 << 16;
+    // the new array first: where there is no memory for it the old one stays.
+    // Stream-ordered release: the arena reuses the block only after the
+    // stream's earlier work
+    u32* const p = static_cast<u32*>(dev_alloc(cap * sizeof(u32)));
+    if (z.p) dev_free(z.p);
+    z.p = p;
+    z.cap = cap;
     z.dirty = true;
   }
   if (z.dirty) {

@@ -116,13 +116,14 @@ bool scan_concurrent() { return g_scan_threads.load(std::memory_order_relaxed) >
 ScanTiles scan_tiles_for(u32 nt) {
   ScanState& st = scan_state();
   if (nt > st.cap) {
-    // a larger tile array; the old one is released once the stream drains
-    if (st.tiles) {
-      sync();
-      dev_free(st.tiles);
-    }
-    st.cap = nt < 1024 ? 1024 : nt;
-    st.tiles = static_cast<u64*>(dev_alloc(sizeof(u64) * st.cap));
+    // a larger tile array (the old one stays where there is no memory for
+    // it); the old one is released once the stream drains
+    u32 const cap = nt < 1024 ? 1024 : nt;
+    if (st.tiles) sync();
+    u64* const tiles = static_cast<u64*>(dev_alloc(sizeof(u64) * cap));
+    if (st.tiles) dev_free(st.tiles);
+    st.tiles = tiles;
+    st.cap = cap;
     OHX_CHECK(hipMemsetAsync(st.tiles, 0xff, sizeof(u64) * st.cap, stream()));
   }
   // epochs stay below 2^30 - 1, so fresh all-ones words never match one

@@ -16,6 +16,7 @@ import pytest
 
 import meshlib as ML
 from omega_h_v1_amd import workloads as W
+from test_gpu_kernels import Dev
 
 pytestmark = pytest.mark.gpu
 
@@ -155,3 +156,61 @@ def test_non_positive_split_quality_is_an_error(product):
         m.refine_by_size(-1.0)
     ok = _c1(product, True)
     assert ok.refine_by_size(min(ok.min_quality(), 0.3)) == 1
+
+
+@pytest.mark.parametrize("entry", ["up_from_down", "exscan"])
+def test_scratch_that_cannot_grow_stays(product, entry):
+    """The scratch that a thread keeps between calls (the counters of the upward
+    adjacency, the tile words of the scans) is still what it was after a call
+    for which it could not grow, and later calls are right."""
+    import threading
+
+    d = product.dll
+    d.ohx_up_from_down.argtypes = [C.c_uint] * 4 + [C.c_void_p] * 5
+    d.ohx_exscan_u32.argtypes = [C.c_void_p, C.c_uint, C.c_void_p, C.c_void_p]
+    d.ohx_set_device_bytes_limit.argtypes = [C.c_ulonglong]
+    d.ohx_device_bytes_high_water.restype = C.c_ulonglong
+    dev = Dev()
+    big = 30_000_000
+    rng = np.random.default_rng(3)
+    a = rng.integers(0, 3, big, dtype=np.uint32)
+    pa, po, ph, pd = dev.put(a), dev.empty(big + 1, np.uint32), dev.empty(64, np.uint32), dev.empty(64, np.uint32)
+    failures = []
+
+    def up(nl):
+        lows = rng.integers(0, nl, 64, dtype=np.uint32)
+        if d.ohx_up_from_down(1, 0, 32, nl, dev.put(lows), po, ph, pd, None):
+            return False
+        order = np.argsort(lows, kind="stable")
+        assert np.array_equal(dev.get(po, nl + 1, np.uint32),
+                              np.concatenate([[0], np.cumsum(np.bincount(lows, minlength=nl))]))
+        assert np.array_equal(dev.get(ph, 64, np.uint32), order // 2)
+        return True
+
+    def scan(n):
+        if d.ohx_exscan_u32(pa, n, po, None):
+            return False
+        assert np.array_equal(dev.get(po, n + 1, np.uint32), np.concatenate([[0], np.cumsum(a[:n], dtype=np.uint32)]))
+        return True
+
+    def calls():  # a thread of its own: its scratch is new
+        try:
+            call = up if entry == "up_from_down" else scan
+            assert call(100)
+            d.ohx_device_reset_high_water()
+            d.ohx_set_device_bytes_limit(d.ohx_device_bytes_high_water() + 4096)
+            refused = not call(big)
+            d.ohx_set_device_bytes_limit(0)
+            assert refused
+            assert call(big // 10) and call(big) and call(100)
+        except BaseException as e:  # shown by the test's own thread
+            failures.append(e)
+        finally:
+            d.ohx_set_device_bytes_limit(0)
+
+    t = threading.Thread(target=calls)
+    t.start()
+    t.join()
+    dev.free()
+    if failures:
+        raise failures[0]
