@@ -96,18 +96,20 @@ ADAPT_ARGS = (1.0 / 3.0, 0.3, 4, 50)
 # profiled run's launches of the kernel; per workload and kernel (the
 # kernels that can be a workload's dominant one)
 TRAFFIC = {
-    ("c2", "scan"): 2764823,
-    ("c2", "indset_round"): 3225804,
-    ("c2", "reflect_down"): 53090816,
-    ("c3", "coarsen_quality_mixed"): 610625883,
-    ("c3", "scan"): 12556348,
-    ("c3", "reflect_down"): 715727174,
-    ("c5", "coarsen_outputs"): 4469509427,
-    ("c5", "up_patch_fill"): 3443524823,
-    ("c5", "scan"): 389051928,
-    ("c5", "coarsen_quality_mixed"): 13300132659,
-    ("c5", "lows_hash_insert"): 2519497975,
-    ("c5", "reflect_down"): 11939056067,
+    ("c2", "scan"): 5021599,
+    ("c2", "indset_round"): 2756403,
+    ("c2", "reflect_down"): 30110413,
+    ("c3", "coarsen_quality_mixed"): 619421925,
+    ("c3", "coarsen_outputs"): 621543728,
+    ("c3", "up_patch_fill"): 176379113,
+    ("c3", "scan"): 38985663,
+    ("c3", "reflect_down"): 594069805,
+    ("c5", "coarsen_outputs"): 13800857119,
+    ("c5", "up_patch_fill"): 3545705667,
+    ("c5", "scan"): 1070093130,
+    ("c5", "coarsen_quality_mixed"): 3435905248,
+    ("c5", "lows_hash_insert"): 1646648411,
+    ("c5", "reflect_down"): 6357101728,
 }
 
 
@@ -429,7 +431,8 @@ def run_c3(args, lib):
                         "is one mesh_adapt cycle (cycle k mod 8 of the sequence, from its input mesh)",
             "precision": "FP32-mixed: split, collapse and swap qualities in FP32 (reject-only screen, or certified "
                          "accept/reject and goodness comparisons), FP64 re-evaluation of every decision within 1e-4; "
-                         "the variant per kernel and size class is the fastest measured, FP64 included",
+                         "the variant per kernel and size class is the fastest measured of those the mode offers "
+                         "(for the collapse qualities of 4096 directions and more these are FP32 forms only)",
             "max_ops": C3_MAX_OPS,
             "ops_per_cycle": [c["passes"] for c in svf["cycles"]],
             "cycles_at_op_limit": sum(1 for c in svf["cycles"] if c["result"] < 0),

@@ -2741,8 +2741,10 @@ __device__ inline u32 edge_ring(u32 edge, u32 f, u32 e, u32 const* ua, u32 const
 // path's.  Accepted candidates store the value (goodness), the ring size
 // and the triangulation code, which swap_cavity uses.  The kernel is built
 // for 4 waves per SIMD (at most 128 VGPRs; its 33 KB of LDS per block allow
-// 4 blocks per CU): with a metric that costs 28 bytes of scratch per lane
-// and measured 4 % less time on the 64^3 x 6 anisotropic box than 3 waves without spills.
+// 4 blocks per CU): with both tets of a triangle on one lane that cost 28
+// bytes of scratch per lane and measured 4 % less time on the 64^3 x 6
+// anisotropic box than 3 waves without spills; with a tet per lane it takes
+// 98 VGPRs and no scratch.
 constexpr u32 SW_G = 8;
 constexpr u32 SW_EDGES = BLOCK / SW_G;
 constexpr u32 SW_MAXTRI = 35;
