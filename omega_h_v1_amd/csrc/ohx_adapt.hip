@@ -1014,9 +1014,10 @@ static u32 refine_common(Mesh& m, Buf<u32>& cand, double qual_floor, bool requir
   if (!total) return 0;
   u32 nsplit[4] = {0, total, got[1], got[2]};
   Mesh mo(m.dim, m.full);
-  // maps are carried through mesh_adapt's loop of split passes, and where the
-  // mesh has the map that only the carrying reads
-  refine_ents(m, mo, gen_off.get(), off, nsplit, carry || (dim == 3 && m.down[3][2]));
+  // maps are carried only through mesh_adapt's loop of split passes: a pass
+  // on its own would make maps of the new mesh that its caller may not read
+  // (384,000 tets with all their maps split once: 375 us, 668 with maps carried)
+  refine_ents(m, mo, gen_off.get(), off, nsplit, carry);
   say("split", total, 1);
   overwrite(m, std::move(mo));
   return 1;

@@ -1,7 +1,9 @@
 """Split passes carry the side maps and the elements around the edges to the
 mesh they make: after any number of passes of mesh_adapt the mesh equals the
 oracle's and every carried map a fresh derivation, from the smallest boxes to
-odd sizes, in both dimensions."""
+odd sizes, in both dimensions.  A split pass on its own carries none."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -55,3 +57,37 @@ def test_split_and_collapse_with_large_scans():
         got.append(m)
     assert got[0].last == got[1].last == (1, 1)
     assert P.diff_states(*got) is None
+
+
+@pytest.mark.parametrize("dim,n", [(2, 5), (3, 3)])
+@pytest.mark.parametrize("kind", ["by size", "uniform"])
+def test_split_pass_on_its_own_makes_no_maps(dim, n, kind):
+    """Whatever maps the mesh has, a single pass does not spend time on the new
+    mesh's: no adjacency is patched, and what is asked for is derived."""
+    lib = ML.load("product")
+    d = lib.dll
+    d.ohx_profile_get.argtypes = [C.c_char_p] + 3 * [C.c_void_p]
+    m = P.make_mesh(lib, dim, n)
+    m.add_field(0, "adapt_size", W.uniform_size(m.count(0), 0.7 / n))
+    for high in range(1, dim + 1):
+        for low in range(high):
+            m.down(high, low), m.up(low, high)
+    before = m.count(dim)
+    d.ohx_profile_enable(1)
+    try:
+        d.ohx_profile_reset()
+        if kind == "uniform":
+            m.uniformly_refine()
+        else:
+            m.refine_by_size(0.1)
+        ms, launches, units = C.c_double(), C.c_ulonglong(), C.c_double()
+        for name in (b"up_patch_count", b"up_patch_fill"):
+            d.ohx_profile_get(name, C.byref(ms), C.byref(launches), C.byref(units))
+            assert launches.value == 0, name
+    finally:
+        d.ohx_profile_enable(0)
+    assert m.count(dim) > before
+    fresh = m.clone()
+    for high in range(2, dim + 1):
+        for low in range(1, high):
+            assert np.array_equal(m.down(high, low), fresh.down(high, low)), (high, low)
