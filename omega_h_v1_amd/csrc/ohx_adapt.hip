@@ -233,8 +233,11 @@ static Buf<u32> indset_rounds(Mesh& m, u32 ent_dim, u32 const* filter, double co
                               u32 const** last_flag, Buf<u32>* start = nullptr, u32 start_done = 0) {
   u32 n = count(m, ent_dim);
   // vertices: neighbours through the edges (indset_round_verts); edges:
-  // through the elements (indset_round_elems)
-  bool const via_edges = ent_dim == 0 && m.dim >= 2, via_elems = ent_dim == 1 && m.dim >= 2;
+  // through the elements (indset_round_elems), unless the star, which holds
+  // each neighbour once, is there already (set of a 162,000-tet mesh's edges:
+  // 343 us by the star, 415 through the elements)
+  bool const via_edges = ent_dim == 0 && m.dim >= 2;
+  bool const via_elems = ent_dim == 1 && m.dim >= 2 && !m.star[1][m.dim];
   Graph empty;
   Graph const& g = (via_elems || via_edges) ? empty : ask_star(m, ent_dim, m.dim);
   Up const* ut = via_elems ? &ask_up(m, 1, m.dim) : via_edges ? &ask_up(m, 0, 1) : nullptr;
