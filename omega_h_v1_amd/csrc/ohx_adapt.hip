@@ -4949,11 +4949,6 @@ struct SwapRun {
   // the run's mesh, gaps closed, becomes m; eq its element qualities, and
   // known and values (when wanted) its edges' words and values
   void finish(Buf<double>& eq, Buf<u32>* known, Buf<double>* values) {
-    // an error of the last pass's kernels shows here, before its output is followed
-    u32 const* err = words.get() + RW_ERR;
-    u32 code;
-    read_many(&err, 1, &code);
-    if (code) fail_device(code);
     // what only the passes need goes first, and the maps of the mesh that
     // goes: there is room then also where a pass found too little
     for (auto* b : {&face_prod, &acc, &eval, &cnt}) b->release();
@@ -4995,6 +4990,16 @@ struct SwapRun {
       }
       return 1u;
     }, fr.get());
+    // an error of the last pass's kernels shows here, before its output is
+    // followed, and how many entities are left.  The faces are counted: around
+    // inverted tets a swap can make an edge whose vertices another edge has,
+    // and the pair rule then takes the faces of both
+    u32 const* ends[4] = {words.get() + RW_ERR, er.get() + nE, tr.get() + nT, fr.get() + nF};
+    u32 left[4];
+    read_many(ends, 4, left);
+    if (left[0]) fail_device(left[0]);
+    OHX_REQUIRE(left[1] == aE && left[2] == aT, "swap run: edges or tets miscounted");
+    aF = left[3];
     Mesh mo(3, true);
     set_ents(mo, 0, m.counts[0], Buf<u32>());
     u32 const alive[4] = {0, aE, aF, aT};

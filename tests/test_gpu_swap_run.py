@@ -43,12 +43,12 @@ def front(lib, n, jitter):
     return m
 
 
-def rough(lib, n, jitter):
+def rough(lib, n, jitter, seed=None):
     """A box of badly shaped tets that are of the desired size: the shape
     loop, which starts with a swap run, is all there is to do."""
     x, c = ML.box(3, n)
     inner = ((x > 0) & (x < 1)).all(1)
-    x = x + (np.random.default_rng(n).random(x.shape) - 0.5) * (jitter / n) * inner[:, None]
+    x = x + (np.random.default_rng(n if seed is None else seed).random(x.shape) - 0.5) * (jitter / n) * inner[:, None]
     m = ML.Mesh(lib, 3, x, c)
     m.derive_model_full()
     m.add_field(0, "adapt_size", W.uniform_size(m.count(0), 10.0))
@@ -197,6 +197,25 @@ def test_pass_seconds_hold_the_whole_run(libs):
         assert end == -1 and stats[0] == 2 and stats[1] >= 2 * m.count(3)
         share = max(share, stats[2] / stats[3])
     assert 0.65 < share <= 1
+
+
+@pytest.mark.parametrize("n,jitter,seed,ops", [(4, 1.1, 5, 3), (4, 1.3, 33, 3), (4, 1.3, 54, 2), (4, 2.2, 44, 1),
+                                               (5, 1.1, 30, 2), (5, 1.1, 31, 1), (6, 1.1, 3, 1)])
+def test_swap_run_makes_an_edge_twice(libs, n, jitter, seed, ops):
+    """Around inverted tets a swap can make an edge whose two vertices another
+    edge has; when one of them goes, so do the faces on both.  The run's mesh
+    has as many faces as are left then, and is the one of whole-mesh passes."""
+    a = rough(libs[0], n, jitter, seed)
+    b = a.clone()
+    b.add_field(3, "mass", np.ones(b.count(3)), transfer=P.CONSERVE)
+    start = a.counts()
+    assert a.adapt(max_ops=ops, **ROUGH) == b.adapt(max_ops=ops, **ROUGH)
+    b.free_field(3, "mass")
+    assert same(a, b) is None
+    # swaps only, and fewer faces than a mesh of so many tets with the box's
+    # surface has, were every face there
+    assert a.count(0) == start[0]
+    assert a.count(2) < (4 * a.count(3) + 12 * n * n) // 2
 
 
 def test_device_error_inside_a_swap_run(libs):
