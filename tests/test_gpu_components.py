@@ -10,6 +10,7 @@ import pytest
 
 import meshlib as ML
 import parity_cases as P
+from omega_h_v1_amd import workloads as W
 
 pytestmark = pytest.mark.gpu
 
@@ -159,6 +160,25 @@ def test_sides_of_a_mesh_of_more_than_a_billion():
     assert m.count(1) == 3 * n * n + 2 * n
     del m
     lib.dll.osh_fini()  # its memory goes back to the device
+
+
+@pytest.mark.parametrize("seed", [10, 33, 34, 60, 81, 113])
+def test_adapting_a_folded_mesh(seed):
+    """Inverted triangles, where the passes make a side with three elements: the
+    sliver layers grow across it as the oracle's do."""
+    n, got = 12, []
+    x, c = ML.box(2, n)
+    inner = ((x[:, :2] > 0) & (x[:, :2] < 1)).all(1)
+    step = (np.random.default_rng(seed).random(x.shape) - 0.5) * (1.1 / n) * inner[:, None]
+    step[:, 2] = 0
+    for which in ("product", "oracle"):
+        m = ML.Mesh(ML.load(which), 2, x + step, c)
+        m.derive_model_full()
+        assert m.min_quality() < 0
+        m.add_field(0, "metric", W.rotating_metric(x + step, 1.0 / n, 4.0, dim=2).ravel())
+        assert m.adapt(max_ops=20) == 1
+        got.append(m)
+    assert P.diff_states(*got) is None
 
 
 def glued(dim, rng, balls, boxes):
